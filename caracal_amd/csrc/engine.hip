@@ -37,130 +37,42 @@ struct TrajArgs {
     Rx rx;
 };
 
-// COM translation and rotation removal over all beads, as src/transrot.f90:36-237
-// computes it (including its total mass of nbeads^2 * M).
-__global__ void transrot_kernel(TrajArgs a)
+// transrot (transrot.hpp) for the split schedule's windows: one wave per
+// trajectory, its lanes over the (atom, bead) pairs, butterfly sums.
+__global__ __launch_bounds__(64 * kParentWaves) void transrot_kernel(TrajArgs a, double totmass)
 {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    const int lane = threadIdx.x % 64, t = blockIdx.x * kParentWaves + threadIdx.x / 64;
     if (t >= a.ntraj) return;
-    const int NA = a.natoms, NB = a.nbeads, NC = 3 * NA;
-    double *q = a.q + (size_t)t * NC * NB, *p = a.p + (size_t)t * NC * NB;
-    auto Q = [&](int d, int i, int k) -> double & { return q[(size_t)(3 * i + d) * NB + k]; };
-    auto P = [&](int d, int i, int k) -> double & { return p[(size_t)(3 * i + d) * NB + k]; };
-    double totmass = 0.0, vtot[3] = { 0, 0, 0 };
-    for (int i = 0; i < NA; ++i) {
-        const double w = a.mass[i];
-        for (int k = 0; k < NB; ++k) {
-            totmass = totmass + w;
-            for (int j = 0; j < 3; ++j) vtot[j] = vtot[j] + (P(j, i, k) / a.mass[i]) * w;
+    const int NA = a.natoms, NB = a.nbeads;
+    const double *q = a.q + (size_t)t * 3 * NA * NB;
+    double *p = a.p + (size_t)t * 3 * NA * NB;
+    auto pairs = [&](auto &&f) {
+        for (int e = lane; e < NA * NB; e += 64) {
+            const size_t o = (size_t)(e / NB) * 3 * NB + e % NB;
+            double x[3], y[3];
+            for (int d = 0; d < 3; ++d) {
+                x[d] = q[o + (size_t)d * NB];
+                y[d] = p[o + (size_t)d * NB];
+            }
+            f(o, x, y, a.mass[e / NB]);
         }
+    };
+    double v1[6] = { 0, 0, 0, 0, 0, 0 }, v2[9] = { 0, 0, 0, 0, 0, 0, 0, 0, 0 }, omega[3];
+    pairs([&](size_t, const double *x, const double *y, double m) { transrot_sums1(x, y, m, v1); });
+#pragma unroll
+    for (int i = 0; i < 6; ++i) {
+        for (int o = 32; o > 0; o >>= 1) v1[i] += __shfl_xor(v1[i], o, 64);
+        v1[i] = v1[i] / totmass;
     }
-    totmass = totmass * NB;
-    for (int j = 0; j < 3; ++j) vtot[j] = vtot[j] / totmass;
-    double xt = 0, yt = 0, zt = 0;
-    for (int i = 0; i < NA; ++i) {
-        const double w = a.mass[i];
-        for (int k = 0; k < NB; ++k) {
-            xt = xt + Q(0, i, k) * w;
-            yt = yt + Q(1, i, k) * w;
-            zt = zt + Q(2, i, k) * w;
-        }
-    }
-    xt = xt / totmass;
-    yt = yt / totmass;
-    zt = zt / totmass;
-    double mang[3] = { 0, 0, 0 };
-    for (int i = 0; i < NA; ++i) {
-        const double w = a.mass[i];
-        for (int k = 0; k < NB; ++k) {
-            const double vx = P(0, i, k) / a.mass[i], vy = P(1, i, k) / a.mass[i], vz = P(2, i, k) / a.mass[i];
-            mang[0] = mang[0] + (Q(1, i, k) * vz - Q(2, i, k) * vy) * w;
-            mang[1] = mang[1] + (Q(2, i, k) * vx - Q(0, i, k) * vz) * w;
-            mang[2] = mang[2] + (Q(0, i, k) * vy - Q(1, i, k) * vx) * w;
-        }
-    }
-    mang[0] = mang[0] - (yt * vtot[2] - zt * vtot[1]) * totmass;
-    mang[1] = mang[1] - (zt * vtot[0] - xt * vtot[2]) * totmass;
-    mang[2] = mang[2] - (xt * vtot[1] - yt * vtot[0]) * totmass;
-    double xx = 0, xy = 0, xz = 0, yy = 0, yz = 0, zz = 0;
-    for (int i = 0; i < NA; ++i) {
-        const double w = a.mass[i];
-        for (int k = 0; k < NB; ++k) {
-            const double xd = Q(0, i, k) - xt, yd = Q(1, i, k) - yt, zd = Q(2, i, k) - zt;
-            xx = xx + xd * xd * w;
-            xy = xy + xd * yd * w;
-            xz = xz + xd * zd * w;
-            yy = yy + yd * yd * w;
-            yz = yz + yd * zd * w;
-            zz = zz + zd * zd * w;
-        }
-    }
-    // tensor, column-major a(row,col) as the reference builds it
-    double ten[3][3];
-    ten[0][0] = yy + zz; ten[0][1] = -xy;    ten[0][2] = -xz;
-    ten[1][0] = -xy;     ten[1][1] = xx + zz; ten[1][2] = -yz;
-    ten[2][0] = -xz;     ten[2][1] = -yz;    ten[2][2] = xx + yy;
-    if (NA <= 2) {
-        ten[0][0] += 0.000001;
-        ten[1][1] += 0.000001;
-        ten[2][2] += 0.000001;
-    }
-    // Gauss-Jordan inversion with full pivoting (src/invert.f90)
-    {
-        int ipiv[3] = { 0, 0, 0 }, indxr[3], indxc[3];
-        for (int i = 0; i < 3; ++i) {
-            double big = 0.0;
-            int irow = 0, icol = 0;
-            for (int j = 0; j < 3; ++j)
-                if (ipiv[j] != 1)
-                    for (int kk = 0; kk < 3; ++kk)
-                        if (ipiv[kk] == 0 && fabs(ten[j][kk]) >= big) {
-                            big = fabs(ten[j][kk]);
-                            irow = j;
-                            icol = kk;
-                        }
-            ipiv[icol] += 1;
-            if (irow != icol)
-                for (int j = 0; j < 3; ++j) {
-                    const double tmp = ten[irow][j];
-                    ten[irow][j] = ten[icol][j];
-                    ten[icol][j] = tmp;
-                }
-            indxr[i] = irow;
-            indxc[i] = icol;
-            const double piv = ten[icol][icol];
-            ten[icol][icol] = 1.0;
-            for (int j = 0; j < 3; ++j) ten[icol][j] = ten[icol][j] / piv;
-            for (int j = 0; j < 3; ++j)
-                if (j != icol) {
-                    const double tmp = ten[j][icol];
-                    ten[j][icol] = 0.0;
-                    for (int kk = 0; kk < 3; ++kk) ten[j][kk] = ten[j][kk] - ten[icol][kk] * tmp;
-                }
-        }
-        for (int i = 2; i >= 0; --i)
-            if (indxr[i] != indxc[i])
-                for (int kk = 0; kk < 3; ++kk) {
-                    const double tmp = ten[kk][indxr[i]];
-                    ten[kk][indxr[i]] = ten[kk][indxc[i]];
-                    ten[kk][indxc[i]] = tmp;
-                }
-    }
-    double vang[3];
-    for (int i = 0; i < 3; ++i) {
-        vang[i] = 0.0;
-        for (int j = 0; j < 3; ++j) vang[i] = vang[i] + ten[i][j] * mang[j];
-    }
-    for (int i = 0; i < NA; ++i)
-        for (int k = 0; k < NB; ++k) {
-            double v[3];
-            for (int j = 0; j < 3; ++j) v[j] = P(j, i, k) / a.mass[i] - vtot[j];
-            const double xd = Q(0, i, k) - xt, yd = Q(1, i, k) - yt, zd = Q(2, i, k) - zt;
-            v[0] = v[0] - vang[1] * zd + vang[2] * yd;
-            v[1] = v[1] - vang[2] * xd + vang[0] * zd;
-            v[2] = v[2] - vang[0] * yd + vang[1] * xd;
-            for (int j = 0; j < 3; ++j) P(j, i, k) = v[j] * a.mass[i];
-        }
+    pairs([&](size_t, const double *x, const double *y, double m) { transrot_sums2(x, y, m, v1 + 3, v2); });
+#pragma unroll
+    for (int i = 0; i < 9; ++i)
+        for (int o = 32; o > 0; o >>= 1) v2[i] += __shfl_xor(v2[i], o, 64);
+    transrot_omega(v1, v1 + 3, v2, totmass, omega);
+    pairs([&](size_t o, const double *x, double *y, double m) {
+        transrot_apply(x, y, m, v1, v1 + 3, omega);
+        for (int d = 0; d < 3; ++d) p[o + (size_t)d * NB] = y[d];
+    });
 }
 
 // Centroid of trajectory t (3*natoms, atom-major).
@@ -919,6 +831,11 @@ StepArgs step_args(cam_engine *e)
     // (the fused window step tests andersen_step > 0)
     a.andersen_step = e->cfg.ensemble == CAM_ENS_UMBRELLA ? e->cfg.andersen_step
                                                           : (e->cfg.andersen_step > 0 ? e->cfg.andersen_step : 1);
+    a.transrot = e->cfg.remove_com;
+    // every atom counted once per bead, then times nbeads (src/transrot.f90:62-72)
+    for (int i = 0; i < e->cfg.natoms; ++i)
+        for (int k = 0; k < e->cfg.nbeads; ++k) a.totmass = a.totmass + e->cfg.mass[i];
+    a.totmass = a.totmass * e->cfg.nbeads;
     a.seed = e->cfg.seed;
     a.dt = e->cfg.dt;
     std::memcpy(a.mass, e->cfg.mass, sizeof a.mass);
@@ -927,10 +844,10 @@ StepArgs step_args(cam_engine *e)
 }
 
 // The kernel launches of nsteps steps on the state a points to: fused (spl
-// steps per launch, transrot after each launch when requested) or split (per
+// steps per launch) or split (per
 // step the normal-mode kernel, then the force kernel; one last half kick).
 hipError_t launch_steps(cam_engine *e, const Kernels &kn, bool split, int spl, StepArgs a, int nsteps,
-                        const TrajArgs *transrot, bool slices = true)
+                        bool slices = true)
 {
     const int grid = (e->cfg.ntraj + e->tpb - 1) / e->tpb;
     hipError_t err = hipSuccess;
@@ -985,11 +902,8 @@ hipError_t launch_steps(cam_engine *e, const Kernels &kn, bool split, int spl, S
                 hipLaunchKernelGGL(umbrella_end_kernel<decltype(na)::value>, dim3(pgrid), dim3(64 * kParentWaves), 0, e->stream, ta, a.g, e->uwin, a.ustat, a.pfail, a.step_base, j, as, a.seed, e->pcheck_max, e->pcheck_xi_tol, e->pcheck_after, a.uhist, a.hbins, a.hmin, a.hinv);
             });
             err = hipGetLastError();
-            if (err == hipSuccess && transrot) {
-                TrajArgs tr = *transrot;
-                tr.q = a.q;
-                tr.p = a.p;
-                hipLaunchKernelGGL(transrot_kernel, dim3((e->cfg.ntraj + 127) / 128), dim3(128), 0, e->stream, tr);
+            if (err == hipSuccess && a.transrot) {
+                hipLaunchKernelGGL(transrot_kernel, dim3(pgrid), dim3(64 * kParentWaves), 0, e->stream, ta, a.totmass);
                 err = hipGetLastError();
             }
         }
@@ -1013,7 +927,6 @@ hipError_t launch_steps(cam_engine *e, const Kernels &kn, bool split, int spl, S
                            e->cfg.natoms, e->cfg.nbeads);
         return hipGetLastError();
     }
-    const int tgrid = (e->cfg.ntraj + 127) / 128;
     const int sgrid = (e->cfg.ntraj + kn.step_tpb - 1) / kn.step_tpb;
     // The launches of one trajectory slice [a.tbegin, a.tend) on stream st.
     const auto slice = [&](StepArgs b, hipStream_t st) {
@@ -1031,10 +944,6 @@ hipError_t launch_steps(cam_engine *e, const Kernels &kn, bool split, int spl, S
                 });
                 rc = hipGetLastError();
             }
-            if (rc == hipSuccess && transrot) {
-                hipLaunchKernelGGL(transrot_kernel, dim3(tgrid), dim3(128), 0, st, *transrot);
-                rc = hipGetLastError();
-            }
         }
         return rc;
     };
@@ -1046,7 +955,7 @@ hipError_t launch_steps(cam_engine *e, const Kernels &kn, bool split, int spl, S
     // Not when the caller's stream is itself a branch forked from another
     // stream (a ragged batch's bucket, whose neighbours fill the chip): the
     // slices fork only from a stream that starts its own work.
-    if (!slices || !kn.folded || transrot || sgrid < 2 * kSliceMinBlocks || !e->slice_stream)
+    if (!slices || !kn.folded || sgrid < 2 * kSliceMinBlocks || !e->slice_stream)
         return slice(a, e->stream);
     StepArgs lo = a, hi = a;
     lo.tend = hi.tbegin = (sgrid / 2) * kn.step_tpb;
@@ -1064,9 +973,7 @@ hipError_t launch_steps(cam_engine *e, const Kernels &kn, bool split, int spl, S
 // (launch_steps); false for a stream that is itself a forked branch.
 int enqueue_run(cam_engine *e, int nsteps, bool slices)
 {
-    const TrajArgs ta = traj_args(e);
-    CAM_HIP(launch_steps(e, e->kern, e->split, e->spl, step_args(e), nsteps, e->cfg.remove_com ? &ta : nullptr,
-                         slices));
+    CAM_HIP(launch_steps(e, e->kern, e->split, e->spl, step_args(e), nsteps, slices));
     if (e->cfg.ensemble == CAM_ENS_CHILD) {
         hipLaunchKernelGGL(kappa_reduce_kernel, dim3(nsteps), dim3(256), 0, e->stream, e->xi_flag, e->weight,
                            e->cfg.ntraj, e->num, e->step_base);
@@ -1177,7 +1084,6 @@ int cam_engine_create(const cam_config *cfg, cam_engine **out)
     e->tpb = kBlock / (L * nb);
     // steps fused per launch: state stays in registers for this many steps
     e->spl = cfg->steps_per_launch > 0 ? cfg->steps_per_launch : 50;
-    if (cfg->remove_com) e->spl = 1;
     if (cfg->nm_kernel != CAM_NMK_AUTO) e->nmk = cfg->nm_kernel;
     else e->nmk = fold_available(cfg) ? CAM_NMK_FOLDED : CAM_NMK_VALU;
     // the FP64 CH5 folded kernel is faster at two waves per SIMD, the unfolded
@@ -1591,7 +1497,7 @@ int cam_engine_run(cam_engine *e, int nsteps)
     // Long runs replay a graph of at most kGraphLaunches step launches (and
     // one graph of the remainder) instead of capturing every step into one
     // graph: a split-schedule step is three or four launches, a fused launch
-    // spl steps (one, plus transrot, when the centre of mass is removed).
+    // spl steps.
     const int steps_per_graph = (e->split ? 1 : e->spl) * kGraphLaunches;
     const int chunk = std::min(nsteps, steps_per_graph);
     const int reps = nsteps / chunk, tail = nsteps % chunk;
@@ -1712,8 +1618,7 @@ static int autotune(cam_engine *e, int trial_steps, cam_tuning *out, bool slices
         if (mfma_bead_count(nb)) nmks.push_back(CAM_NMK_MFMA);
         if (fold_available(&c)) nmks.push_back(CAM_NMK_FOLDED);
     }
-    if (c.remove_com) spls.push_back(1);
-    else if (c.steps_per_launch > 0) spls.push_back(c.steps_per_launch);
+    if (c.steps_per_launch > 0) spls.push_back(c.steps_per_launch);
     else
         for (int v : { 10, 25, 50, 100 }) spls.push_back(v);
     // Trials run on a copy of the state with their own flag rows and step
@@ -1788,9 +1693,9 @@ static int autotune(cam_engine *e, int trial_steps, cam_tuning *out, bool slices
         if (err == hipSuccess) err = hipMemcpyAsync(a.g, e->g, nstate * sizeof(double), hipMemcpyDeviceToDevice, e->stream);
         // one untimed launch sequence, then the timed trial
         if (err == hipSuccess)
-            err = launch_steps(e, kn, tr.split != 0, tr.spl, a, std::min(tr.spl, trial_steps), nullptr, slices);
+            err = launch_steps(e, kn, tr.split != 0, tr.spl, a, std::min(tr.spl, trial_steps), slices);
         if (err == hipSuccess) err = hipEventRecord(t0, e->stream);
-        if (err == hipSuccess) err = launch_steps(e, kn, tr.split != 0, tr.spl, a, trial_steps, nullptr, slices);
+        if (err == hipSuccess) err = launch_steps(e, kn, tr.split != 0, tr.spl, a, trial_steps, slices);
         if (err == hipSuccess) err = hipEventRecord(t1, e->stream);
         if (err == hipSuccess) err = hipEventSynchronize(t1);
         float ms = 0.f;

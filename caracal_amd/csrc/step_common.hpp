@@ -12,6 +12,7 @@
 #include "pes_o3.hpp"
 #include "pes_oh3.hpp"
 #include "nhc.hpp"
+#include "transrot.hpp"
 
 namespace cam {
 
@@ -124,6 +125,8 @@ struct StepArgs {
     int tbegin, tend;            // trajectories of this launch (folded kernels and xi_flag_kernel;
                                  // the other kernels take all ntraj)
     int andersen_step;
+    int transrot;                // fused kernels: remove translation and rotation after every step
+    double totmass;              //   with this total mass (transrot.hpp)
     uint64_t seed;
     double dt;
     double mass[CAM_MAX_ATOMS];

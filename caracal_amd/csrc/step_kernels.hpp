@@ -488,6 +488,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE))) v
     constexpr bool NHC = ENS == CAM_ENS_NHC;
     __shared__ double nred[NHC ? kBlock : 1];
     __shared__ double nscale[NHC ? TPB : 1];
+    // transrot after every step (not for children, and not in the split
+    // schedule's kernel): the sums of each trajectory
+    constexpr bool TRANSROT = !SPLIT && ENS != CAM_ENS_CHILD;
+    __shared__ double trsum[TRANSROT && NB > 1 ? TPB * 9 : 1];
 
     const int tid = threadIdx.x;
     const int r = tid % L;
@@ -614,6 +618,37 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE))) v
         }
     }
 
+    // The sum of each trajectory's NV per-bead values v (the same on every
+    // lane of a bead), on every lane, in a fixed order: staged in the
+    // normal-mode columns, added by four lanes per sum.
+    [[maybe_unused]] auto traj_sum = [&](auto nv, double *v) {
+        if constexpr (TRANSROT && NB > 1) {
+            constexpr int NV = decltype(nv)::value, P = NB % 4 == 0 ? 4 : 2, Q = NB / P;
+            static_assert(XS >= TPB * NB * NV && NB % P == 0, "the column buffer holds nine values per bead");
+            __syncthreads();                          // the transform's reads, and the last sums' reads
+            if (live && r == 0) {
+#pragma unroll
+                for (int i = 0; i < NV; ++i) X[(tl * NV + i) * NB + k] = v[i];
+            }
+            __syncthreads();
+            for (int i = tid; i < TPB * NV * P; i += kBlock) {
+                // each sum starts at another bead, so that the sums a wave reads spread over the banks
+                int j = i / P % Q;
+                double s = 0.0;
+#pragma unroll
+                for (int n = 0; n < Q; ++n) {
+                    s += X[(i / P) * NB + i % P + P * j];
+                    j = j + 1 < Q ? j + 1 : 0;
+                }
+                s += quad::dpp<quad::perm(1, 0, 3, 2)>(s);
+                if constexpr (P == 4) s += quad::dpp<quad::perm(2, 3, 0, 1)>(s);
+                if (i % P == 0) trsum[i / P] = s;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < NV; ++i) v[i] = trsum[tl * NV + i];
+        }
+    };
     if constexpr (UMB) {
         for (int i = tid; i < TPB; i += kBlock) ubad[i] = 0;
     }
@@ -879,6 +914,34 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE))) v
                     const double sd = sqrt((TAB ? smass[cc[s] / 3] : m[s]) / (beta / NB));
                     p[s] = andersen_normal(a.seed, (uint32_t)traj, istep, cc[s], k) * sd;
                 }
+            }
+        }
+        if constexpr (TRANSROT) {
+            // src/verlet.f90:1299-1305.  In the step loop because a launch
+            // per step of a kernel with one lane per trajectory (serial loads
+            // over all its beads) cost more than the step: 212 us against
+            // 27 for 1001 OH3 trajectories of 24 beads, 31 against 23 for
+            // one H3 window of 8.  Here its sums run over all lanes and the
+            // state stays in registers.
+            if (a.transrot) {
+                auto atoms = [&](auto &&f) {          // this lane's atoms: slots come in (x, y, z) triples
+#pragma unroll
+                    for (int s = 0; s < SL; s += 3)
+                        if (S::valid(s, r)) f(s, TAB ? smass[cc[s] / 3] : m[s]);
+                };
+                double v1[6] = { 0, 0, 0, 0, 0, 0 }, v2[9] = { 0, 0, 0, 0, 0, 0, 0, 0, 0 }, omega[3];
+                atoms([&](int s, double ms) { transrot_sums1(q + s, p + s, ms, v1); });
+                if constexpr (L == 4)
+                    for (int i = 0; i < 6; ++i) v1[i] = quad::sum(v1[i]);
+                traj_sum(std::integral_constant<int, 6>{}, v1);
+#pragma unroll
+                for (int i = 0; i < 6; ++i) v1[i] = v1[i] / a.totmass;
+                atoms([&](int s, double ms) { transrot_sums2(q + s, p + s, ms, v1 + 3, v2); });
+                if constexpr (L == 4)
+                    for (int i = 0; i < 9; ++i) v2[i] = quad::sum(v2[i]);
+                traj_sum(std::integral_constant<int, 9>{}, v2);
+                transrot_omega(v1, v1 + 3, v2, a.totmass, omega);
+                atoms([&](int s, double ms) { transrot_apply(q + s, p + s, ms, v1, v1 + 3, omega); });
             }
         }
     }

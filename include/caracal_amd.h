@@ -346,7 +346,7 @@ int cam_engine_device_state(cam_engine *eng, double **q, double **p, double **dv
  * split launches (schedule AUTO, remove_com off), and for the fused schedule
  * the register budget (waves_per_eu 1 or 2; FP64 CH4H with waves_per_eu 0)
  * and the steps fused per launch (10, 25, 50, 100; only when
- * steps_per_launch is 0 and remove_com is off).  Captured graphs are dropped.  No counterpart in
+ * steps_per_launch is 0).  Captured graphs are dropped.  No counterpart in
  * the reference, which has one schedule. */
 #define CAM_MAX_TRIALS 32
 typedef struct {
