@@ -590,6 +590,7 @@ struct cam_engine {
     double *pdxi = nullptr;           // PARENT: constraint directions [traj][3*natoms]
     int *pfail = nullptr;             // PARENT, UMBRELLA: trajectory flags (kPf*)
     double *uwin = nullptr;           // UMBRELLA: (xi_ideal, k_force) per trajectory
+    XiTable *xitab = nullptr;         // UMBRELLA: the reaction coordinate's distances
     double *ustat = nullptr;          // UMBRELLA: running sums of xi, xi^2 per trajectory
     double *nhc = nullptr;            // NHC: thermostat velocities [traj][4]
     long ustat_steps = 0;             // UMBRELLA: steps in those sums
@@ -692,6 +693,38 @@ bool fold_available(const cam_config *cfg)
     int tpb = 0;
     return fold_eligible(cfg) &&
            fold_step_kernel_for(cfg->surface, cfg->precision, cfg->nbeads, cfg->ensemble, 1, 1, &tpb) != nullptr;
+}
+
+// The distances of the reaction coordinate (xi_group.hpp): breaking bonds,
+// forming bonds, then the pairs of reactant centres.
+XiTable xi_table(const Rx &rx, int natoms)
+{
+    XiTable t{};
+    t.n_reac = rx.n_reac;
+    for (int pass = 0; pass < 2; ++pass)
+        for (int i = 0; i < (pass == 0 ? rx.n_break : rx.n_form); ++i) {
+            const int *ab = pass == 0 ? rx.brk[i] : rx.form[i];
+            const int j = t.nd++;
+            t.pa[j] = 3 * ab[0];
+            t.pb[j] = 3 * ab[1];
+            t.wt[j] = pass == 0 ? rx.inv_nbreak : -rx.inv_nform;
+            t.ref[j] = pass == 0 ? rx.break_ref[i] : rx.form_ref[i];
+            t.B[j][ab[0]] += 1.0;
+            t.B[j][ab[1]] -= 1.0;
+        }
+    t.nbond = t.nd;
+    for (int i = 0; i < rx.n_reac; ++i)
+        for (int k = i + 1; k < rx.n_reac; ++k) {
+            const int j = t.nd++;
+            t.pa[j] = 3 * (natoms + k);
+            t.pb[j] = 3 * (natoms + i);
+            t.wt[j] = -rx.inv_terms;
+            t.ref[j] = rx.r_inf;
+            for (int at = 0; at < natoms; ++at) t.B[j][at] = rx.fw[k][at] - rx.fw[i][at];
+        }
+    std::memcpy(t.fw, rx.fw, sizeof t.fw);
+    std::memcpy(t.inv_mass, rx.inv_mass, sizeof t.inv_mass);
+    return t;
 }
 
 bool select_kernels(cam_engine *e, int wpe, int nmk, Kernels &k)
@@ -814,6 +847,7 @@ StepArgs step_args(cam_engine *e)
     a.pfail = e->pfail;
     a.ustat = e->ustat;
     a.uwin = e->uwin;
+    a.xitab = e->xitab;
     a.nhc = e->nhc;
     a.uhist = e->uhist;
     a.hbins = e->hbins;
@@ -1133,6 +1167,9 @@ int cam_engine_create(const cam_config *cfg, cam_engine **out)
         for (int t = 0; t < cfg->ntraj; ++t) w[2 * (size_t)t] = rx.xi_ideal;
         CAM_HIP(hipMalloc(&e->uwin, w.size() * sizeof(double)));
         CAM_HIP(hipMemcpy(e->uwin, w.data(), w.size() * sizeof(double), hipMemcpyHostToDevice));
+        const XiTable xt = xi_table(rx, na);
+        CAM_HIP(hipMalloc(&e->xitab, sizeof xt));
+        CAM_HIP(hipMemcpy(e->xitab, &xt, sizeof xt, hipMemcpyHostToDevice));
         CAM_HIP(hipMalloc(&e->ustat, w.size() * sizeof(double)));
         CAM_HIP(hipMemset(e->ustat, 0, w.size() * sizeof(double)));
     }
@@ -1171,6 +1208,7 @@ int cam_engine_destroy(cam_engine *e)
     for (double *b : bufs)
         if (b) (void)hipFree(b);
     if (e->pfail) (void)hipFree(e->pfail);
+    if (e->xitab) (void)hipFree(e->xitab);
     if (e->uhist) (void)hipFree(e->uhist);
     if (e->xi_flag) (void)hipFree(e->xi_flag);
     if (e->step_base) (void)hipFree(e->step_base);

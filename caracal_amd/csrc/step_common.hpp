@@ -102,6 +102,8 @@ __device__ inline void count_xi(unsigned *h, int hbins, double hmin, double hinv
     if (j >= 1.0 && j <= (double)hbins) atomicAdd(h + (size_t)traj * hbins + ((int)j - 1), 1u);
 }
 
+struct XiTable;                  // xi_group.hpp
+
 struct StepArgs {
     double *q, *p, *g, *vbead;
     const double *beta;          // [ntraj]
@@ -113,6 +115,7 @@ struct StepArgs {
     int *pfail;                  // PARENT, UMBRELLA: trajectory flags
     double *ustat;               // UMBRELLA: running sums of xi and xi^2 [traj][2]
     const double *uwin;          // UMBRELLA: (xi_ideal, k_force) of each trajectory's window
+    const XiTable *xitab;        // UMBRELLA: the reaction coordinate as a list of distances
     double epot_max, xi_tol;     // PARENT, UMBRELLA: trajectory check
     int check_after;             //   armed after this many steps (never if < 0)
     double *nhc;                 // NHC: thermostat velocities [traj][4]

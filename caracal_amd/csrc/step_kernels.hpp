@@ -14,6 +14,7 @@
 
 #include "philox.hpp"
 #include "step_common.hpp"
+#include "xi_group.hpp"
 
 namespace cam {
 namespace {
@@ -481,6 +482,11 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE))) v
     // energies and a flag for positions that are not finite
     constexpr bool UMB = ENS == CAM_ENS_UMBRELLA;
     constexpr bool CENT = ENS == CAM_ENS_CHILD || UMB;
+    using XG = XiGroup<S::NA>;
+    constexpr int NG = kBlock / XG::GL;      // groups of lanes, a trajectory each
+    __shared__ typename std::conditional<UMB, XiTable, int>::type xt;
+    __shared__ typename std::conditional<UMB, typename XG::Work, int>::type xw[UMB ? NG : 1];
+    __shared__ double uxi[UMB ? TPB : 1];
     __shared__ double ubias[UMB ? TPB * 2 * NC : 1];
     __shared__ double uvb[UMB ? TPB * NB : 1];
     __shared__ int ubad[UMB ? TPB : 1];
@@ -651,6 +657,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE))) v
     };
     if constexpr (UMB) {
         for (int i = tid; i < TPB; i += kBlock) ubad[i] = 0;
+        static_assert(sizeof(XiTable) % 4 == 0, "copied word by word");
+        for (int i = tid; i < (int)(sizeof(XiTable) / 4); i += kBlock)
+            reinterpret_cast<int *>(&xt)[i] = reinterpret_cast<const int *>(a.xitab)[i];
     }
     if constexpr (SPLIT) {
         if (a.step_off > 0) {
@@ -846,40 +855,50 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE))) v
         }
         if constexpr (UMB) {
             // umbrella mode 0 at the centroid of this step's positions
-            // (src/verlet.f90:1046, src/umbrella.f90:109-173): one lane per
-            // trajectory evaluates it; every bead adds it, the force-constant
-            // part first.  That lane also sums xi and runs the window check
-            // (rpmd_check traj_type 2/3, src/rpmd_check.f90:74-112).
+            // (src/verlet.f90:1046, src/umbrella.f90:109-173): a group of
+            // lanes per trajectory evaluates it (xi_group.hpp); every bead
+            // adds it, the force-constant part first.  One lane per
+            // trajectory then sums xi and runs the window check (rpmd_check
+            // traj_type 2/3, src/rpmd_check.f90:74-112).
             bool qbad = false;
 #pragma unroll
             for (int s = 0; s < SL; ++s) qbad = qbad || (S::valid(s, r) && (q[s] != q[s] || q[s] > DBL_MAX));
             if (live && r == 0) uvb[tl * NB + k] = vb;
             if (live && qbad) ubad[tl] = 1;
             __syncthreads();
-            if (live && k == 0 && r == 0) {
-                double dxi[NC], gk[NC], gh[NC], xi1;
-                const double xw = a.uwin[2 * traj], kw = a.uwin[2 * traj + 1];
-                (void)umbrella_bias<S::NA>(a.rx, cent + tl * NC, beta, kw, xw, xi1, dxi, gk, gh);
-#pragma unroll
-                for (int i = 0; i < NC; ++i) {
-                    ubias[(2 * tl) * NC + i] = gk[i];
-                    ubias[(2 * tl + 1) * NC + i] = gh[i];
+            {
+                const int gi = tid % XG::GL;
+                for (int t = tid / XG::GL; t < TPB; t += NG) {
+                    const int tr = blockIdx.x * TPB + t;
+                    if (tr >= a.ntraj) break;
+                    auto &w = xw[tid / XG::GL];
+                    if (gi < NC) w.pts[gi] = cent[t * NC + gi];
+                    double xi1, gk, gh;
+                    XG::bias(xt, w, gi, a.beta[tr], a.uwin[2 * tr + 1], a.uwin[2 * tr], xi1, gk, gh);
+                    if (gi < NC) {
+                        ubias[(2 * t) * NC + gi] = gk;
+                        ubias[(2 * t + 1) * NC + gi] = gh;
+                    }
+                    if (gi == 0) uxi[t] = xi1;
                 }
+            }
+            __syncthreads();
+            // slots past the last trajectory hold a copy of it: not counted
+            if (act && k == 0 && r == 0) {
+                const double xi1 = uxi[tl], xw_ = a.uwin[2 * traj];
                 usum += xi1;
                 usq += xi1 * xi1;
-                // slots past the last trajectory evaluate a copy of it: not counted
-                if (act) count_xi(a.uhist, a.hbins, a.hmin, a.hinv, traj, xi1);
+                count_xi(a.uhist, a.hbins, a.hmin, a.hinv, traj, xi1);
                 const uint64_t istep = a.step_base[1] + (uint64_t)(a.step_off + it) + 1;
                 if (a.check_after >= 0 && istep > (uint64_t)a.check_after) {
                     double ep = 0.0;
                     for (int kk = 0; kk < NB; ++kk) ep = ep + uvb[tl * NB + kk];
                     const bool bad = ubad[tl] != 0 || ep != ep || ep > DBL_MAX || ep > a.epot_max ||
-                                     fabs(xi1 - xw) > a.xi_tol;
+                                     fabs(xi1 - xw_) > a.xi_tol;
                     if (bad) ucheck = true;
                 }
                 ubad[tl] = 0;
             }
-            __syncthreads();
 #pragma unroll
             for (int s = 0; s < SL; ++s)
                 if (S::valid(s, r)) g[s] = (g[s] + ubias[(2 * tl) * NC + cc[s]]) + ubias[(2 * tl + 1) * NC + cc[s]];
