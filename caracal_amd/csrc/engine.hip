@@ -143,14 +143,13 @@ __global__ void constrain_kernel(TrajArgs a, int project_p, int *status)
 }
 
 // ---------------------------------------------------------------------------
-// Recrossing parent (verlet with constrain = 1).  One wave per trajectory:
-// its lanes cover the beads of each coordinate, and the scalar work of the
-// constraint (xi, Newton's iteration) is repeated by every lane on the same
-// values, so no lane waits for a broadcast.  pdxi[traj][3*natoms] carries the
-// constraint direction from one step to the next; pfail holds per trajectory
-// kPfConstraint (a constraint did not converge since the start), kPfCheck
-// (the per-step trajectory check failed) and kPfThisStep (this step's
-// constraint did not converge).
+// Start of a recrossing parent (its steps are in step_kernels.hpp) and of a
+// window: one wave per trajectory, its lanes over the beads of each
+// coordinate, the scalar work repeated by every lane on the same values.
+// pdxi[traj][3*natoms] carries a parent's constraint direction from one launch
+// to the next; pfail holds per trajectory kPfConstraint (a constraint did not
+// converge since the start) and kPfCheck (the per-step trajectory check
+// failed).
 // ---------------------------------------------------------------------------
 
 // Centroid of trajectory t in every lane: lane i < 3*natoms sums coordinate
@@ -209,123 +208,6 @@ __global__ __launch_bounds__(64 * kParentWaves) void parent_begin_kernel(TrajArg
     const double mine = pick_lane<NC>(dxi, lane);
     if (lane < NC) pdxi[(size_t)t * NC + lane] = mine;
     if (lane == 0) pfail[t] = 0;
-}
-
-// Between the free ring-polymer step and the forces (src/verlet.f90:649,
-// :744-756): constrain_q (src/constrain_q.f90:35-113) on the centroid c of
-// the propagated beads with the previous step's direction, then the next
-// direction, the gradient of xi (mode 2) at the same c (umbrella mode 1,
-// src/verlet.f90:1048, src/umbrella.f90:117-122).  A constraint that does not
-// converge in 200 iterations leaves the beads as they are and is counted,
-// where the reference prints a warning and gives the step an energy penalty.
-template <int NA>
-__global__ __launch_bounds__(64 * kParentWaves) void parent_constrain_kernel(TrajArgs a, double *pdxi, int *pfail)
-{
-    constexpr int NC = 3 * NA;
-    const int lane = threadIdx.x % 64, t = blockIdx.x * kParentWaves + threadIdx.x / 64;
-    if (t >= a.ntraj) return;
-    const int NB = a.nbeads;
-    double *q = a.q + (size_t)t * NC * NB, *p = a.p + (size_t)t * NC * NB;
-    double c[NC], dprev[NC], qt[NC], dxn[NC];
-    wave_centroid<NA>(q, NB, lane, c);
-#pragma unroll
-    for (int i = 0; i < NC; ++i) dprev[i] = pdxi[(size_t)t * NC + i];
-    double mult = 0.0, coeff = 0.0;
-    bool good = true;
-    for (int iter = 1; iter <= 200; ++iter) {
-        coeff = mult * a.dt * a.dt / NB;
-#pragma unroll
-        for (int i = 0; i < NC; ++i) qt[i] = c[i] + coeff * dprev[i] / a.mass[i / 3];
-        const double sigma = calc_xi<NA>(a.rx, qt, dxn);
-        double dsigma = 0.0;
-        #pragma unroll
-        for (int d = 0; d < 3; ++d)
-            #pragma unroll
-            for (int at = 0; at < NA; ++at)
-                dsigma = dsigma + dxn[3 * at + d] * a.dt * a.dt * dprev[3 * at + d] / (a.mass[at] * NB);
-        const double dx = sigma / dsigma;
-        mult = mult - dx;
-        // single-precision literals 1.0E-8 and 1.0E-10 of the reference
-        if (fabs(dx) < (double)1.0e-8f || fabs(sigma) < (double)1.0e-10f) break;
-        if (iter == 200) good = false;
-    }
-    if (good) {
-        // the shift uses the coefficient of the last iteration, computed
-        // before its multiplier update, as the reference does
-#pragma unroll
-        for (int i = 0; i < NC; ++i) {
-            const double dq = coeff / a.mass[i / 3] * dprev[i], dp = mult * a.dt / NB * dprev[i];
-            for (int k = lane; k < NB; k += 64) {
-                q[(size_t)i * NB + k] = q[(size_t)i * NB + k] + dq;
-                p[(size_t)i * NB + k] = p[(size_t)i * NB + k] + dp;
-            }
-        }
-    }
-    if (lane == 0) pfail[t] = good ? (pfail[t] & ~kPfThisStep) : (pfail[t] | kPfConstraint | kPfThisStep);
-    double dnew[NC];
-    (void)calc_xi<NA>(a.rx, c, dnew);
-    const double mine = pick_lane<NC>(dnew, lane);
-    if (lane < NC) pdxi[(size_t)t * NC + lane] = mine;
-}
-
-// The end of a parent step (src/verlet.f90:1060-1083, :1159-1165): the
-// second half kick, constrain_p (src/constrain_p.f90:36-76) with this step's
-// direction, and the Andersen draw when the step number istep is a multiple
-// of andersen_step.  istep counts from the start (cam_engine_begin_parent,
-// first step 1), as the reference's verlet loops restart after each mdinit;
-// the draw is keyed by the steps since the engine's creation, so restarts
-// draw fresh momenta.
-// Then rpmd_check as the recrossing driver calls it for a parent
-// (src/rpmd_check.f90:74-98, traj_type 1 at src/recross_serial.f90:125-135
-// and :290-299), from step check_after + 1 after the start on (never if
-// check_after < 0): a position that is NaN or above HUGE, or an energy (the
-// sum over the beads, plus verlet's 1e5 penalty after a failed constraint,
-// src/verlet.f90:749-755) that is NaN, above HUGE or above epot_max, sets
-// kPfCheck.  step_base[1] counts the steps since the start.
-template <int NA>
-__global__ __launch_bounds__(64 * kParentWaves) void parent_end_kernel(TrajArgs a, const double *pdxi, int *pfail,
-                                                                       const uint64_t *step_base, int step_off,
-                                                                       int andersen_step, uint64_t seed,
-                                                                       double epot_max, int check_after)
-{
-    constexpr int NC = 3 * NA;
-    const int lane = threadIdx.x % 64, t = blockIdx.x * kParentWaves + threadIdx.x / 64;
-    if (t >= a.ntraj) return;
-    const int NB = a.nbeads;
-    double *p = a.p + (size_t)t * NC * NB;
-    const double *g = a.g + (size_t)t * NC * NB;
-    double dxi[NC];
-#pragma unroll
-    for (int i = 0; i < NC; ++i) dxi[i] = pdxi[(size_t)t * NC + i];
-    double c1 = 0.0, c2 = 0.0;
-#pragma unroll
-    for (int i = 0; i < NC; ++i)
-        for (int k = lane; k < NB; k += 64) {
-            const double pn = p[(size_t)i * NB + k] - 0.5 * a.dt * g[(size_t)i * NB + k];
-            p[(size_t)i * NB + k] = pn;
-            c1 = c1 + dxi[i] * pn / a.mass[i / 3];
-        }
-    for (int off = 32; off > 0; off >>= 1) c1 += __shfl_xor(c1, off, 64);
-    #pragma unroll
-    for (int d = 0; d < 3; ++d)
-        #pragma unroll
-        for (int at = 0; at < NA; ++at) c2 = c2 + dxi[3 * at + d] * dxi[3 * at + d] / a.mass[at];
-    const double lam = -c1 / c2 / NB;
-    const uint64_t istep = step_base[1] + (uint64_t)step_off + 1;
-    const uint64_t key = step_base[0] + (uint64_t)step_off + 1;
-    const bool draw = andersen_step > 0 && istep % (uint64_t)andersen_step == 0;
-    const double beta = a.beta[t];
-#pragma unroll
-    for (int i = 0; i < NC; ++i) {
-        const double sd = sqrt(a.mass[i / 3] / (beta / NB));
-        for (int k = lane; k < NB; k += 64)
-            p[(size_t)i * NB + k] = draw ? andersen_normal(seed, (uint32_t)t, key, i, k) * sd
-                                         : p[(size_t)i * NB + k] + lam * dxi[i];
-    }
-    if (check_after >= 0 && step_base[1] + (uint64_t)step_off + 1 > (uint64_t)check_after) {
-        const double penalty = (pfail[t] & kPfThisStep) ? 1.0e5 : 0.0;
-        if (trajectory_fails(a, t, lane, penalty, epot_max) && lane == 0) pfail[t] = pfail[t] | kPfCheck;
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -590,7 +472,7 @@ struct cam_engine {
     double *pdxi = nullptr;           // PARENT: constraint directions [traj][3*natoms]
     int *pfail = nullptr;             // PARENT, UMBRELLA: trajectory flags (kPf*)
     double *uwin = nullptr;           // UMBRELLA: (xi_ideal, k_force) per trajectory
-    XiTable *xitab = nullptr;         // UMBRELLA: the reaction coordinate's distances
+    XiTable *xitab = nullptr;         // PARENT, UMBRELLA: the reaction coordinate's distances
     double *ustat = nullptr;          // UMBRELLA: running sums of xi, xi^2 per trajectory
     double *nhc = nullptr;            // NHC: thermostat velocities [traj][4]
     long ustat_steps = 0;             // UMBRELLA: steps in those sums
@@ -731,12 +613,11 @@ bool select_kernels(cam_engine *e, int wpe, int nmk, Kernels &k)
 {
     const cam_config *cfg = &e->cfg;
     const int nb = cfg->nbeads;
-    // a parent's or window's split-schedule normal-mode kernel is the NVE
-    // one: its constraint or bias and the end of its step are kernels of
-    // their own.  Windows also have a fused step; parents do not.
+    // a window's split-schedule normal-mode kernel is the NVE one: its bias
+    // and the end of its step are a kernel of their own
     const bool steered = cfg->ensemble == CAM_ENS_PARENT || cfg->ensemble == CAM_ENS_UMBRELLA;
     const int ens_nm = steered || cfg->ensemble == CAM_ENS_NHC ? CAM_ENS_NVE : cfg->ensemble;
-    const int ens = cfg->ensemble == CAM_ENS_PARENT ? CAM_ENS_NVE : cfg->ensemble;
+    const int ens = cfg->ensemble;
     const bool mfma = nmk == CAM_NMK_MFMA;
     bool ok;
     if (cfg->surface == CAM_SURFACE_H3)
@@ -861,9 +742,10 @@ StepArgs step_args(cam_engine *e)
     a.ntraj = e->cfg.ntraj;
     a.tbegin = 0;
     a.tend = e->cfg.ntraj;
-    // ANDERSEN draws every andersen_step >= 1 steps; a window's 0 means never
-    // (the fused window step tests andersen_step > 0)
-    a.andersen_step = e->cfg.ensemble == CAM_ENS_UMBRELLA ? e->cfg.andersen_step
+    // ANDERSEN draws every andersen_step >= 1 steps; a window's or parent's 0
+    // means never (their steps test andersen_step > 0)
+    a.andersen_step = e->cfg.ensemble == CAM_ENS_UMBRELLA || e->cfg.ensemble == CAM_ENS_PARENT
+                          ? e->cfg.andersen_step
                                                           : (e->cfg.andersen_step > 0 ? e->cfg.andersen_step : 1);
     a.transrot = e->cfg.remove_com;
     // every atom counted once per bead, then times nbeads (src/transrot.f90:62-72)
@@ -885,36 +767,6 @@ hipError_t launch_steps(cam_engine *e, const Kernels &kn, bool split, int spl, S
 {
     const int grid = (e->cfg.ntraj + e->tpb - 1) / e->tpb;
     hipError_t err = hipSuccess;
-    if (e->cfg.ensemble == CAM_ENS_PARENT) {
-        // per step: kick and free ring polymer; constraint; forces; second
-        // half kick, constrain_p and Andersen
-        TrajArgs ta = traj_args(e);
-        ta.q = a.q;
-        ta.p = a.p;
-        ta.g = a.g;
-        const int pgrid = (e->cfg.ntraj + kParentWaves - 1) / kParentWaves;
-        for (int j = 0; j < nsteps && err == hipSuccess; ++j) {
-            a.nsteps = 1;
-            a.step_off = 0;                // no previous step to finish inside the kernel
-            hipLaunchKernelGGL(kn.nm, dim3(grid), dim3(kBlock), 0, e->stream, a);
-            err = hipGetLastError();
-            if (err != hipSuccess) break;
-            with_natoms(e->cfg.natoms, [&](auto na) {
-                hipLaunchKernelGGL(parent_constrain_kernel<decltype(na)::value>, dim3(pgrid), dim3(64 * kParentWaves), 0, e->stream, ta, a.pdxi, a.pfail);
-            });
-            err = hipGetLastError();
-            if (err != hipSuccess) break;
-            hipLaunchKernelGGL(kn.fsplit, dim3(grid), dim3(kBlock), 0, e->stream, a.q, a.g, a.vbead, a.ntraj);
-            err = hipGetLastError();
-            if (err != hipSuccess) break;
-            const int as = e->cfg.andersen_step;
-            with_natoms(e->cfg.natoms, [&](auto na) {
-                hipLaunchKernelGGL(parent_end_kernel<decltype(na)::value>, dim3(pgrid), dim3(64 * kParentWaves), 0, e->stream, ta, a.pdxi, a.pfail, a.step_base, j, as, a.seed, e->pcheck_max, e->pcheck_after);
-            });
-            err = hipGetLastError();
-        }
-        return err;
-    }
     if (e->cfg.ensemble == CAM_ENS_UMBRELLA && split) {
         // per step: kick and free ring polymer; forces; bias, sums, second half kick, Andersen
         TrajArgs ta = traj_args(e);
@@ -1126,7 +978,7 @@ int cam_engine_create(const cam_config *cfg, cam_engine **out)
     e->wpe = ch4h64 && (cfg->waves_per_eu == 2 || (cfg->waves_per_eu == 0 && e->nmk == CAM_NMK_FOLDED)) ? 2 : 1;
     // windows run fused unless split is asked for or MFMA normal modes are
     // (their fused step has the vector-ALU transform only)
-    e->split = cfg->schedule == CAM_SCHED_SPLIT || cfg->ensemble == CAM_ENS_PARENT ||
+    e->split = (cfg->schedule == CAM_SCHED_SPLIT && cfg->ensemble != CAM_ENS_PARENT) ||
                (cfg->ensemble == CAM_ENS_UMBRELLA && e->nmk == CAM_NMK_MFMA);
     const bool ok = select_kernels(e.get(), e->wpe, e->nmk, e->kern);
     if (!ok) {
@@ -1150,6 +1002,9 @@ int cam_engine_create(const cam_config *cfg, cam_engine **out)
         CAM_HIP(hipMalloc(&e->cbuf, steps * cfg->ntraj * 3 * na * sizeof(double)));
     }
     if (steered) {
+        const XiTable xt = xi_table(rx, na);
+        CAM_HIP(hipMalloc(&e->xitab, sizeof xt));
+        CAM_HIP(hipMemcpy(e->xitab, &xt, sizeof xt, hipMemcpyHostToDevice));
         CAM_HIP(hipMalloc(&e->pfail, (size_t)cfg->ntraj * sizeof(int)));
         CAM_HIP(hipMemset(e->pfail, 0, (size_t)cfg->ntraj * sizeof(int)));
     }
@@ -1167,9 +1022,6 @@ int cam_engine_create(const cam_config *cfg, cam_engine **out)
         for (int t = 0; t < cfg->ntraj; ++t) w[2 * (size_t)t] = rx.xi_ideal;
         CAM_HIP(hipMalloc(&e->uwin, w.size() * sizeof(double)));
         CAM_HIP(hipMemcpy(e->uwin, w.data(), w.size() * sizeof(double), hipMemcpyHostToDevice));
-        const XiTable xt = xi_table(rx, na);
-        CAM_HIP(hipMalloc(&e->xitab, sizeof xt));
-        CAM_HIP(hipMemcpy(e->xitab, &xt, sizeof xt, hipMemcpyHostToDevice));
         CAM_HIP(hipMalloc(&e->ustat, w.size() * sizeof(double)));
         CAM_HIP(hipMemset(e->ustat, 0, w.size() * sizeof(double)));
     }
@@ -1534,7 +1386,7 @@ int cam_engine_run(cam_engine *e, int nsteps)
     if (nsteps == 0) return CAM_OK;
     // Long runs replay a graph of at most kGraphLaunches step launches (and
     // one graph of the remainder) instead of capturing every step into one
-    // graph: a split-schedule step is three or four launches, a fused launch
+    // graph: a split-schedule step is two to four launches, a fused launch
     // spl steps.
     const int steps_per_graph = (e->split ? 1 : e->spl) * kGraphLaunches;
     const int chunk = std::min(nsteps, steps_per_graph);
@@ -1684,7 +1536,9 @@ static int autotune(cam_engine *e, int trial_steps, cam_tuning *out, bool slices
             for (int wpe : wpes)
                 if (!vfused || wpe == 1)
                     for (int spl : spls) cand.push_back({ nmk, wpe, spl, 0, 0.0 });
-        if (try_split) cand.push_back({ nmk, 1, 1, 1, 0.0 });
+        if (parent)                         // one schedule, reported as split; its transform unit is the choice
+            cand.push_back({ nmk, 1, c.steps_per_launch > 0 ? c.steps_per_launch : e->spl, 0, 0.0 });
+        else if (try_split) cand.push_back({ nmk, 1, 1, 1, 0.0 });
     }
     auto fail = [&](hipError_t err) {
         set_error("HIP error in autotune: %s", hipGetErrorString(err));
@@ -1772,7 +1626,7 @@ static int autotune(cam_engine *e, int trial_steps, cam_tuning *out, bool slices
             out->nm_kernel[i] = trials[i].nmk;
             out->steps_per_launch[i] = trials[i].spl;
             out->waves_per_eu[i] = trials[i].wpe;
-            out->split[i] = trials[i].split;
+            out->split[i] = parent ? 1 : trials[i].split;
             out->us_per_step[i] = trials[i].us;
         }
     }

@@ -115,7 +115,7 @@ struct StepArgs {
     int *pfail;                  // PARENT, UMBRELLA: trajectory flags
     double *ustat;               // UMBRELLA: running sums of xi and xi^2 [traj][2]
     const double *uwin;          // UMBRELLA: (xi_ideal, k_force) of each trajectory's window
-    const XiTable *xitab;        // UMBRELLA: the reaction coordinate as a list of distances
+    const XiTable *xitab;        // PARENT, UMBRELLA: the reaction coordinate as a list of distances
     double epot_max, xi_tol;     // PARENT, UMBRELLA: trajectory check
     int check_after;             //   armed after this many steps (never if < 0)
     double *nhc;                 // NHC: thermostat velocities [traj][4]

@@ -23,11 +23,10 @@ namespace {
 // per-trajectory kernels, step launches per captured graph (a split-schedule
 // step is one launch sequence; a fused launch advances steps_per_launch
 // steps), and the bits of the per-trajectory flags (a constraint did not
-// converge since the start; the trajectory check failed; this step's
-// constraint did not converge).
+// converge since the start; the trajectory check failed).
 constexpr int kParentWaves = 4;
 constexpr int kGraphLaunches = 1000;
-constexpr int kPfConstraint = 1, kPfCheck = 2, kPfThisStep = 4;
+constexpr int kPfConstraint = 1, kPfCheck = 2;
 // Folded launches of at least 2 x kSliceMinBlocks blocks (the CU count) are
 // issued as two trajectory slices on two streams (launch_steps).
 constexpr int kSliceMinBlocks = 256;
@@ -444,11 +443,19 @@ __device__ __forceinline__ void nm_mfma(double *xs, double *ys, const double *pr
 
 // ---------------------------------------------------------------------------
 // The step kernel.  ENS: CAM_ENS_NVE, CAM_ENS_ANDERSEN, CAM_ENS_CHILD,
-// CAM_ENS_UMBRELLA or CAM_ENS_NHC (the chain before the first and after the
-// second half kick).  One step: p -= dt/2 g; free ring-polymer propagation in
-// normal-mode space; [CHILD: xi of the centroid]; forces; [UMBRELLA: the
-// window's bias at the centroid, added to every bead]; p -= dt/2 g;
-// [ANDERSEN, UMBRELLA: resample].
+// CAM_ENS_UMBRELLA, CAM_ENS_PARENT or CAM_ENS_NHC (the chain before the first
+// and after the second half kick).  One step: p -= dt/2 g; free ring-polymer
+// propagation in normal-mode space; [CHILD: xi of the centroid]; [PARENT:
+// constrain_q]; forces; [UMBRELLA: the window's bias at the centroid, added to
+// every bead]; p -= dt/2 g; [PARENT: constrain_p]; [ANDERSEN, UMBRELLA,
+// PARENT: resample].
+//
+// PARENT (verlet with constrain = 1): constrain_q and the next step's
+// direction by a group of lanes per trajectory on the centroid the transform
+// left in LDS, constrain_p's flux as a sum over the block's lanes, the
+// direction in LDS from step to step.  As four launches a step, two of them
+// one wave per trajectory, 64 parents of 16 CH5 beads took 57 us a step, 39 of
+// them in those two; in the step loop 15 us.
 //
 // SPLIT: the same step without its force phase, one step per launch, for the
 // split schedule (forces in force_kernel at its own register budget).  The
@@ -480,24 +487,31 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE))) v
     __shared__ double wcom[ENS == CAM_ENS_CHILD ? CAM_MAX_REAC : 1][S::NA];
     // UMBRELLA: the two parts of each trajectory's bias gradient, its bead
     // energies and a flag for positions that are not finite
-    constexpr bool UMB = ENS == CAM_ENS_UMBRELLA;
-    constexpr bool CENT = ENS == CAM_ENS_CHILD || UMB;
+    constexpr bool UMB = ENS == CAM_ENS_UMBRELLA, PAR = ENS == CAM_ENS_PARENT, XI = UMB || PAR;
+    constexpr bool CENT = ENS == CAM_ENS_CHILD || XI;
     using XG = XiGroup<S::NA>;
     constexpr int NG = kBlock / XG::GL;      // groups of lanes, a trajectory each
-    __shared__ typename std::conditional<UMB, XiTable, int>::type xt;
-    __shared__ typename std::conditional<UMB, typename XG::Work, int>::type xw[UMB ? NG : 1];
+    __shared__ typename std::conditional<XI, XiTable, int>::type xt;
+    __shared__ typename std::conditional<XI, typename XG::Work, int>::type xw[XI ? NG : 1];
     __shared__ double uxi[UMB ? TPB : 1];
     __shared__ double ubias[UMB ? TPB * 2 * NC : 1];
-    __shared__ double uvb[UMB ? TPB * NB : 1];
-    __shared__ int ubad[UMB ? TPB : 1];
+    __shared__ double uvb[XI ? TPB * NB : 1];
+    __shared__ int ubad[XI ? TPB : 1];
+    // PARENT: constraint direction, the step's shifts of q and p, whether its
+    // constraint converged, and |direction|^2 over the masses
+    __shared__ double pdir[PAR ? TPB * NC : 1];
+    __shared__ double pshift[PAR ? TPB * 2 * NC : 1];
+    __shared__ int pgood[PAR ? TPB : 1];
+    __shared__ double pnorm[PAR ? TPB : 1];
     // NHC: the lanes' kinetic-energy parts and each trajectory's scale factor
     constexpr bool NHC = ENS == CAM_ENS_NHC;
     __shared__ double nred[NHC ? kBlock : 1];
     __shared__ double nscale[NHC ? TPB : 1];
     // transrot after every step (not for children, and not in the split
     // schedule's kernel): the sums of each trajectory
-    constexpr bool TRANSROT = !SPLIT && ENS != CAM_ENS_CHILD;
-    __shared__ double trsum[TRANSROT && NB > 1 ? TPB * 9 : 1];
+    constexpr bool TRANSROT = !SPLIT && ENS != CAM_ENS_CHILD && !PAR;
+    constexpr bool TSUM = (TRANSROT || PAR) && NB > 1;
+    __shared__ double trsum[TSUM ? TPB * 9 : 1];
 
     const int tid = threadIdx.x;
     const int r = tid % L;
@@ -552,7 +566,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE))) v
     const double hdt = 0.5 * a.dt;
     double vb = 0.0;
     double usum = 0.0, usq = 0.0;            // UMBRELLA: this launch's sums of xi, xi^2
-    bool ucheck = false;                     // UMBRELLA: the window check failed in this launch
+    bool ucheck = false;                     // UMBRELLA, PARENT: the trajectory check failed in this launch
+    bool pfailed = false;                    // PARENT: a constraint did not converge in this launch
     // NHC: the chain of this lane's trajectory lives in the registers of its
     // bead-0 lane for the launch; masses and kT as mdinit and nhc set them
     // (src/mdinit.f90:139-146; src/nhc.f90:53, a default-REAL quotient)
@@ -628,7 +643,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE))) v
     // lane of a bead), on every lane, in a fixed order: staged in the
     // normal-mode columns, added by four lanes per sum.
     [[maybe_unused]] auto traj_sum = [&](auto nv, double *v) {
-        if constexpr (TRANSROT && NB > 1) {
+        if constexpr (TSUM) {
             constexpr int NV = decltype(nv)::value, P = NB % 4 == 0 ? 4 : 2, Q = NB / P;
             static_assert(XS >= TPB * NB * NV && NB % P == 0, "the column buffer holds nine values per bead");
             __syncthreads();                          // the transform's reads, and the last sums' reads
@@ -655,11 +670,15 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE))) v
             for (int i = 0; i < NV; ++i) v[i] = trsum[tl * NV + i];
         }
     };
-    if constexpr (UMB) {
+    if constexpr (XI) {
         for (int i = tid; i < TPB; i += kBlock) ubad[i] = 0;
         static_assert(sizeof(XiTable) % 4 == 0, "copied word by word");
         for (int i = tid; i < (int)(sizeof(XiTable) / 4); i += kBlock)
             reinterpret_cast<int *>(&xt)[i] = reinterpret_cast<const int *>(a.xitab)[i];
+        if constexpr (PAR)
+            for (int i = tid; i < TPB * NC; i += kBlock)
+                pdir[i] = a.pdxi[(size_t)min((int)blockIdx.x * TPB + i / NC, a.ntraj - 1) * NC + i % NC];
+        __syncthreads();
     }
     if constexpr (SPLIT) {
         if (a.step_off > 0) {
@@ -825,11 +844,66 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE))) v
             }
         }
 
-        if constexpr (UMB && NB == 1) {
+        if constexpr (XI && NB == 1) {
             __syncthreads();
 #pragma unroll
             for (int s = 0; s < SL; ++s)
                 if (S::valid(s, r)) cent[tl * NC + cc[s]] = q[s];
+        }
+        if constexpr (PAR) {
+            // constrain_q (src/verlet.f90:649, :744-756, src/constrain_q.f90:35-113)
+            // on the centroid c of the propagated beads with the previous
+            // step's direction, and the next direction, the gradient of xi
+            // (mode 2) at the same c (src/verlet.f90:1048,
+            // src/umbrella.f90:117-122): the gradient of the first iteration,
+            // which starts at c.  The shift uses the coefficient of the last
+            // iteration, computed before its multiplier update, as the
+            // reference does.  A constraint that does not converge in 200
+            // iterations leaves the beads as they are and is counted, where
+            // the reference prints a warning and gives the step an energy
+            // penalty.
+            if constexpr (NB == 1) __syncthreads();
+            const int gi = tid % XG::GL;
+            for (int t = tid / XG::GL; t < TPB; t += NG) {
+                if ((int)blockIdx.x * TPB + t >= a.ntraj) break;
+                auto &w = xw[tid / XG::GL];
+                const bool on = gi < NC;
+                const double c = on ? cent[t * NC + gi] : 0.0, dprev = on ? pdir[t * NC + gi] : 0.0;
+                const double dm = on ? dprev * xt.inv_mass[gi / 3] : 0.0;
+                double mult = 0.0, coeff = 0.0, dnew = 0.0;
+                bool good = true;
+                for (int iter = 1; iter <= 200; ++iter) {
+                    coeff = mult * a.dt * a.dt / NB;
+                    if (on) w.pts[gi] = c + coeff * dm;
+                    double s0, s1, ds0, ds1;
+                    XG::surfaces(xt, w, gi, s0, s1, ds0, ds1);
+                    const double sigma = a.rx.xi_ideal * s1 + (1.0 - a.rx.xi_ideal) * s0;
+                    const double dxn = a.rx.xi_ideal * ds1 + (1.0 - a.rx.xi_ideal) * ds0;
+                    if (iter == 1) dnew = dxn;
+                    const double dx = sigma / (XG::sum(dxn * dm) * (a.dt * a.dt / NB));
+                    mult = mult - dx;
+                    // single-precision literals 1.0E-8 and 1.0E-10 of the reference
+                    if (fabs(dx) < (double)1.0e-8f || fabs(sigma) < (double)1.0e-10f) break;
+                    if (iter == 200) good = false;
+                }
+                const double n2 = XG::sum(on ? dnew * dnew * xt.inv_mass[gi / 3] : 0.0);
+                if (on) {
+                    pdir[t * NC + gi] = dnew;
+                    pshift[(2 * t) * NC + gi] = good ? coeff * dm : 0.0;
+                    pshift[(2 * t + 1) * NC + gi] = good ? mult * a.dt / NB * dprev : 0.0;
+                }
+                if (gi == 0) {
+                    pgood[t] = good;
+                    pnorm[t] = n2;
+                }
+            }
+            __syncthreads();
+#pragma unroll
+            for (int s = 0; s < SL; ++s)
+                if (S::valid(s, r)) {
+                    q[s] = q[s] + pshift[(2 * tl) * NC + cc[s]];
+                    p[s] = p[s] + pshift[(2 * tl + 1) * NC + cc[s]];
+                }
         }
         if constexpr (SPLIT) continue;     // one step per launch; forces come next
         // forces of every bead (src/verlet.f90:772-777)
@@ -907,6 +981,55 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE))) v
 #pragma unroll
         for (int s = 0; s < SL; ++s) p[s] = p[s] - hdt * g[s];
 
+        if constexpr (PAR) {
+            // constrain_p (src/constrain_p.f90:36-76) with this step's
+            // direction, or the Andersen draw when the step number since
+            // begin_parent is a multiple of andersen_step (src/verlet.f90:1081,
+            // :1159-1165; the draw keyed by the steps since the engine's
+            // creation, so restarts draw fresh momenta).  Then rpmd_check as the
+            // recrossing driver calls it for a parent (src/rpmd_check.f90:74-98,
+            // traj_type 1 at src/recross_serial.f90:125-135 and :290-299): a
+            // position that is NaN or above HUGE, or an energy (the sum over the
+            // beads, plus verlet's 1e5 penalty after a failed constraint,
+            // src/verlet.f90:749-755) that is NaN, above HUGE or above epot_max.
+            bool qbad = false;
+            double flux = 0.0;
+#pragma unroll
+            for (int s = 0; s < SL; ++s)
+                if (S::valid(s, r)) {
+                    qbad = qbad || q[s] != q[s] || q[s] > DBL_MAX;
+                    flux += pdir[tl * NC + cc[s]] * p[s] * xt.inv_mass[cc[s] / 3];
+                }
+            if (live && r == 0) uvb[tl * NB + k] = vb;
+            if (live && qbad) ubad[tl] = 1;
+            if constexpr (L == 4) flux = quad::sum(flux);
+            traj_sum(std::integral_constant<int, 1>{}, &flux);
+            if constexpr (NB == 1) __syncthreads();
+            const uint64_t istep = a.step_base[1] + (uint64_t)(a.step_off + it) + 1;
+            if (a.andersen_step > 0 && istep % (uint64_t)a.andersen_step == 0) {
+                const uint64_t key = a.step_base[0] + (uint64_t)(a.step_off + it) + 1;
+#pragma unroll
+                for (int s = 0; s < SL; ++s) {
+                    const double sd = sqrt((TAB ? smass[cc[s] / 3] : m[s]) / (beta / NB));
+                    p[s] = andersen_normal(a.seed, (uint32_t)traj, key, cc[s], k) * sd;
+                }
+            } else {
+                const double lam = -flux / pnorm[tl] / NB;
+#pragma unroll
+                for (int s = 0; s < SL; ++s)
+                    if (S::valid(s, r)) p[s] = p[s] + lam * pdir[tl * NC + cc[s]];
+            }
+            if (act && k == 0 && r == 0) {
+                const bool good = pgood[tl] != 0;
+                pfailed = pfailed || !good;
+                if (a.check_after >= 0 && istep > (uint64_t)a.check_after) {
+                    double ep = good ? 0.0 : 1.0e5;
+                    for (int kk = 0; kk < NB; ++kk) ep = ep + uvb[tl * NB + kk];
+                    if (ubad[tl] != 0 || ep != ep || ep > DBL_MAX || ep > a.epot_max) ucheck = true;
+                }
+                ubad[tl] = 0;
+            }
+        }
         if constexpr (NHC) nhc_apply();             // src/verlet.f90:1086-1106
         if constexpr (UMB) {
             // Andersen every andersen_step steps counted from the segment's
@@ -985,6 +1108,13 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE))) v
                 a.ustat[2 * traj + 1] = a.ustat[2 * traj + 1] + usq;
                 if (ucheck) a.pfail[traj] = a.pfail[traj] | kPfCheck;
             }
+        }
+        if constexpr (PAR) {
+            if (k == 0 && r == 0 && (ucheck || pfailed))
+                a.pfail[traj] = a.pfail[traj] | (ucheck ? kPfCheck : 0) | (pfailed ? kPfConstraint : 0);
+#pragma unroll
+            for (int s = 0; s < SL; ++s)
+                if (S::valid(s, r) && k == 0) a.pdxi[(size_t)traj * NC + cc[s]] = pdir[tl * NC + cc[s]];
         }
     }
 }
@@ -1070,11 +1200,14 @@ template <class S, int NB, typename T, int WPE, bool SPLIT = false>
 step_fn pick_step_w(int ens, bool mfma)
 {
     constexpr bool MF = mfma_bead_count(NB);
-    // umbrella windows and the Nose-Hoover chain: the fused step only, with
-    // the vector-ALU transform
+    // umbrella windows, parents and the Nose-Hoover chain: the fused step
+    // only, windows and the chain with the vector-ALU transform
     if constexpr (!SPLIT && WPE == 1) {
         if (ens == CAM_ENS_UMBRELLA) return step_kernel<S, NB, T, CAM_ENS_UMBRELLA, 1, false, false>;
         if (ens == CAM_ENS_NHC) return step_kernel<S, NB, T, CAM_ENS_NHC, 1, false, false>;
+        if (ens == CAM_ENS_PARENT)
+            return mfma && MF ? step_kernel<S, NB, T, CAM_ENS_PARENT, 1, MF, false>
+                              : step_kernel<S, NB, T, CAM_ENS_PARENT, 1, false, false>;
     }
     if (mfma && MF) {
         if (ens == CAM_ENS_NVE) return step_kernel<S, NB, T, CAM_ENS_NVE, WPE, MF, SPLIT>;
@@ -1093,7 +1226,8 @@ template <class S, int NB, typename T>
 step_fn pick_step(int ens, int wpe, bool mfma)
 {
     if constexpr (S::L == 4 && std::is_same<T, double>::value)
-        if (wpe == 2 && ens != CAM_ENS_UMBRELLA && ens != CAM_ENS_NHC) return pick_step_w<S, NB, T, 2>(ens, mfma);
+        if (wpe == 2 && ens != CAM_ENS_UMBRELLA && ens != CAM_ENS_NHC && ens != CAM_ENS_PARENT)
+            return pick_step_w<S, NB, T, 2>(ens, mfma);
     return pick_step_w<S, NB, T, 1>(ens, mfma);
 }
 

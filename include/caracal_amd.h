@@ -124,8 +124,10 @@ enum { CAM_NM_REFERENCE = 0, CAM_NM_ORTHOGONAL = 1 };
  *              on the dividing surface (constrain_q before the forces,
  *              constrain_p after the second half kick) and, if
  *              andersen_step > 0, the momenta are redrawn every andersen_step
- *              steps.  Runs on the split schedule; start it with
- *              cam_engine_begin_parent;
+ *              steps.  It has one schedule, its whole step inside one kernel
+ *              that advances steps_per_launch steps, chosen by AUTO and SPLIT
+ *              (FUSED is rejected) and reported as split by the autotuner;
+ *              start it with cam_engine_begin_parent;
  *  UMBRELLA -- umbrella-sampling window trajectories (verlet with constrain
  *              = 0 in the sampling loops of src/calc_rate.f90:1556-1645):
  *              after the forces, the umbrella bias of the centroid
