@@ -453,6 +453,7 @@ using namespace cam;
 struct Kernels {
     step_fn step = nullptr, nm = nullptr;
     force_fn force = nullptr, fsplit = nullptr;
+    int tpb = 1;                      // trajectories per block of force, nm and fsplit
     int step_tpb = 1;                 // trajectories per block of step
     bool folded = false;              // step is a folded kernel (takes a trajectory range)
 };
@@ -501,7 +502,6 @@ struct cam_engine {
     double last_ms = 0.0;
     int last_launches = 0;            // step launches of the last cam_engine_run
     long last_steps = 0;              // steps of the last cam_engine_run
-    int tpb = 1;                      // trajectories per block of the step kernel
 };
 
 namespace {
@@ -574,7 +574,7 @@ bool fold_available(const cam_config *cfg)
 {
     int tpb = 0;
     return fold_eligible(cfg) &&
-           fold_step_kernel_for(cfg->surface, cfg->precision, cfg->nbeads, cfg->ensemble, 1, 1, &tpb) != nullptr;
+           fold_step_kernel_for(cfg->surface, cfg->precision, cfg->nbeads, cfg->ensemble, 1, 1, false, &tpb) != nullptr;
 }
 
 // The distances of the reaction coordinate (xi_group.hpp): breaking bonds,
@@ -609,6 +609,28 @@ XiTable xi_table(const Rx &rx, int natoms)
     return t;
 }
 
+// Whether the H3, OH3, BrH2 and O3 kernels of an engine take four lanes per
+// bead (CH5 always does).  With few beads a step is the latency of one wave's
+// serial surface evaluation and transform, a third of it on four lanes; with
+// many, the lane that has no atom and the terms repeated on every lane cost
+// throughput.  The line is in blocks of the four-lane kernels: up to six
+// waves per SIMD folded, the two that fit unfolded, and one for BrH2, whose
+// eigenproblem is repeated on every lane.  us per step, one lane -> four:
+//   folded   H3  100 x 8  14.1 ->  5.0   4096 x 32 (1366 blocks) 17.9 -> 14.9   16384 x 32 (5462) 38 -> 51
+//            O3  100 x 8  12.5 ->  4.1   4096 x 32               19.8 -> 12.5   2048 x 64 (2048)  18 -> 23
+//            OH3 100 x 8  15.3 ->  5.7   4096 x 32               19.3 -> 18.6   16384 x 32        42 -> 62
+//            BrH2 512 x 32 (171) 11.5 -> 8.5   2048 x 32 (683) 11.8 -> 18.9
+//   Andersen H3  512 x 64 (512) 41.8 -> 24.3   2048 x 24 (1024) 25.6 -> 23.8   8192 x 8 (1024) 15.6 -> 17.7
+//            O3  512 x 64 (512) 29.9 -> 23.5   2048 x 24 (1024) 15.2 -> 22.7
+//            BrH2 512 x 24 (256) 25.5 -> 13.8  2048 x 24 (1024) 26.7 -> 37.6
+bool quad_lanes(const cam_config *cfg, bool folded)
+{
+    if (cfg->surface == CAM_SURFACE_CH4H) return true;
+    const int per_block = kBlock / 4 / (folded ? cfg->nbeads / 2 + 1 : cfg->nbeads);
+    const int limit = cfg->surface == CAM_SURFACE_BRH2 ? 256 : folded ? 1536 : 512;
+    return (cfg->ntraj + per_block - 1) / per_block <= limit;
+}
+
 bool select_kernels(cam_engine *e, int wpe, int nmk, Kernels &k)
 {
     const cam_config *cfg = &e->cfg;
@@ -620,17 +642,20 @@ bool select_kernels(cam_engine *e, int wpe, int nmk, Kernels &k)
     const int ens = cfg->ensemble;
     const bool mfma = nmk == CAM_NMK_MFMA;
     bool ok;
+    const bool quad = quad_lanes(cfg, nmk == CAM_NMK_FOLDED);
     if (cfg->surface == CAM_SURFACE_H3)
-        ok = pick_kernels_h3(cfg->precision, nb, ens, ens_nm, wpe, mfma, k.step, k.force, k.nm, k.fsplit);
+        ok = (quad ? pick_kernels_h3_quad : pick_kernels_h3)(cfg->precision, nb, ens, ens_nm, wpe, mfma, k.step,
+                                                             k.force, k.nm, k.fsplit);
     else if (cfg->surface == CAM_SURFACE_CH4H)
         ok = pick_kernels_ch4h(cfg->precision, nb, ens, ens_nm, wpe, mfma, k.step, k.force, k.nm, k.fsplit);
     else
-        ok = pick_kernels_fp64(cfg->surface, nb, ens, ens_nm, wpe, mfma, k.step, k.force, k.nm, k.fsplit);
-    k.step_tpb = e->tpb;
+        ok = (quad ? pick_kernels_fp64_quad : pick_kernels_fp64)(cfg->surface, nb, ens, ens_nm, wpe, mfma, k.step,
+                                                                 k.force, k.nm, k.fsplit);
+    k.tpb = k.step_tpb = kBlock / ((quad ? 4 : 1) * nb);
     if (ok && nmk == CAM_NMK_FOLDED) {
         int tpb = 0;
         const step_fn f =
-            fold_eligible(cfg) ? fold_step_kernel_for(cfg->surface, cfg->precision, nb, ens, wpe, e->fold_nbuf, &tpb)
+            fold_eligible(cfg) ? fold_step_kernel_for(cfg->surface, cfg->precision, nb, ens, wpe, e->fold_nbuf, quad, &tpb)
                                : nullptr;
         if (!f) return false;
         k.step = f;
@@ -659,7 +684,7 @@ TrajArgs traj_args(cam_engine *e)
 
 int run_forces(cam_engine *e)
 {
-    const int grid = (e->cfg.ntraj + e->tpb - 1) / e->tpb;
+    const int grid = (e->cfg.ntraj + e->kern.tpb - 1) / e->kern.tpb;
     hipLaunchKernelGGL(e->kern.force, dim3(grid), dim3(kBlock), 0, e->stream, e->q, e->g, e->vbead, e->cfg.ntraj);
     CAM_LAUNCH_CHECK();
     return CAM_OK;
@@ -765,7 +790,7 @@ StepArgs step_args(cam_engine *e)
 hipError_t launch_steps(cam_engine *e, const Kernels &kn, bool split, int spl, StepArgs a, int nsteps,
                         bool slices = true)
 {
-    const int grid = (e->cfg.ntraj + e->tpb - 1) / e->tpb;
+    const int grid = (e->cfg.ntraj + kn.tpb - 1) / kn.tpb;
     hipError_t err = hipSuccess;
     if (e->cfg.ensemble == CAM_ENS_UMBRELLA && split) {
         // per step: kick and free ring polymer; forces; bias, sums, second half kick, Andersen
@@ -966,8 +991,6 @@ int cam_engine_create(const cam_config *cfg, cam_engine **out)
     std::unique_ptr<cam_engine> e(new cam_engine());
     e->cfg = *cfg;
     e->rx = rx;
-    const int L = surf == CAM_SURFACE_CH4H ? 4 : 1;
-    e->tpb = kBlock / (L * nb);
     // steps fused per launch: state stays in registers for this many steps
     e->spl = cfg->steps_per_launch > 0 ? cfg->steps_per_launch : 50;
     if (cfg->nm_kernel != CAM_NMK_AUTO) e->nmk = cfg->nm_kernel;

@@ -11,6 +11,8 @@ namespace cam {
 step_fn fold_kernel_ch4h(int precision, int nbeads, int ensemble, int wpe, int *tpb);
 step_fn fold_kernel_h3(int precision, int nbeads, int ensemble, int nbuf, int *tpb);
 
+step_fn fold_kernel_quad(int surface, int precision, int nbeads, int ensemble, int *tpb);
+
 template <class S>
 step_fn fold_fp64(int nbeads, int ensemble, int nbuf, int *tpb)
 {
@@ -18,10 +20,13 @@ step_fn fold_fp64(int nbeads, int ensemble, int nbuf, int *tpb)
                      : fold::pick_fold_w<S, double, 1, 1>(nbeads, ensemble, tpb);
 }
 
-step_fn fold_step_kernel_for(int surface, int precision, int nbeads, int ensemble, int wpe, int nbuf, int *tpb)
+step_fn fold_step_kernel_for(int surface, int precision, int nbeads, int ensemble, int wpe, int nbuf, bool quad,
+                             int *tpb)
 {
     if (ensemble != CAM_ENS_NVE && ensemble != CAM_ENS_CHILD) return nullptr;
     const bool f64 = precision == CAM_PREC_FP64;
+    if (quad && surface != CAM_SURFACE_CH4H)
+        return f64 || surface == CAM_SURFACE_H3 ? fold_kernel_quad(surface, precision, nbeads, ensemble, tpb) : nullptr;
     if (surface == CAM_SURFACE_H3) return fold_kernel_h3(precision, nbeads, ensemble, nbuf, tpb);
     if (surface == CAM_SURFACE_OH3) return f64 ? fold_fp64<SurfOH3>(nbeads, ensemble, nbuf, tpb) : nullptr;
     if (surface == CAM_SURFACE_BRH2) return f64 ? fold_fp64<SurfBrH2>(nbeads, ensemble, nbuf, tpb) : nullptr;

@@ -20,6 +20,7 @@
 // the accurate one there (within 1e-14 of an 80-bit evaluation where
 // EISPACK's derivatives are off by up to 6e-11).
 #pragma once
+#include "quad.hpp"
 
 namespace cam {
 namespace brh2 {
@@ -35,11 +36,11 @@ constexpr double kXib = 0.5 * (kXih + kXix), kC3 = 1.0 / 3.0;
 constexpr double kGr = kG / kRhx;
 constexpr double kRt34 = 0.25 * 1.7320508075688772, kRt38 = 0.5 * kRt34;
 
-// HBr curves at r: (1S, 3S, 1P, 3P) and their r-derivatives
-__device__ inline void vhx(double r, double v[4], double dv[4])
+// HBr curves at rdif = r - Re with exp(-A rdif) and exp(-B rdif^3): (1S, 3S,
+// 1P, 3P) and their r-derivatives
+__device__ inline void vhx(double rdif, double ex1, double ex2, double v[4], double dv[4])
 {
-    const double rdif = r - kRhx, rdif2 = rdif * rdif;
-    const double ex1 = exp(-kAhx * rdif), ex2 = exp(-kBhx * rdif2 * rdif);
+    const double rdif2 = rdif * rdif;
     const double t1 = kDhx * ex1 * ex2, v1 = t1 * (ex1 + 2.0);
     v[0] = t1 * (ex1 - 2.0);
     v[1] = kEta3S * v1;
@@ -56,30 +57,46 @@ __device__ inline void vhx(double r, double v[4], double dv[4])
 // packed lower triangle, row-wise (0-based)
 __host__ __device__ constexpr int pk(int i, int j) { return i >= j ? i * (i + 1) / 2 + j : j * (j + 1) / 2 + i; }
 
-// One Jacobi rotation in the (P, Q) plane of the packed symmetric matrix a,
-// accumulated into the eigenvector columns v[.][P], v[.][Q].
-template <int P, int Q>
-__device__ inline void rotate(double a[10], double v[4][4])
+// Tangent and cosine of the Jacobi rotation that clears apq.
+__device__ inline void rotation(double app, double aqq, double apq, double &t, double &c)
 {
-    const double apq = a[pk(P, Q)];
-    if (apq == 0.0) return;
-    const double theta = (a[pk(Q, Q)] - a[pk(P, P)]) / (2.0 * apq);
-    double t = 1.0 / (fabs(theta) + sqrt(theta * theta + 1.0));
-    t = theta < 0.0 ? -t : t;
-    const double c = 1.0 / sqrt(t * t + 1.0), s = t * c;
-    a[pk(P, P)] -= t * apq;
-    a[pk(Q, Q)] += t * apq;
-    a[pk(P, Q)] = 0.0;
+    const double d = aqq - app, b = 2.0 * apq;
+    const double h = fabs(d) + sqrt(d * d + b * b);
+    t = apq == 0.0 ? 0.0 : (d < 0.0 ? -b : b) / h;
+    c = rsqrt(t * t + 1.0);
+}
+
+// The rotations in the (P, Q) and the (R, S) plane of the packed symmetric
+// matrix a, accumulated into the eigenvector columns.  The two planes are
+// disjoint, so their angles (a root, a division and a reciprocal root each, in
+// series) overlap; one after the other they were most of the surface's time.
+template <int P, int Q, int R, int S>
+__device__ inline void rotate2(double a[10], double v[4][4])
+{
+    double t1, c1, t2, c2;
+    const double apq = a[pk(P, Q)], ars = a[pk(R, S)];
+    rotation(a[pk(P, P)], a[pk(Q, Q)], apq, t1, c1);
+    rotation(a[pk(R, R)], a[pk(S, S)], ars, t2, c2);
+    const double s1 = t1 * c1, s2 = t2 * c2;
+    a[pk(P, P)] -= t1 * apq;
+    a[pk(Q, Q)] += t1 * apq;
+    a[pk(R, R)] -= t2 * ars;
+    a[pk(S, S)] += t2 * ars;
+    a[pk(P, Q)] = a[pk(R, S)] = 0.0;
+    // the 2 x 2 block between the planes: columns by (c1, s1), rows by (c2, s2)
+    const double pr = c1 * a[pk(P, R)] - s1 * a[pk(Q, R)], qr = s1 * a[pk(P, R)] + c1 * a[pk(Q, R)];
+    const double ps = c1 * a[pk(P, S)] - s1 * a[pk(Q, S)], qs = s1 * a[pk(P, S)] + c1 * a[pk(Q, S)];
+    a[pk(P, R)] = c2 * pr - s2 * ps;
+    a[pk(P, S)] = s2 * pr + c2 * ps;
+    a[pk(Q, R)] = c2 * qr - s2 * qs;
+    a[pk(Q, S)] = s2 * qr + c2 * qs;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-        if (r != P && r != Q) {
-            const double arp = a[pk(r, P)], arq = a[pk(r, Q)];
-            a[pk(r, P)] = c * arp - s * arq;
-            a[pk(r, Q)] = s * arp + c * arq;
-        }
-        const double vrp = v[r][P], vrq = v[r][Q];
-        v[r][P] = c * vrp - s * vrq;
-        v[r][Q] = s * vrp + c * vrq;
+        const double vp = v[r][P], vq = v[r][Q], vr = v[r][R], vs = v[r][S];
+        v[r][P] = c1 * vp - s1 * vq;
+        v[r][Q] = s1 * vp + c1 * vq;
+        v[r][R] = c2 * vr - s2 * vs;
+        v[r][S] = s2 * vr + c2 * vs;
     }
 }
 
@@ -95,12 +112,9 @@ __device__ inline double lowest_eigenpair(double a[10], double u[4])
         const double off = fabs(a[1]) + fabs(a[3]) + fabs(a[4]) + fabs(a[6]) + fabs(a[7]) + fabs(a[8]);
         const double diag = fabs(a[0]) + fabs(a[2]) + fabs(a[5]) + fabs(a[9]);
         if (off <= 0x1p-60 * diag) break;
-        rotate<0, 1>(a, v);
-        rotate<0, 2>(a, v);
-        rotate<0, 3>(a, v);
-        rotate<1, 2>(a, v);
-        rotate<1, 3>(a, v);
-        rotate<2, 3>(a, v);
+        rotate2<0, 1, 2, 3>(a, v);
+        rotate2<0, 2, 1, 3>(a, v);
+        rotate2<0, 3, 1, 2>(a, v);
     }
     double e = a[0];
 #pragma unroll
@@ -116,7 +130,11 @@ __device__ inline double lowest_eigenpair(double a[10], double u[4])
     return e;
 }
 
-// POT_brh2: r = (R(1), R(2), R(3)) = (Br-Ha, Ha-Hc, Br-Hc), dedr in the same order
+// POT_brh2: r = (R(1), R(2), R(3)) = (Br-Ha, Ha-Hc, Br-Hc), dedr in the same
+// order.  QUAD: called by a quad with the same r on every lane; the three
+// exponentials that belong to one distance are evaluated on one lane each
+// (lane 0 R(1), lane 1 R(2), lane 2 R(3)).
+template <bool QUAD>
 __device__ inline double pot(const double r[3], double dedr[3])
 {
     double r1 = r[0], r2 = r[2], r3 = r[1];
@@ -162,19 +180,42 @@ __device__ inline double pot(const double r[3], double dedr[3])
     t = 2.0 * t;
     const double dcsg21 = t * c2x / (r1 * r12), dcsg22 = t * c1x / (r12 * r2), dcsg23 = -t * r3 / r12;
 
+    // exp(-A (r - Re)), exp(-B (r - Re)^3) and the overlaps' exp(-xi r) of the three distances
+    const double rd[3] = {r1 - kRhx, r3 - kRhh, r2 - kRhx};
+    double exa[3], exb[3], exs[3];
+    if constexpr (QUAD) {
+        const int i = threadIdx.x & 3;
+        const double x = i == 0 ? rd[0] : i == 1 ? rd[1] : rd[2], rr = i == 0 ? r1 : i == 1 ? r3 : r2;
+        const bool hh = i == 1;
+        const double ea = exp(-(hh ? kAhh : kAhx) * x), eb = exp(-(hh ? kBhh : kBhx) * (x * x * x));
+        const double es = exp(-(hh ? kXih : kXib) * rr);
+        exa[0] = quad::bcast<0>(ea);
+        exa[1] = quad::bcast<1>(ea);
+        exa[2] = quad::bcast<2>(ea);
+        exb[0] = quad::bcast<0>(eb);
+        exb[1] = quad::bcast<1>(eb);
+        exb[2] = quad::bcast<2>(eb);
+        exs[0] = quad::bcast<0>(es);
+        exs[1] = quad::bcast<1>(es);
+        exs[2] = quad::bcast<2>(es);
+    } else {
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            exa[j] = exp(-(j == 1 ? kAhh : kAhx) * rd[j]);
+            exb[j] = exp(-(j == 1 ? kBhh : kBhx) * (rd[j] * rd[j] * rd[j]));
+            exs[j] = exp(-(j == 1 ? kXih * r3 : kXib * (j == 0 ? r1 : r2)));
+        }
+    }
     // H2 singlet and triplet
-    double rdif = r3 - kRhh;
-    double ex1 = exp(-kAhh * rdif);
-    const double rdif2 = rdif * rdif, ex2 = exp(-kBhh * rdif * rdif2);
-    const double h1 = kDhh * ex1 * ex2;
-    const double v1hh = h1 * (ex1 - 2.0), v3hh = kEtaHH * h1 * (ex1 + 2.0);
-    const double h2 = 2.0 * kAhh * h1, h3 = 3.0 * kBhh * rdif2;
-    const double dv1hh = h2 * (1.0 - ex1) - h3 * v1hh;
-    const double dv3hh = -h2 * kEtaHH * (1.0 + ex1) - h3 * v3hh;
+    const double h1 = kDhh * exa[1] * exb[1];
+    const double v1hh = h1 * (exa[1] - 2.0), v3hh = kEtaHH * h1 * (exa[1] + 2.0);
+    const double h2 = 2.0 * kAhh * h1, h3 = 3.0 * kBhh * (rd[1] * rd[1]);
+    const double dv1hh = h2 * (1.0 - exa[1]) - h3 * v1hh;
+    const double dv3hh = -h2 * kEtaHH * (1.0 + exa[1]) - h3 * v3hh;
 
     double w1[4], dw1[4], w2[4], dw2[4];
-    vhx(r1, w1, dw1);
-    vhx(r2, w2, dw2);
+    vhx(rd[0], exa[0], exb[0], w1, dw1);
+    vhx(rd[2], exa[2], exb[2], w2, dw2);
     const double s11 = w1[0] + 3.0 * w1[1], s12 = w2[0] + 3.0 * w2[1];
     const double s21 = 3.0 * w1[0] + w1[1], s22 = 3.0 * w2[0] + w2[1];
     const double s31 = w1[0] - w1[1], s32 = w2[0] - w2[1];
@@ -251,18 +292,17 @@ __device__ inline double pot(const double r[3], double dedr[3])
     const double tx = kXib * kRhx;
     const double inv_denom = 1.0 / (2.0 * kRhx * (1.0 + tx * (1.0 + kC3 * tx)) * exp(-tx));
     t = kXih * r3;
-    ex1 = exp(-t);
-    const double shh = (1.0 + t * (1.0 + kC3 * t)) * ex1;
-    const double dshh = -kXih * t * (1.0 + t) * kC3 * ex1;
+    const double shh = (1.0 + t * (1.0 + kC3 * t)) * exs[1];
+    const double dshh = -kXih * t * (1.0 + t) * kC3 * exs[1];
     t = kXib * r1;
-    ex1 = exp(-t) * inv_denom;
+    double ex1 = exs[0] * inv_denom;
     const double shx1 = r1 * (1.0 + t * (1.0 + kC3 * t)) * ex1;
     const double dshx1 = (1.0 + t * (1.0 - kC3 * t * t)) * ex1;
     t = kXib * r2;
-    ex1 = exp(-t) * inv_denom;
+    ex1 = exs[2] * inv_denom;
     const double shx2 = r2 * (1.0 + t * (1.0 + kC3 * t)) * ex1;
     const double dshx2 = (1.0 + t * (1.0 - kC3 * t * t)) * ex1;
-    rdif = r1 - r2;
+    const double rdif = r1 - r2;
     const double b1 = kGr * exp(-kAlfw * rdif * rdif);
     const double b2 = shh * (shx1 + shx2) + shx1 * shx2;
     const double b3 = 2.0 * kAlfw * rdif * csg2;
@@ -286,13 +326,38 @@ __device__ inline void egrad_bead(const double *x, double &v, double *g)
                          sqrt(ac[0] * ac[0] + ac[1] * ac[1] + ac[2] * ac[2]),
                          sqrt(bc[0] * bc[0] + bc[1] * bc[1] + bc[2] * bc[2])};
     double d[3];
-    v = pot(r, d);
+    v = pot<false>(r, d);
     const double f0 = d[0] / r[0], f1 = d[1] / r[1], f2 = d[2] / r[2];
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
         g[c] = f1 * ac[c] - f0 * ab[c];
         g[3 + c] = f0 * ab[c] - f2 * bc[c];
         g[6 + c] = f2 * bc[c] - f1 * ac[c];
+    }
+}
+
+// One bead on a quad of lanes: lane i owns atom i (Ha, Br, Hc) and one of the
+// distances Br-Ha, Ha-Hc, Br-Hc (lane 3 repeats lane 2); the matrix and its
+// eigenproblem are repeated on every lane.  x = this lane's atom (lane 3: any
+// values), V on every lane, g = dV/dx of this lane's atom.
+__device__ inline void egrad_quad(const double *x, double &v, double *g)
+{
+    const int i = threadIdx.x & 3;
+    double d[3], s = 0.0;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        d[c] = quad::dpp<quad::perm(1, 0, 2, 2)>(x[c]) - quad::dpp<quad::perm(0, 2, 1, 1)>(x[c]);
+        s += d[c] * d[c];
+    }
+    s = sqrt(s);
+    const double r[3] = {quad::bcast<0>(s), quad::bcast<1>(s), quad::bcast<2>(s)};
+    double dv[3];
+    v = pot<true>(r, dv);
+    const double f = (i == 0 ? dv[0] : i == 1 ? dv[1] : dv[2]) / s;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        const double F = f * d[c];
+        g[c] = quad::dpp<quad::perm(1, 0, 2, 2)>(F) - quad::dpp<quad::perm(0, 2, 1, 1)>(F);
     }
 }
 

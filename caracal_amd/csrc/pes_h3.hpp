@@ -11,6 +11,7 @@
 #include <hip/hip_runtime.h>
 #include <type_traits>
 
+#include "quad.hpp"
 #include "rt_math.hpp"
 
 namespace cam {
@@ -448,6 +449,269 @@ __device__ __forceinline__ void egrad_bead(const double x[9], double& v, double 
         g[3 + d] = f0 * ab[d] - f2 * bc[d];
         g[6 + d] = f2 * bc[d] - f1 * ac[d];
     }
+}
+
+// ---------------------------------------------------------------------------
+// The same surface on a quad of lanes.  Lane i owns atom i and the distance
+// R_(i+1) (lane 3 repeats lane 2); what belongs to one distance (the H2
+// curves, the angle opposite to it, every derivative by it) is evaluated on
+// its lane, the rest (the sums over the three and the two bending families)
+// on all of them.  All terms are cyclic in the three distances, so a lane
+// sees them as (own, next, next but one), moved by DPP.  Forces as accurate as
+// the one-lane form's (against 80-bit arithmetic, near the saddle and wide).
+//
+// Half of the one-lane work or less sits on each lane (the H2 curves and 48 of
+// 75 divisions go from three to one).  A step of a batch that leaves the SIMDs
+// with one wave each is this serial chain: 100 trajectories of 8 beads take
+// 14.1 us a step on one lane a bead, 5.6 on four.
+// ---------------------------------------------------------------------------
+namespace q4 {
+template <typename T>
+__device__ __forceinline__ T next(T v) { return quad::dpp<quad::perm(1, 2, 0, 0)>(v); }
+template <typename T>
+__device__ __forceinline__ T after(T v) { return quad::dpp<quad::perm(2, 0, 1, 1)>(v); }
+// What the three lanes share is summed in one order on all of them: rounded
+// differently per lane, the common parts of the three derivatives, O(1) near
+// the saddle, would no longer cancel (forces off by 5e-16 instead of 1e-16
+// hartree/bohr there).
+template <typename T>
+__device__ __forceinline__ T sum3(T v) { return quad::bcast<0>(v) + quad::bcast<1>(v) + quad::bcast<2>(v); }
+
+// singlet() and triplet() with 1/r at hand; the triplet's short-range patch
+// reuses the singlet of the same distance.
+__device__ __forceinline__ void curves(double r, double ri, double &e1, double &de1, double &e3, double &de3)
+{
+    const double a0 = CAM_SP(0.03537359271649620), a1 = CAM_SP(2.013977588700072), a2 = CAM_SP(-2.827452449964767),
+                 a3 = CAM_SP(2.713257715593500), a4 = CAM_SP(-2.792039234205731), a5 = CAM_SP(2.166542078766724),
+                 a6 = CAM_SP(-1.272679684173909), a7 = CAM_SP(0.5630423099212294), a8 = CAM_SP(-0.1879397372273814),
+                 a9 = CAM_SP(0.04719891893374140), a10 = CAM_SP(-0.008851622656489644),
+                 a11 = CAM_SP(0.001224998776243630), a12 = -1.227820520228028e-04, a13 = 8.638783190083473e-06,
+                 a14 = -4.036967926499151e-07, a15 = 1.123286608335365e-08, a16 = -1.406619156782167e-10;
+    const double r0 = 3.5284882, dd = 0.160979391, c6 = 6.499027, c8 = 124.3991, c10 = 3285.828;
+    const double a[16] = { a1, a2, a3, a4, a5, a6, a7, a8, a9, a10, a11, a12, a13, a14, a15, a16 };
+    // sum a_i r^(i-1) and its derivative as singlet() forms them
+    double poly = a[15], dpoly = 15.0 * a[15];
+#pragma unroll
+    for (int k = 14; k >= 0; --k) {
+        poly = fma(poly, r, a[k]);
+        if (k > 0) dpoly = fma(dpoly, r, k * a[k]);
+    }
+    const double a0r = a0 * ri;
+    const double alpha = a0r + poly, dalpha = dpoly - a0r * ri;
+    const double ex = ::exp(alpha), exm1 = ex - 1.0;
+    const double r2 = r * r, r4 = r2 * r2, r6 = r4 * r2;
+    const double r02 = r0 * r0, r04 = r02 * r02, r06 = r04 * r02;
+    const double i2 = 1.0 / (r2 + r02), i4 = 1.0 / (r4 + r04), i6 = 1.0 / (r6 + r06);
+    const double i22 = i2 * i2, i25 = i22 * i22 * i2;
+    e1 = dd * exm1 * exm1 - dd - c6 * i6 - c8 * i4 * i4 - c10 * i25;
+    de1 = 2.0 * dd * exm1 * ex * dalpha + 6.0 * c6 * r4 * r * i6 * i6 + 8.0 * c8 * r2 * r * i4 * i4 * i4
+          + 10.0 * c10 * r * i25 * i2;
+    const double rl = 0.95, rr = 1.15;
+    const double t1 = CAM_SP(-0.0298546962), t2 = CAM_SP(-23.9604445036), t3 = CAM_SP(-42.5185569474),
+                 t4 = CAM_SP(2.0382390988), t5 = CAM_SP(-11.5214861455), t6 = CAM_SP(1.5309487826),
+                 c1 = CAM_SP(-0.4106358351531854), c2 = CAM_SP(-0.0770355790707090), c3 = CAM_SP(0.4303193846943223);
+    const double exdr = ::exp(-t4 * r), ra6 = ::exp(-t6 * ::log(r));
+    e3 = t1 * (t2 + r + t3 * r2 + t5 * ra6) * exdr;
+    de3 = t1 * exdr * (1.0 - t2 * t4 + (2.0 * t3 - t4) * r - t3 * t4 * r2 - t5 * t6 * ra6 * ri - t4 * t5 * ra6);
+    if (!(r >= rr)) {
+        const double dr = r - rl;
+        const bool in = r <= rl;
+        e3 = in ? e1 + c2 * dr + c3 : e1 + c1 * dr * dr * dr + c2 * dr + c3;
+        de3 = in ? de1 + c2 : de1 + 3.0 * c1 * dr * dr + c2;
+    }
+}
+
+// bend() for the derivative by the lane's own distance; t, dt: this lane's
+// compactness switch and its derivative, sumt the sum of the three.
+__device__ __forceinline__ void bend(double r, double rb, double rc, double ri, bool compact, double dt,
+                                     double sumt, double &v, double &dv)
+{
+    const double r1 = quad::bcast<0>(r), r2 = quad::bcast<1>(r), r3 = quad::bcast<2>(r);
+    const double rs = r1 + r2 + r3, rsq = rs * rs;
+    const double t = r * r - rb * rb - rc * rc, tb = next(t), tc = after(t);
+    const double cs = t / (-2.0 * rb * rc);
+    const double c3 = 4.0 * cs * cs * cs - 3.0 * cs;
+    const double csum = sum3(cs), cos3 = sum3(c3);
+    const double b1fam[2] = { 1.0 - csum, 1.0 - (0.625 * cos3 + 0.375 * csum) };
+    const double q = 12.0 * cs * cs - 3.0, qb = next(q), qc = after(q);
+    const double dcs = -r / (rb * rc), rr = r * r;
+    const double dcb = (tb / rr + 2.0) / (2.0 * rc), dcc = (tc / rr + 2.0) / (2.0 * rb);
+    const double dcsum = dcs + dcb + dcc;
+    const double db1[2] = { -dcsum, -0.625 * (q * dcs + qb * dcb + qc * dcc) - 0.375 * dcsum };
+    const double b2 = sum3(ri), db2 = -ri * ri;
+    const double b3 = (r2 - r1) * (r2 - r1) + (r3 - r2) * (r3 - r2) + (r1 - r3) * (r1 - r3);
+    const double b3b = ::sqrt(b3 + 1.0e-12);
+    const double db3 = 4.0 * r - 2.0 * rb - 2.0 * rc, ib3b = 0.5 / b3b;
+    const double beta1 = 0.52, beta2 = 0.052, beta3 = 0.79;
+    const double exp1 = ::exp(-beta1 * rs), exp2 = ::exp(-beta2 * rsq), exp7 = ::exp(-beta3 * rs);
+    const double dexp1 = -beta1 * exp1, dexp2 = -2.0 * beta2 * rs * exp2, dexp7 = -beta3 * exp7;
+#pragma unroll
+    for (int fam = 0; fam < 2; ++fam) {
+        const double *c = kVbend[fam];
+        const double b1 = b1fam[fam];
+        const double b12 = b1 * b1, b13 = b12 * b1, b14 = b13 * b1, b15 = b14 * b1;
+        const double asum = c[0] + c[1] * rs + c[2] * rsq;
+        const double bsum = c[3] * b12 + c[4] * b13 + c[5] * b14 + c[6] * b15;
+        const double csm = c[7] * b1 * exp1 + c[8] * b12 * exp2;
+        const double ds1 = c[9] * exp1 + c[10] * exp2, ds2 = c[11] * exp1 + c[12] * exp2;
+        const double fsum = c[13] + c[14] * rs + c[15] * rsq;
+        v += b1 * asum * exp1 + bsum * exp2 + b2 * csm + (b1 * b3 * ds1 + b1 * b3b * ds2) + b1 * fsum * exp7;
+        const double dasum = c[1] + 2.0 * c[2] * rs;
+        const double dbsum = 2.0 * c[3] * b1 + 3.0 * c[4] * b12 + 4.0 * c[5] * b13 + 5.0 * c[6] * b14;
+        const double dds1 = c[9] * dexp1 + c[10] * dexp2, dds2 = c[11] * dexp1 + c[12] * dexp2;
+        const double dfsum = c[14] + 2.0 * c[15] * rs;
+        const double k0 = b1 * dasum * exp1 + b1 * asum * dexp1 + bsum * dexp2
+                          + b2 * (c[7] * b1 * dexp1 + c[8] * b12 * dexp2) + b1 * b3 * dds1 + b1 * b3b * dds2
+                          + b1 * dfsum * exp7 + b1 * fsum * dexp7;
+        const double kb1 = asum * exp1 + dbsum * exp2 + b2 * (c[7] * exp1 + 2.0 * c[8] * b1 * exp2) + b3 * ds1
+                           + b3b * ds2 + fsum * exp7;
+        dv += k0 + db1[fam] * kb1 + db2 * csm + b1 * db3 * ds1 + b1 * db3 * ib3b * ds2;
+    }
+    if (!compact) return;
+    const double rcu = rsq * rs, p = r1 * r2 * r3, ip = 1.0 / p, ip2 = ip * ip, ip3 = ip2 * ip, dp = rb * rc;
+    const double e7 = ::exp(-beta2 * rcu), de7 = -3.0 * beta2 * rsq * e7;
+    const double irs = 1.0 / rs, irs2 = irs * irs, irs3 = irs2 * irs;
+#pragma unroll
+    for (int fam = 0; fam < 2; ++fam) {
+        const double *c = kCbend[fam];
+        const double b1 = b1fam[fam];
+        const double b12 = b1 * b1, b13 = b12 * b1, b14 = b13 * b1, b15 = b14 * b1;
+        const double x1 = c[15] + c[28];            // C51 + C83
+        const double asum = c[0] + c[1] * rs + c[2] * rsq + c[3] * irs + c[4] * irs2;
+        const double bsum = c[5] * b12 + c[6] * b13 + c[7] * b14 + c[8] * b15;
+        const double csm = c[9] * b1 * exp1 + c[10] * b12 * exp2;
+        const double ds1 = c[11] * exp1 + c[12] * exp2, ds2 = c[13] * exp1 + c[14] * exp2;
+        const double fsum = x1 + c[16] * rs + c[17] * rsq;
+        const double gsum = c[18] + c[19] * irs + c[20] * irs2;
+        const double aasum = c[21] + c[22] * p + c[23] * p * p + c[24] * ip + c[25] * ip2;
+        const double ffsum = c[26] * p + c[27] * p * p + c[29] * ip2;
+        const double dasum = c[1] + 2.0 * c[2] * rs - c[3] * irs2 - 2.0 * c[4] * irs3;
+        const double dbsum = 2.0 * c[5] * b1 + 3.0 * c[6] * b12 + 4.0 * c[7] * b13 + 5.0 * c[8] * b14;
+        const double dds1 = c[11] * dexp1 + c[12] * dexp2, dds2 = c[13] * dexp1 + c[14] * dexp2;
+        const double dfsum = c[16] + 2.0 * c[17] * rs, dgsum = -c[19] * irs2 - 2.0 * c[20] * irs3;
+        const double daasum = c[22] + 2.0 * c[23] * p - c[24] * ip2 - 2.0 * c[25] * ip3;
+        const double dffsum = c[26] + 2.0 * c[27] * p - 2.0 * c[29] * ip3;
+        const double cbnds = b1 * asum * exp1 * ip + bsum * exp2 + b2 * csm + (b1 * b3 * ds1 + b1 * b3b * ds2)
+                             + b1 * fsum * e7 * ip + b1 * gsum * e7 + b1 * aasum * exp2 + b1 * ffsum * e7;
+        v += sumt * cbnds;
+        const double k0 = b1 * dasum * exp1 * ip + b1 * asum * dexp1 * ip + bsum * dexp2
+                          + b2 * (c[9] * b1 * dexp1 + c[10] * b12 * dexp2) + b1 * b3 * dds1 + b1 * b3b * dds2
+                          + b1 * dfsum * e7 * ip + b1 * fsum * de7 * ip + b1 * dgsum * e7 + b1 * gsum * de7
+                          + b1 * aasum * dexp2 + b1 * ffsum * de7;
+        const double kb1 = asum * exp1 * ip + dbsum * exp2 + b2 * (c[9] * exp1 + 2.0 * c[10] * b1 * exp2) + b3 * ds1
+                           + b3b * ds2 + fsum * e7 * ip + gsum * e7 + aasum * exp2 + ffsum * e7;
+        const double kdp = -b1 * asum * exp1 * ip2 - b1 * fsum * e7 * ip2 + b1 * daasum * exp2 + b1 * dffsum * e7;
+        const double dsum = k0 + db1[fam] * kb1 + db2 * csm + b1 * db3 * ds1 + b1 * db3 * ib3b * ds2 + dp * kdp;
+        dv += dt * cbnds + sumt * dsum;
+    }
+}
+
+// The asymmetric and compact corrections in T: own, next and next but one
+// distance; v and the derivative by the own one are added to, t, dt and sumt
+// returned for bend.
+template <typename T>
+__device__ __forceinline__ void corrections(T r, T rb, T rc, T &v, T &dv, bool &compact, T &dt, T &sumt)
+{
+    const T r1 = quad::bcast<0>(r), r2 = quad::bcast<1>(r), r3 = quad::bcast<2>(r);
+    const T rs = r1 + r2 + r3, rsq = rs * rs;
+    T a = (r1 - r2) * (r2 - r3) * (r3 - r1), da = (-T(2) * r + rb + rc) * (rb - rc);
+    da = a < T(0) ? -da : da;
+    a = a < T(0) ? -a : a;
+    {
+        const T aa1 = T(CAM_SP(0.3788951192E-02)), aa2 = T(CAM_SP(0.1478100901E-02)),
+                aa3 = T(CAM_SP(-.1848513849E-03)), aa4 = T(CAM_SP(0.9230803609E-05)),
+                aa5 = T(CAM_SP(-.1293180255E-06)), aa6 = T(CAM_SP(0.5237179303E+00)),
+                aa7 = T(CAM_SP(-.1112326215E-02));
+        const T a2 = a * a, a3 = a2 * a, a4 = a3 * a, a5 = a4 * a;
+        const T exp1 = rt::exp(-aa1 * rsq * rs), exp6 = rt::exp(-aa6 * rs);
+        const T s = aa2 * a2 + aa3 * a3 + aa4 * a4 + aa5 * a5;
+        const T ir = T(1) / rs;
+        v += s * exp1 + aa7 * a2 * exp6 * ir;
+        const T common = -T(3) * aa1 * rsq * s * exp1 - aa7 * a2 * exp6 * ir * ir - aa6 * aa7 * a2 * exp6 * ir;
+        const T dsda = (T(2) * aa2 * a + T(3) * aa3 * a2 + T(4) * aa4 * a3 + T(5) * aa5 * a4);
+        dv += common + dsda * da * exp1 + T(2) * aa7 * a * da * exp6 * ir;
+    }
+    const T rrc = T(1.15), rpc = T(1.25);
+    compact = r < rrc || rb < rrc || rc < rrc;        // the same on the whole quad
+    dt = sumt = T(0);
+    if (!compact) return;
+    T t = T(0), g = T(0), dg = T(0);
+    const T v1 = T(CAM_SP(-.2071708868E+00)), v2 = T(CAM_SP(-.5672350377E+00)), v3 = T(CAM_SP(0.9058780367E-02));
+    if (r < rrc) {
+        const T top = rrc - r, bot = rpc - r, top2 = top * top, top3 = top2 * top;
+        t = top3 / bot;
+        dt = -T(3) * top2 / bot + top3 / (bot * bot);
+        const T sv = v1 + v1 * v2 * r;
+        g = t * sv;
+        dg = t / bot * sv - T(3) * (top2 / bot) * sv + t * v1 * v2;
+    }
+    sumt = sum3(t);
+    const T sumg = sum3(g);
+    const T exp3 = rt::exp(-v3 * rsq * rs);
+    v += sumg * exp3;
+    dv += dg * exp3 + sumg * (-T(3) * v3 * rsq * exp3);
+    const T u1 = T(CAM_SP(0.2210243144E+00)), u2 = T(CAM_SP(0.4367417579E+00)), u3 = T(CAM_SP(0.6994985432E-02)),
+            u4 = T(CAM_SP(0.1491096501E+01)), u5 = T(CAM_SP(0.1602896673E+01)), u6 = T(CAM_SP(-.2821747323E+01)),
+            u7 = T(CAM_SP(0.4948310833E+00)), u8 = T(CAM_SP(-.3540394679E-01)), u9 = T(CAM_SP(-.3305809954E+01)),
+            u10 = T(CAM_SP(0.3644382172E+01)), u11 = T(CAM_SP(-.9997570970E+00)), u12 = T(CAM_SP(0.7989919534E-01)),
+            u13 = T(CAM_SP(-.1075807322E-02));
+    const T pr = r1 * r2 * r3, ipr = T(1) / pr, ipr2 = ipr * ipr, ipr3 = ipr2 * ipr, a2 = a * a;
+    const T s2 = u9 * ipr2 + u10 * ipr + u11 + u12 * pr + u13 * pr * pr;
+    const T series = T(1) + u4 * ipr2 + u5 * ipr + u6 + u7 * pr + u8 * pr * pr + a * s2;
+    const T term1 = u1 * rt::exp(-u2 * rt::log(pr));   // u1 / pr^u2
+    const T eterm = rt::exp(-u3 * rsq * rs);
+    const T base = term1 * series * eterm;
+    v += sumt * a2 * base;
+    const T dpr_all = -T(2) * u4 * ipr3 - u5 * ipr2 + u7 + T(2) * u8 * pr;
+    const T dpr_a = -T(2) * u9 * ipr3 - u10 * ipr2 + u12 + T(2) * u13 * pr;
+    const T dpr = rb * rc;
+    const T dterm1 = -u2 * term1 * ipr * dpr;
+    const T determ = eterm * (-T(3) * u3 * rsq);
+    const T dseries = dpr * dpr_all + da * s2 + a * dpr * dpr_a;
+    dv += dt * a2 * base + T(2) * a * da * sumt * base + sumt * a2 * eterm * (dterm1 * series + dseries * term1)
+          + determ * sumt * a2 * term1 * series;
+}
+}  // namespace q4
+
+// One bead on a quad: x = this lane's atom (lane 3: any values), returns V on
+// every lane and g = dV/dx of this lane's atom.
+template <typename T>
+__device__ __forceinline__ void egrad_quad(const double x[3], double &v, double g[3])
+{
+    double d[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+        d[c] = quad::dpp<quad::perm(1, 0, 2, 2)>(x[c]) - quad::dpp<quad::perm(0, 2, 1, 1)>(x[c]);
+    const double r = ::sqrt(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]), ri = 1.0 / r;
+    const double rb = q4::next(r), rc = q4::after(r);
+    double e1, de1, e3, de3;
+    q4::curves(r, ri, e1, de1, e3, de3);
+    const double jj = 0.5 * (e1 - e3), jb = q4::next(jj), jc = q4::after(jj);
+    const double j1 = quad::bcast<0>(jj), j2 = quad::bcast<1>(jj), j3 = quad::bcast<2>(jj);
+    const double d21 = j2 - j1, d32 = j3 - j2, d31 = j3 - j1;
+    const double root = ::sqrt(0.5 * (d21 * d21 + d32 * d32 + d31 * d31) + 1.0e-12);
+    v = q4::sum3(0.5 * (e1 + e3)) - root;
+    double dv = 0.5 * (de1 + de3) - (2.0 * jj - jb - jc) * (de1 - de3) * (0.25 / root);
+    bool compact;
+    double dt, sumt;
+    if constexpr (std::is_same<T, double>::value) {
+        q4::corrections(r, rb, rc, v, dv, compact, dt, sumt);
+    } else {
+        // binary32 corrections are summed on their own and added once
+        T v32 = T(0), dv32 = T(0), dt32, sumt32;
+        q4::corrections(T(r), T(rb), T(rc), v32, dv32, compact, dt32, sumt32);
+        v += double(v32);
+        dv += double(dv32);
+        dt = double(dt32);
+        sumt = double(sumt32);
+    }
+    q4::bend(r, rb, rc, ri, compact, dt, sumt, v, dv);
+    // the three distances' forces cancel on each atom: divided by r and fused
+    const double f = dv / r;
+    const double fp = quad::dpp<quad::perm(1, 0, 2, 2)>(f), fm = quad::dpp<quad::perm(0, 2, 1, 1)>(f);
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+        g[c] = fma(fp, quad::dpp<quad::perm(1, 0, 2, 2)>(d[c]), -(fm * quad::dpp<quad::perm(0, 2, 1, 1)>(d[c])));
 }
 
 #undef CAM_SP

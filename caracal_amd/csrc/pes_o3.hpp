@@ -22,6 +22,7 @@
 // its dispersion routine, so its gradient sees R moved by up to an ulp; here
 // every term is evaluated at R as computed (a difference at rounding level).
 #pragma once
+#include "quad.hpp"
 
 namespace cam {
 namespace o3 {
@@ -192,6 +193,39 @@ __device__ inline void egrad_bead(const double *x, double &v, double *g)
             g[3 * pa[i] + c] += f * d[i][c];
             g[3 * pb[i] + c] -= f * d[i][c];
         }
+    }
+}
+
+// One bead on a quad of lanes: lane i owns atom i and pair i of (0,1), (0,2),
+// (1,2) (lane 3 repeats lane 2): its curve, its dispersion and the pass of the
+// recursion with its MEG variable first.  x = this lane's atom (lane 3: any
+// values), V on every lane, g = dV/dx of this lane's atom.  The three passes
+// are the bulk of the one-lane evaluation; at one wave per SIMD they are its
+// time: 4096 x 32 beads 19.8 us a step on one lane a bead, 12.5 on four.
+__device__ inline void egrad_quad(const double *x, double &v, double *g)
+{
+    const int i = threadIdx.x & 3;
+    double d[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+        d[c] = (quad::dpp<quad::perm(0, 0, 1, 1)>(x[c]) - quad::dpp<quad::perm(1, 2, 2, 2)>(x[c])) * kCconv;
+    const double r = sqrt(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]);
+    const double u = r - kMegRb;
+    const double m = exp(-(r - kMegRa) / kMegA - u * u / kMegAB), dm = (-2.0 * u / kMegAB - 1.0 / kMegA) * m;
+    double dv2, dd;
+    const double e2 = v2(r, dv2) + disp(r, dd);
+    const double m0 = quad::bcast<0>(m), m1 = quad::bcast<1>(m), m2 = quad::bcast<2>(m);
+    double vp, dp;
+    poly(m, i >= 2 ? m1 : m2, i == 0 ? m1 : m0, vp, dp);
+    // lane 2's pass has the reference's monomial order
+    const double e = kTwoDe + quad::bcast<0>(e2) + quad::bcast<1>(e2) + quad::bcast<2>(e2) + quad::bcast<2>(vp);
+    v = e * kEconv + kEref;
+    const double f = (dv2 + dd + dp * dm) * kGconv / r;
+    const double s1 = i == 0 ? 1.0 : -1.0, s2 = i >= 2 ? -1.0 : 1.0;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        const double F = f * d[c];
+        g[c] = s1 * quad::dpp<quad::perm(0, 0, 1, 1)>(F) + s2 * quad::dpp<quad::perm(1, 2, 2, 2)>(F);
     }
 }
 

@@ -63,6 +63,31 @@ struct SurfO3 {
     __device__ static void egrad(const double *own, double &v, double *g) { o3::egrad_bead(own, v, g); }
 };
 
+// The same surfaces on a quad of lanes: lane i holds the three coordinates of
+// atom i (lane 3 none where there are three atoms).
+template <int NATOMS>
+struct QuadAtoms {
+    static constexpr int NA = NATOMS, NC = 3 * NATOMS, L = 4, SLOTS = 3;
+    __device__ static int coord(int slot, int r) { return 3 * (r < NA ? r : NA - 1) + slot; }
+    __device__ static bool valid(int, int r) { return r < NA; }
+};
+struct SurfH3Q : QuadAtoms<3> {
+    template <typename T>
+    __device__ static void egrad(const double *own, double &v, double *g) { h3::egrad_quad<T>(own, v, g); }
+};
+struct SurfOH3Q : QuadAtoms<4> {
+    template <typename T>
+    __device__ static void egrad(const double *own, double &v, double *g) { oh3::egrad_quad(own, v, g); }
+};
+struct SurfBrH2Q : QuadAtoms<3> {
+    template <typename T>
+    __device__ static void egrad(const double *own, double &v, double *g) { brh2::egrad_quad(own, v, g); }
+};
+struct SurfO3Q : QuadAtoms<3> {
+    template <typename T>
+    __device__ static void egrad(const double *own, double &v, double *g) { o3::egrad_quad(own, v, g); }
+};
+
 struct SurfCH4H {
     static constexpr int NA = 6, NC = 18, L = 4, SLOTS = 6;
     // slot 0..2: methane H number r; slot 3..5: C on lane 0, Hb on lane 1
@@ -182,21 +207,27 @@ typedef void (*force_fn)(const double *, double *, double *, int);
 // normal-mode step (ensemble ens_nm) and force kernel; false if the bead count
 // has none.  wpe: waves per SIMD asked of the compiler (2 only for the FP64
 // CH5 step); mfma: the MFMA normal-mode transform where the bead count has
-// one.  Built in engine_h3.hip, engine_ch4h.hip and engine_fp64.hip (OH3,
-// BrH2, O3: FP64 only).
+// one; the _quad forms: four lanes per bead instead of one.  Built in
+// engine_h3.hip, engine_h3_quad.hip, engine_ch4h.hip, engine_fp64.hip and
+// engine_fp64_quad.hip (OH3, BrH2, O3: FP64 only).
 bool pick_kernels_h3(int precision, int nb, int ens, int ens_nm, int wpe, bool mfma, step_fn &st, force_fn &fo,
                      step_fn &nm, force_fn &fs);
+bool pick_kernels_h3_quad(int precision, int nb, int ens, int ens_nm, int wpe, bool mfma, step_fn &st, force_fn &fo,
+                          step_fn &nm, force_fn &fs);
 bool pick_kernels_ch4h(int precision, int nb, int ens, int ens_nm, int wpe, bool mfma, step_fn &st, force_fn &fo,
                        step_fn &nm, force_fn &fs);
 bool pick_kernels_fp64(int surface, int nb, int ens, int ens_nm, int wpe, bool mfma, step_fn &st, force_fn &fo,
                        step_fn &nm, force_fn &fs);
+bool pick_kernels_fp64_quad(int surface, int nb, int ens, int ens_nm, int wpe, bool mfma, step_fn &st, force_fn &fo,
+                            step_fn &nm, force_fn &fs);
 
 // The folded step kernel (fold.hip) of a configuration, or nullptr if it has
 // none; *tpb receives its trajectories per block.  nbuf: LDS column buffers
 // of the one-lane-per-bead surfaces' kernels (1: more blocks per CU; 2: one
 // block per CU, for engines that share the chip with other engines); the CH5
 // kernels take 2 whatever is asked.
-step_fn fold_step_kernel_for(int surface, int precision, int nbeads, int ensemble, int wpe, int nbuf, int *tpb);
+step_fn fold_step_kernel_for(int surface, int precision, int nbeads, int ensemble, int wpe, int nbuf, bool quad,
+                             int *tpb);
 
 // Folded reference transform M[r][c] = w_c cos(2 pi r c / nbeads) / sqrt(nbeads),
 // r, c < nbeads/2, w_0 = 1 and w_c = 2 otherwise, row-major.

@@ -1225,7 +1225,7 @@ step_fn pick_step_w(int ens, bool mfma)
 template <class S, int NB, typename T>
 step_fn pick_step(int ens, int wpe, bool mfma)
 {
-    if constexpr (S::L == 4 && std::is_same<T, double>::value)
+    if constexpr (std::is_same<S, SurfCH4H>::value && std::is_same<T, double>::value)
         if (wpe == 2 && ens != CAM_ENS_UMBRELLA && ens != CAM_ENS_NHC && ens != CAM_ENS_PARENT)
             return pick_step_w<S, NB, T, 2>(ens, mfma);
     return pick_step_w<S, NB, T, 1>(ens, mfma);
@@ -1236,7 +1236,7 @@ step_fn pick_step(int ens, int wpe, bool mfma)
 template <class S, int NB, typename T>
 force_fn pick_force_split()
 {
-    if constexpr (S::L == 4 && std::is_same<T, double>::value) return force_kernel<S, NB, T, 2>;
+    if constexpr (std::is_same<S, SurfCH4H>::value && std::is_same<T, double>::value) return force_kernel<S, NB, T, 2>;
     else return force_kernel<S, NB, T, 1>;
 }
 
