@@ -3,18 +3,19 @@
 // one structure at once: the box engine's force field for QMDFF boxes.
 //
 // Kernels of one evaluation (positions and gradients [bead][atom][3]):
-//   qm_inter_kernel   pairs of atoms of different molecules (dispersion,
-//                     repulsion, Coulomb; src/ff_nonb.f90:198-332, :453-509):
-//                     one lane per atom i, j atoms tiled through LDS, the j
-//                     range split over blocks; each lane sums its own i, so
-//                     every pair is evaluated from both sides and no atomics
-//                     are needed (partials [split][bead][atom][3]);
-//   qm_hbacc_kernel,  intermolecular hydrogen bonds (src/ff_hb.f90:198-276):
-//   qm_hbdon_kernel   every donor bond A-H against every acceptor atom j of
-//                     another molecule, once from the acceptor's side (its
-//                     gradient and the energy) and once from the donor's (the
-//                     A and H gradients);
-//   qm_gather_kernel  one lane per (bead, atom): the bonded terms, the nci
+//   qm_terms_kernel   everything that does not depend on other terms, a role
+//                     per block:
+//     pairs of atoms of different molecules (dispersion, repulsion, Coulomb;
+//       src/ff_nonb.f90:198-332, :453-509): one wave per atom i; the atoms j
+//       within the cutoff are queued and evaluated 64 at a time (qinter); every
+//       pair is evaluated from both sides, so no atomics are needed;
+//     intermolecular hydrogen bonds (src/ff_hb.f90:198-276): every donor bond
+//       A-H against every acceptor atom j of another molecule, once from the
+//       acceptor's side (its gradient and the energy) and once from the
+//       donor's (the A and H gradients), one wave each;
+//     the slots of bonds, bends, torsions, nci pairs and listed hydrogen bonds,
+//       one lane each;
+//   qm_gather_kernel  four lanes per (bead, atom): the bonded terms, the nci
 //                     pairs and the listed hydrogen bonds the atom takes part
 //                     in (a term is evaluated once per atom it moves and its
 //                     energy counted at its first atom), plus the partials
@@ -33,24 +34,25 @@
 #include <vector>
 
 #include "qmdff.hpp"
+#include "quad.hpp"
 
 namespace cam {
 
 constexpr int kQTile = 256;         // lanes per block; j atoms per LDS tile
-constexpr int kQSplit = 8;          // blocks over the j range of one i tile
+constexpr int kQWaves = kQTile / 64;    // waves per block: atoms i of an intermolecular block
 constexpr int kQMaxElem = 16;       // distinct elements of one force field
 constexpr int kQImageCap = 64;      // minimum-image iterations (the reference loops until inside)
 
 struct QDev {
     int n, ne, nbond, nangl, ntors, nnci, nhb, ndon, nacc;
     int periodic, zahn, inter;          // inter: more than one molecule
-    double box[3], box2[3];
+    double box[3], box2[3], ibox[3];
     double coul_cut, vdw_cut, cut_low, zahn_a, zahn_par;
     double eps1[6], eps2[6];
     const int *elem;                    // n: element slot 0..ne-1
     const int *mol;                     // n: molecule number
     const double *q;                    // n
-    const double *c6;                   // n * n
+    const double *c6;                   // n * n, [i][j]: the row of atom i holds the C6 its pairs use
     const double *r0, *r06, *sr42, *zab, *alpha;   // ne * ne: [slot_i][slot_j]
     const double *rad;                  // ne (bohr)
     const int *bond, *angl, *tors, *nci, *hb;      // 0-based atoms
@@ -432,7 +434,7 @@ __device__ void qnci(const QDev &f, const double *x, int m, int role, double &e,
     const double vdw = f.periodic ? f.vdw_cut : 10.0 / 0.52917721092;
     double ga[3] = { 0.0, 0.0, 0.0 }, gc[3];
     e = 0.0;
-    if (!(f.periodic && r > vdw)) qdisp_rep<double>(f, f.elem[i1], f.elem[i2], f.c6[(size_t)i2 * f.n + i1], d, r2, r,
+    if (!(f.periodic && r > vdw)) qdisp_rep<double>(f, f.elem[i1], f.elem[i2], f.c6[(size_t)i1 * f.n + i2], d, r2, r,
                                                     f.eps2[nk], e, ga);
     double ec;
     if (qcoulomb<double>(f, f.q[i1], f.q[i2], d, r2, r, f.eps1[nk], ec, gc)) {
@@ -559,115 +561,187 @@ __device__ double qhbinter(const QDev &f, const double *x, int dn, int ac, doubl
 
 // ---------------------------------------------------------------------------
 
-template <typename T>
-struct QAcc {
-    double s = 0.0;
-    __device__ void add(T v) { s = s + (double)v; }
-    __device__ double get() const { return s; }
-};
-template <>
-struct QAcc<float> {                    // compensated FP64 accumulation of binary32 terms
-    double s = 0.0, c = 0.0;
-    __device__ void add(float v)
-    {
-        const double y = (double)v - c;
-        const double t = s + y;
-        c = (t - s) - y;
-        s = t;
-    }
-    __device__ double get() const { return s; }
+// FP64 reciprocal and reciprocal square root from the hardware estimates with
+// two Newton steps each (positive normal arguments); binary32: 1 ulp.
+__device__ __forceinline__ double qrcp(double a)
+{
+    double y = __builtin_amdgcn_rcp(a);
+    y = y * fma(-a, y, 2.0);
+    return y * fma(-a, y, 2.0);
+}
+__device__ __forceinline__ float qrcp(float a) { return 1.0f / a; }
+__device__ __forceinline__ double qrsq(double a)
+{
+    double y = __builtin_amdgcn_rsq(a);
+    const double h = 0.5 * a;
+    y = y * fma(-h * y, y, 1.5);
+    return y * fma(-h * y, y, 1.5);
+}
+__device__ __forceinline__ float qrsq(float a) { return 1.0f / sqrtf(a); }
+
+// Intermolecular pairs of atom i (one wave) with every other atom of a bead,
+// terms as qdisp_rep and qcoulomb.
+//
+// A fifth of the atoms of the 51 bohr ethanol box lies within the 19 bohr
+// cutoff.  With a lane per atom i and the block's 64 or 256 atoms walking all j
+// together, nearly every j was inside for some lane, so every lane went
+// through the whole pair (262 us for 1125 atoms x 16 beads).  Here the lanes
+// stand for 64 atoms j: the distance check is 1/5 of a pair's work, those
+// inside are compacted into a queue, and the pair runs with all lanes full;
+// the sums over the lanes are butterflies, in a fixed order.  The per-element
+// tables are in LDS, C6 is read along the row of i, one reciprocal stands for
+// 1/t6 and 1/t8 and one reciprocal root for r and 1/r: with the slots and the
+// hydrogen bonds in the same launch 113 us, 329 us as four kernels before.
+struct QTile {
+    double x[3][kQTile];                // j atoms of the tile
+    int mol[kQTile], elem[kQTile];
+    int queue[kQWaves][128];            // per wave: accepted atoms, at most 63 + 64: j and its element << 20
+    double tab[5][kQMaxElem * kQMaxElem];
+    double e[kQWaves];
 };
 
 template <typename T>
-__global__ __launch_bounds__(kQTile) void qm_inter_kernel(QDev f, const double *__restrict__ xall, double *gpart,
-                                                          double *epart)
+__device__ void qinter(const QDev &f, const double *__restrict__ x, int blk, QTile &s, double *gpart, double *epart)
 {
-    __shared__ double sx[3 * kQTile];
-    __shared__ double sq[kQTile];
-    __shared__ int se[kQTile], sm[kQTile];
-    __shared__ double sred[kQTile / 64];
-    const int n = f.n, b = blockIdx.z, split = blockIdx.y, nsplit = gridDim.y;
-    const double *x = xall + (size_t)b * n * 3;
-    const int i = blockIdx.x * kQTile + threadIdx.x;
+    const int n = f.n, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int i = blk * kQWaves + wave;
     const bool act = i < n;
-    double xi[3] = { 0.0, 0.0, 0.0 }, qi = 0.0;
-    int ei = 0, mi = -1;
-    if (act) {
-        xi[0] = x[3 * i];
-        xi[1] = x[3 * i + 1];
-        xi[2] = x[3 * i + 2];
-        qi = f.q[i];
-        ei = f.elem[i];
-        mi = f.mol[i];
+    const int ii = act ? i : n - 1;
+    const double xi0 = x[3 * ii], xi1 = x[3 * ii + 1], xi2 = x[3 * ii + 2];
+    const int mi = f.mol[ii], ei = f.elem[ii] * f.ne;
+    const T qi = (T)f.q[ii];
+    const double *c6 = f.c6 + (size_t)ii * n;
+    for (int k = tid; k < f.ne * f.ne; k += kQTile) {
+        s.tab[0][k] = f.r0[k];
+        s.tab[1][k] = f.r06[k];
+        s.tab[2][k] = f.sr42[k];
+        s.tab[3][k] = f.zab[k];
+        s.tab[4][k] = f.alpha[k];
     }
-    const int chunk = (n + nsplit - 1) / nsplit;
-    const int j0 = split * chunk, j1 = min(n, j0 + chunk);
-    const T vdw = f.periodic ? (T)f.vdw_cut : (T)(10.0 / 0.52917721092);
-    QAcc<T> gx, gy, gz, ee;
-    for (int t0 = j0; t0 < j1; t0 += kQTile) {
-        __syncthreads();
-        const int jj = t0 + threadIdx.x;
-        if (jj < j1) {
-            sx[3 * threadIdx.x] = x[3 * jj];
-            sx[3 * threadIdx.x + 1] = x[3 * jj + 1];
-            sx[3 * threadIdx.x + 2] = x[3 * jj + 2];
-            sq[threadIdx.x] = f.q[jj];
-            se[threadIdx.x] = f.elem[jj];
-            sm[threadIdx.x] = f.mol[jj];
-        }
-        __syncthreads();
-        const int nt = min(kQTile, j1 - t0);
-        if (!act) continue;
-        for (int u = 0; u < nt; ++u) {
-            if (sm[u] == mi) continue;                      // same molecule (and i itself)
-            double dd[3] = { xi[0] - sx[3 * u], xi[1] - sx[3 * u + 1], xi[2] - sx[3 * u + 2] };
-            qimg(f, dd);
-            const T d[3] = { (T)dd[0], (T)dd[1], (T)dd[2] };
-            const T r2 = (d[0] * d[0] + d[1] * d[1]) + d[2] * d[2];
-            const T r = sqrt(r2);
-            T ga[3] = { (T)0, (T)0, (T)0 }, e = (T)0;
-            if (!(f.periodic && r > vdw))
-                qdisp_rep<T>(f, ei, se[u], f.c6[(size_t)(t0 + u) * n + i], d, r2, r, (T)1.0, e, ga);
-            T ec, gc[3];
-            if (qcoulomb<T>(f, qi, sq[u], d, r2, r, (T)1.0, ec, gc)) {
-                e = e + ec;
-                ga[0] = ga[0] + gc[0];
-                ga[1] = ga[1] + gc[1];
-                ga[2] = ga[2] + gc[2];
+    const T vdw = (T)f.vdw_cut, coul = (T)f.coul_cut;
+    // the queue holds every pair either cutoff takes; a NaN distance is kept
+    const double rmax = f.vdw_cut > f.coul_cut ? f.vdw_cut : f.coul_cut;
+    const double cut2 = f.periodic ? rmax * rmax * (1.0 + 1e-6) : INFINITY;
+    auto image = [&](double *d) {
+        if (!f.periodic) return;
+        d[0] = fma(-f.box[0], rint(d[0] * f.ibox[0]), d[0]);
+        d[1] = fma(-f.box[1], rint(d[1] * f.ibox[1]), d[1]);
+        d[2] = fma(-f.box[2], rint(d[2] * f.ibox[2]), d[2]);
+    };
+    double gx = 0.0, gy = 0.0, gz = 0.0, ee = 0.0;
+    auto pairs = [&](int m) {
+        const bool on = lane < m;
+        const int l = on ? lane : 0, code = s.queue[wave][l];
+        const int j = code & 0xFFFFF, pe = ei + (code >> 20);
+        double dd[3] = { xi0 - x[3 * j], xi1 - x[3 * j + 1], xi2 - x[3 * j + 2] };
+        image(dd);
+        const T d0 = (T)dd[0], d1 = (T)dd[1], d2 = (T)dd[2];
+        const T r2 = (d0 * d0 + d1 * d1) + d2 * d2;
+        const T oner = qrsq(r2), r = r2 * oner, ir2 = oner * oner;
+        T e = (T)0, dr = (T)0;                     // gradient of i = d * dr
+        if (!(f.periodic && r > vdw)) {
+            const T R0 = (T)s.tab[0][pe], r06 = (T)s.tab[1][pe];
+            const T r4 = r2 * r2, r6 = r4 * r2;
+            const T t6 = r6 + r06, t8 = r6 * r2 + r06 * R0 * R0;
+            // beyond 1e5 bohr (no cutoff without periodicity) the terms are below 1e-25 hartree
+            const T c = r2 < (T)1e10 ? (T)c6[j] : (T)0;
+            const T ip = qrcp(r2 < (T)1e10 ? (sizeof(T) == 8 ? t6 * t8 : t8) : (T)1);
+            const T i6 = sizeof(T) == 8 ? t8 * ip : (T)1 / t6, i8 = sizeof(T) == 8 ? t6 * ip : ip;
+            const T c6t6 = c * i6;
+            T t27 = (T)s.tab[2][pe] * (c * i8);
+            e = -(c6t6 + t27);
+            dr = c6t6 * (T)6.0 * r4 * i6 + (T)8.0 * t27 * r6 * i8;
+            if (r < (T)25) {
+                const T alpha = (T)s.tab[4][pe];
+                t27 = (T)s.tab[3][pe] * exp(-alpha * r) * oner;
+                e = e + t27;
+                dr = dr - t27 * (alpha * r + (T)1.0) * ir2;
             }
-            gx.add(ga[0]);
-            gy.add(ga[1]);
-            gz.add(ga[2]);
-            ee.add(e);
+        }
+        if (!(r > coul)) {
+            const T qq = qi * (T)f.q[j];
+            T ec;
+            if (f.zahn) {
+                ec = qq * ((erfc((T)f.zahn_a * r) * oner) - (T)f.zahn_par * (r - coul));
+            } else {
+                T sw = (T)1.0;
+                if (f.periodic && r > (T)f.cut_low) {
+                    const T xv = (r - (T)f.cut_low) / (coul - (T)f.cut_low);
+                    sw = (T)exp(1.0) * exp((T)1.0 / (xv - (T)1.0));
+                }
+                ec = qq * oner * sw;
+            }
+            e = e + ec;
+            dr = dr - ec * ir2;
+        }
+        gx += on ? (double)(d0 * dr) : 0.0;
+        gy += on ? (double)(d1 * dr) : 0.0;
+        gz += on ? (double)(d2 * dr) : 0.0;
+        ee += on ? (double)e : 0.0;
+    };
+    int count = 0;
+    for (int t0 = 0; t0 < n; t0 += kQTile) {
+        __syncthreads();
+        const int jt = t0 + tid;
+        if (jt < n) {
+            for (int c = 0; c < 3; ++c) s.x[c][tid] = x[3 * jt + c];
+            s.mol[tid] = f.mol[jt];
+            s.elem[tid] = f.elem[jt];
+        }
+        __syncthreads();
+        const int nt = min(kQTile, n - t0);
+        if (!act) continue;                        // the whole wave
+        for (int u0 = 0; u0 < nt; u0 += 64) {
+            const int u = u0 + lane;
+            const int uu = u < nt ? u : 0;
+            bool in = u < nt && s.mol[uu] != mi;                  // not i's own molecule (nor i)
+            double d[3] = { xi0 - s.x[0][uu], xi1 - s.x[1][uu], xi2 - s.x[2][uu] };
+            image(d);
+            in = in && !((d[0] * d[0] + d[1] * d[1]) + d[2] * d[2] > cut2);
+            const unsigned long long m = __ballot(in);
+            if (in) s.queue[wave][count + __popcll(m & ((1ull << lane) - 1ull))] = (t0 + u) | s.elem[uu] << 20;
+            count += __popcll(m);
+            // the queue is this wave's alone and its LDS accesses are in order
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            const bool last = t0 + u0 + 64 >= n;
+            while (count >= 64 || (last && count > 0)) {
+                const int k = min(count, 64);
+                pairs(k);
+                count -= k;
+                const int rest = s.queue[wave][64 + lane];
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                if (lane < count) s.queue[wave][lane] = rest;
+            }
         }
     }
-    if (act) {
-        double *gp = gpart + (((size_t)split * gridDim.z + b) * n + i) * 3;
-        gp[0] = gx.get();
-        gp[1] = gy.get();
-        gp[2] = gz.get();
+    for (int o = 32; o > 0; o >>= 1) {
+        gx += __shfl_xor(gx, o);
+        gy += __shfl_xor(gy, o);
+        gz += __shfl_xor(gz, o);
+        ee += __shfl_xor(ee, o);
     }
-    // block energy (every pair counted from both sides: half of it)
-    double v = act ? 0.5 * ee.get() : 0.0;
-    for (int o = 32; o > 0; o >>= 1) v = v + __shfl_xor(v, o);
-    if ((threadIdx.x & 63) == 0) sred[threadIdx.x >> 6] = v;
+    if (lane == 0) {
+        if (act) {
+            gpart[3 * i] = gx;
+            gpart[3 * i + 1] = gy;
+            gpart[3 * i + 2] = gz;
+        }
+        s.e[wave] = act ? 0.5 * ee : 0.0;          // every pair counted from both sides
+    }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        double s = 0.0;
-        for (int w = 0; w < kQTile / 64; ++w) s = s + sred[w];
-        epart[((size_t)b * gridDim.x + blockIdx.x) * nsplit + split] = s;
-    }
+    if (tid == 0) *epart = ((s.e[0] + s.e[1]) + s.e[2]) + s.e[3];
 }
 
 // Every (term, atom) slot of the bonded terms, nci pairs and listed hydrogen
 // bonds: the term's gradient on that atom, and its energy at the slot of its
 // first atom (block sums in a fixed order).  Slots are contiguous per kind.
-__global__ __launch_bounds__(256) void qm_slot_kernel(QDev f, const double *__restrict__ xall, double *gslot,
-                                                      double *eslot)
+__device__ void qslot(const QDev &f, const double *__restrict__ x, int blk, double *sred, double *gslot, double *eslot)
 {
-    __shared__ double sred[4];
-    const int sl = blockIdx.x * blockDim.x + threadIdx.x, b = blockIdx.y;
-    const double *x = xall + (size_t)b * f.n * 3;
+    const int sl = blk * kQTile + threadIdx.x;
     double e = 0.0;
     if (sl < f.nslot) {
         double et = 0.0, gv[3] = { 0.0, 0.0, 0.0 };
@@ -682,7 +756,7 @@ __global__ __launch_bounds__(256) void qm_slot_kernel(QDev f, const double *__re
         case kTNci: qnci(f, x, idx, role, et, gv); break;
         default: qhblist(f, x, idx, role, et, gv); break;
         }
-        double *o = gslot + ((size_t)b * f.nslot + sl) * 3;
+        double *o = gslot + (size_t)sl * 3;
         o[0] = gv[0];
         o[1] = gv[1];
         o[2] = gv[2];
@@ -691,17 +765,15 @@ __global__ __launch_bounds__(256) void qm_slot_kernel(QDev f, const double *__re
     for (int o = 32; o > 0; o >>= 1) e = e + __shfl_xor(e, o);
     if ((threadIdx.x & 63) == 0) sred[threadIdx.x >> 6] = e;
     __syncthreads();
-    if (threadIdx.x == 0) eslot[(size_t)b * gridDim.x + blockIdx.x] = ((sred[0] + sred[1]) + sred[2]) + sred[3];
+    if (threadIdx.x == 0) *eslot = ((sred[0] + sred[1]) + sred[2]) + sred[3];
 }
 
 // acceptor side: one wave per acceptor atom, lanes over the donor bonds; the
 // acceptor's gradient and the energy (butterfly sums: a fixed order)
-__global__ __launch_bounds__(256) void qm_hbacc_kernel(QDev f, const double *__restrict__ xall, double *gacc,
-                                                       double *eacc)
+__device__ void qhbacc(const QDev &f, const double *__restrict__ x, int ac, double *gacc, double *eacc)
 {
-    const int lane = threadIdx.x & 63, ac = blockIdx.x * 4 + (threadIdx.x >> 6), b = blockIdx.y;
+    const int lane = threadIdx.x & 63;
     if (ac >= f.nacc) return;
-    const double *x = xall + (size_t)b * f.n * 3;
     double g[3] = { 0.0, 0.0, 0.0 }, e = 0.0, gj[3], ga[3], gh[3];
     for (int dn = lane; dn < f.ndon; dn += 64) {
         e = e + qhbinter(f, x, dn, ac, gj, ga, gh);
@@ -714,20 +786,16 @@ __global__ __launch_bounds__(256) void qm_hbacc_kernel(QDev f, const double *__r
         for (int c = 0; c < 3; ++c) g[c] = g[c] + __shfl_xor(g[c], o);
     }
     if (lane == 0) {
-        double *out = gacc + ((size_t)b * f.nacc + ac) * 3;
-        out[0] = g[0];
-        out[1] = g[1];
-        out[2] = g[2];
-        eacc[(size_t)b * f.nacc + ac] = e;
+        for (int c = 0; c < 3; ++c) gacc[3 * (size_t)ac + c] = g[c];
+        eacc[ac] = e;
     }
 }
 
 // donor side: one wave per donor bond, lanes over the acceptors; the A and H gradients
-__global__ __launch_bounds__(256) void qm_hbdon_kernel(QDev f, const double *__restrict__ xall, double *gdon)
+__device__ void qhbdon(const QDev &f, const double *__restrict__ x, int dn, double *gdon)
 {
-    const int lane = threadIdx.x & 63, dn = blockIdx.x * 4 + (threadIdx.x >> 6), b = blockIdx.y;
+    const int lane = threadIdx.x & 63;
     if (dn >= f.ndon) return;
-    const double *x = xall + (size_t)b * f.n * 3;
     double sa[3] = { 0.0, 0.0, 0.0 }, sh[3] = { 0.0, 0.0, 0.0 }, gj[3], ga[3], gh[3];
     for (int ac = lane; ac < f.nacc; ac += 64) {
         (void)qhbinter(f, x, dn, ac, gj, ga, gh);
@@ -742,26 +810,68 @@ __global__ __launch_bounds__(256) void qm_hbdon_kernel(QDev f, const double *__r
             sh[c] = sh[c] + __shfl_xor(sh[c], o);
         }
     if (lane == 0) {
-        double *out = gdon + ((size_t)b * f.ndon + dn) * 6;
         for (int c = 0; c < 3; ++c) {
-            out[c] = sa[c];
-            out[3 + c] = sh[c];
+            gdon[(size_t)dn * 6 + c] = sa[c];
+            gdon[(size_t)dn * 6 + 3 + c] = sh[c];
         }
     }
 }
 
-// one lane per (bead, atom): its term slots, hydrogen-bond parts and
-// intermolecular partials in a fixed order; the acceptors' energies
-__global__ __launch_bounds__(256) void qm_gather_kernel(QDev f, int nsplit, int nbeads, const double *gslot,
-                                                        const double *gpart, const double *gacc, const double *eacc,
-                                                        const double *gdon, double *gout, double *egather)
+// Blocks of one bead (blockIdx.y), in this order: ninter of the intermolecular
+// pairs, nacc and ndon of the hydrogen bonds, nslot of the slots.  One launch:
+// the hydrogen-bond and slot blocks, 17 to 25 us each as kernels of their own
+// that fill a part of the chip, run beside the pairs.
+struct QBlocks {
+    int ninter, nacc, ndon, nslot;
+};
+
+//
+// Built without machine-level loop-invariant code motion (see the Makefile):
+// with it the constants of exp and erfc were held in 128 registers across the
+// loops and others spilled inside them; without, 103 registers, and five waves
+// per SIMD cost 28 bytes of spills in the slots (FP64 call 151 us, 132 us at
+// four waves, 126 us at five, 134 us at six).
+template <typename T>
+__global__ __launch_bounds__(kQTile) __attribute__((amdgpu_waves_per_eu(5))) void qm_terms_kernel(
+    QDev f, QBlocks nb, const double *__restrict__ xall, double *gpart, double *epart, double *gacc, double *eacc,
+    double *gdon, double *gslot, double *eslot)
+{
+    __shared__ QTile s;
+    const int b = blockIdx.y, wave = threadIdx.x >> 6;
+    const double *x = xall + (size_t)b * f.n * 3;
+    int k = blockIdx.x;
+    if (k < nb.ninter) {
+        qinter<T>(f, x, k, s, gpart + (size_t)b * f.n * 3, epart + (size_t)b * nb.ninter + k);
+        return;
+    }
+    k -= nb.ninter;
+    if (k < nb.nacc) {
+        qhbacc(f, x, k * kQWaves + wave, gacc + (size_t)b * f.nacc * 3, eacc + (size_t)b * f.nacc);
+        return;
+    }
+    k -= nb.nacc;
+    if (k < nb.ndon) {
+        qhbdon(f, x, k * kQWaves + wave, gdon + (size_t)b * f.ndon * 6);
+        return;
+    }
+    k -= nb.ndon;
+    qslot(f, x, k, s.e, gslot + (size_t)b * f.nslot * 3, eslot + (size_t)b * nb.nslot + k);
+}
+
+// Four lanes per (bead, atom): its term slots and hydrogen-bond parts, every
+// fourth of the list to a lane (the loads of a list entry wait for its code, so
+// one lane's list was a chain of some twenty memory latencies: 16 us, now
+// 7.5), then the intermolecular sum; the acceptors' energies.
+__global__ __launch_bounds__(256) void qm_gather_kernel(QDev f, const double *gslot, const double *gpart,
+                                                        const double *gacc, const double *eacc, const double *gdon,
+                                                        double *gout, double *egather)
 {
     __shared__ double sred[4];
-    const int i = blockIdx.x * blockDim.x + threadIdx.x, b = blockIdx.y;
+    const int i = blockIdx.x * 64 + (threadIdx.x >> 2), sub = threadIdx.x & 3, b = blockIdx.y;
     const bool act = i < f.n;
     double g[3] = { 0.0, 0.0, 0.0 }, e = 0.0;
     if (act) {
-        for (int k = f.rptr[i]; k < f.rptr[i + 1]; ++k) {
+        for (int k = f.rptr[i] + sub; k < f.rptr[i + 1]; k += 4) {
             const int code = f.rcode[k];
             const int kind = code >> 28, payload = code & 0x0FFFFFFF;
             const double *src;
@@ -778,37 +888,31 @@ __global__ __launch_bounds__(256) void qm_gather_kernel(QDev f, int nsplit, int 
             g[1] = g[1] + src[1];
             g[2] = g[2] + src[2];
         }
-        if (f.inter)
-            for (int s = 0; s < nsplit; ++s) {
-                const double *gp = gpart + (((size_t)s * nbeads + b) * f.n + i) * 3;
-                g[0] = g[0] + gp[0];
-                g[1] = g[1] + gp[1];
-                g[2] = g[2] + gp[2];
-            }
-        if (gout) {
-            double *o = gout + ((size_t)b * f.n + i) * 3;
-            o[0] = g[0];
-            o[1] = g[1];
-            o[2] = g[2];
-        }
     }
-    double v = act ? e : 0.0;
-    for (int o = 32; o > 0; o >>= 1) v = v + __shfl_xor(v, o);
-    if ((threadIdx.x & 63) == 0) sred[threadIdx.x >> 6] = v;
+    for (int c = 0; c < 3; ++c) g[c] = quad::sum(g[c]);
+    if (act && gout && sub < 3) {
+        const size_t o = ((size_t)b * f.n + i) * 3 + sub;
+        const double own = sub == 0 ? g[0] : sub == 1 ? g[1] : g[2];
+        gout[o] = f.inter ? own + gpart[o] : own;
+    }
+    for (int o = 32; o > 0; o >>= 1) e = e + __shfl_xor(e, o);
+    if ((threadIdx.x & 63) == 0) sred[threadIdx.x >> 6] = e;
     __syncthreads();
     if (threadIdx.x == 0) egather[(size_t)b * gridDim.x + blockIdx.x] = ((sred[0] + sred[1]) + sred[2]) + sred[3];
 }
 
-__global__ void qm_reduce_kernel(const double *eslot, int nsl, const double *epart, int ninter, const double *egather,
-                                 int ngather, double *e)
+// One wave per bead: lanes over each list of block sums, then a butterfly (a
+// fixed order).
+__global__ __launch_bounds__(64) void qm_reduce_kernel(const double *eslot, int nsl, const double *epart, int ninter,
+                                                       const double *egather, int ngather, double *e)
 {
-    const int b = blockIdx.x;
-    if (threadIdx.x != 0) return;
+    const int b = blockIdx.x, lane = threadIdx.x;
     double s = 0.0;
-    for (int k = 0; k < nsl; ++k) s = s + eslot[(size_t)b * nsl + k];
-    for (int k = 0; k < ngather; ++k) s = s + egather[(size_t)b * ngather + k];
-    for (int k = 0; k < ninter; ++k) s = s + epart[(size_t)b * ninter + k];
-    e[b] = s;
+    for (int k = lane; k < nsl; k += 64) s = s + eslot[(size_t)b * nsl + k];
+    for (int k = lane; k < ngather; k += 64) s = s + egather[(size_t)b * ngather + k];
+    for (int k = lane; k < ninter; k += 64) s = s + epart[(size_t)b * ninter + k];
+    for (int o = 32; o > 0; o >>= 1) s = s + __shfl_xor(s, o);
+    if (lane == 0) e[b] = s;
 }
 
 // src/verlet.f90:540-640 (orthorhombic box): an atom whose coordinate left
@@ -930,6 +1034,7 @@ int qmdff_build(const cam_qmdff_desc *in, QmdffDev **out)
     for (int c = 0; c < 3; ++c) {
         d.box[c] = in->box[c];
         d.box2[c] = 0.5 * in->box[c];
+        d.ibox[c] = 1.0 / in->box[c];
     }
     d.coul_cut = in->coul_cut;
     d.vdw_cut = in->vdw_cut;
@@ -1060,7 +1165,9 @@ int qmdff_build(const cam_qmdff_desc *in, QmdffDev **out)
         rptr[i + 1] = rptr[i] + (int)roles[i].size();
         rcode.insert(rcode.end(), roles[i].begin(), roles[i].end());
     }
-    std::vector<double> c6(in->c6xy, in->c6xy + (size_t)n * n);
+    std::vector<double> c6((size_t)n * n);          // transposed: a wave reads along the row of its atom
+    for (int i = 0; i < n; ++i)
+        for (int j = 0; j < n; ++j) c6[(size_t)i * n + j] = in->c6xy[(size_t)j * n + i];
     std::vector<double> qv(in->q, in->q + n);
     std::vector<double> vbond(in->vbond, in->vbond + 3 * (size_t)in->nbond);
     std::vector<double> vangl(in->vangl, in->vangl + 2 * (size_t)in->nangl);
@@ -1093,10 +1200,10 @@ int qmdff_ensure(QmdffDev *q, int nbeads)
             *p = nullptr;
         }
     const QDev &d = q->d;
-    const int nbx = (d.n + kQTile - 1) / kQTile;
-    const int ngx = (d.n + 255) / 256;
-    CAM_HIP(hipMalloc(&q->gpart, (size_t)kQSplit * nbeads * d.n * 3 * sizeof(double)));
-    CAM_HIP(hipMalloc(&q->epart, ((size_t)nbeads * nbx * kQSplit + (size_t)nbeads * ngx) * sizeof(double)));
+    const int nbx = (d.n + kQWaves - 1) / kQWaves;
+    const int ngx = (d.n + 63) / 64;
+    CAM_HIP(hipMalloc(&q->gpart, (size_t)nbeads * d.n * 3 * sizeof(double)));
+    CAM_HIP(hipMalloc(&q->epart, (size_t)nbeads * (nbx + ngx) * sizeof(double)));
     CAM_HIP(hipMalloc(&q->gacc, ((size_t)std::max(1, d.nacc) * nbeads * 4) * sizeof(double)));
     CAM_HIP(hipMalloc(&q->eacc, ((size_t)std::max(1, d.nacc) * nbeads) * sizeof(double)));
     CAM_HIP(hipMalloc(&q->gdon, ((size_t)std::max(1, d.ndon) * nbeads * 6) * sizeof(double)));
@@ -1113,30 +1220,23 @@ int qmdff_launch(QmdffDev *q, const double *x, int nbeads, double *e, double *g,
     int rc = qmdff_ensure(q, nbeads);
     if (rc != CAM_OK) return rc;
     const QDev &d = q->d;
-    const int nbx = (d.n + kQTile - 1) / kQTile;
-    const int ngx = (d.n + 255) / 256;
-    double *egather = q->epart + (size_t)nbeads * nbx * kQSplit;
-    if (d.inter) {
-        hipLaunchKernelGGL(qm_inter_kernel<T>, dim3(nbx, kQSplit, nbeads), dim3(kQTile), 0, s, d, x, q->gpart,
-                           q->epart);
+    const int nbx = (d.n + kQWaves - 1) / kQWaves, nsx = (d.nslot + kQTile - 1) / kQTile;
+    const int ngx = (d.n + 63) / 64;
+    double *egather = q->epart + (size_t)nbeads * nbx;
+    const bool hb = d.nacc > 0 && d.ndon > 0;
+    const QBlocks nb{ d.inter ? nbx : 0, hb ? (d.nacc + kQWaves - 1) / kQWaves : 0,
+                      hb ? (d.ndon + kQWaves - 1) / kQWaves : 0, nsx };
+    const int nblk = nb.ninter + nb.nacc + nb.ndon + nb.nslot;
+    if (nblk > 0) {
+        hipLaunchKernelGGL(qm_terms_kernel<T>, dim3(nblk, nbeads), dim3(kQTile), 0, s, d, nb, x, q->gpart, q->epart,
+                           q->gacc, q->eacc, q->gdon, q->gslot, q->eslot);
         CAM_LAUNCH_CHECK();
     }
-    if (d.nacc > 0 && d.ndon > 0) {
-        hipLaunchKernelGGL(qm_hbacc_kernel, dim3((d.nacc + 3) / 4, nbeads), dim3(256), 0, s, d, x, q->gacc, q->eacc);
-        CAM_LAUNCH_CHECK();
-        hipLaunchKernelGGL(qm_hbdon_kernel, dim3((d.ndon + 3) / 4, nbeads), dim3(256), 0, s, d, x, q->gdon);
-        CAM_LAUNCH_CHECK();
-    }
-    const int nsx = (d.nslot + 255) / 256;
-    if (nsx > 0) {
-        hipLaunchKernelGGL(qm_slot_kernel, dim3(nsx, nbeads), dim3(256), 0, s, d, x, q->gslot, q->eslot);
-        CAM_LAUNCH_CHECK();
-    }
-    hipLaunchKernelGGL(qm_gather_kernel, dim3(ngx, nbeads), dim3(256), 0, s, d, kQSplit, nbeads, q->gslot, q->gpart,
+    hipLaunchKernelGGL(qm_gather_kernel, dim3(ngx, nbeads), dim3(256), 0, s, d, q->gslot, q->gpart,
                        q->gacc, q->eacc, q->gdon, g, egather);
     CAM_LAUNCH_CHECK();
     hipLaunchKernelGGL(qm_reduce_kernel, dim3(nbeads), dim3(64), 0, s, q->eslot, nsx, q->epart,
-                       d.inter ? nbx * kQSplit : 0, egather, ngx, e);
+                       nb.ninter, egather, ngx, e);
     CAM_LAUNCH_CHECK();
     return CAM_OK;
 }
