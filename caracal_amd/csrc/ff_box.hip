@@ -27,6 +27,7 @@
 #include "nhc.hpp"
 #include "philox.hpp"
 #include "qmdff.hpp"
+#include "transrot.hpp"
 
 namespace cam {
 namespace {
@@ -1573,9 +1574,21 @@ struct BoxNM {
     const double *tfwd, *tinv; // [nb][nb], element (j,k) = T[k][j]
     int natoms, nb;
     double dt, beta;
+    const double *scale;       // Nose-Hoover factor of the momenta (NULL: none)
+    int wrap;                  // the reference's periodic wrap after the step
+    double box[3];
 };
 
 // One block: 256/nb columns (atom, dim) x nb beads.
+//
+// The wrap (src/verlet.f90:540-640): a coordinate that left [0, L] in some
+// bead is moved in all its beads, bead by bead in order.  The block holds
+// every bead of its columns, so it only has to look whether one is outside;
+// then bead kb's position goes to all lanes of its column, which follow its
+// shifts and add them to their own in the same order.  As a kernel of its own
+// with a lane per column reading the beads one after the other it took 38 us
+// for 1125 atoms x 16 beads, longer than the step itself (5.6 us; 9.2 with
+// the wrap and the Nose-Hoover factor, once a kernel too).
 __global__ __launch_bounds__(256) void box_nm_kernel(BoxNM a)
 {
     extern __shared__ double smem[];
@@ -1589,7 +1602,9 @@ __global__ __launch_bounds__(256) void box_nm_kernel(BoxNM a)
     const size_t o = (size_t)k * ncol + col;
     double p = 0.0, q = 0.0;
     if (act) {
-        p = a.p[o] - 0.5 * a.dt * a.g[o];
+        p = a.p[o];
+        if (a.scale) p = *a.scale * p;
+        p = p - 0.5 * a.dt * a.g[o];
         q = a.q[o];
     }
     sp[lc * nb + k] = p;
@@ -1625,28 +1640,66 @@ __global__ __launch_bounds__(256) void box_nm_kernel(BoxNM a)
         xp = fma(t, sp[lc * nb + j], xp);
         xq = fma(t, sq[lc * nb + j], xq);
     }
+    if (a.wrap) {
+        const double L = a.box[col % 3];
+        if (__syncthreads_or(act && (xq < 0.0 || xq > L))) {
+            // two rows of one value per column in turn, so that one barrier per bead is enough
+            for (int kb = 0; kb < nb; ++kb) {
+                double *row = (kb & 1) ? sq : sp;
+                if (k == kb) row[lc] = xq;
+                __syncthreads();
+                double w = row[lc];
+                int tries = 0;
+                while (w < 0.0 && tries <= 100) {
+                    w = w + L;
+                    xq = xq + L;
+                    ++tries;
+                }
+                while (w > L && tries <= 100) {
+                    w = w - L;
+                    xq = xq - L;
+                    ++tries;
+                }
+            }
+        }
+    }
     if (act) {
         a.p[o] = xp;
         a.q[o] = xq;
     }
 }
 
-__global__ void box_kick_kernel(double *p, const double *g, const double *mass, int natoms, int nb, double dt,
-                                double beta, int andersen_step, uint64_t seed, const uint64_t *step_base, int step_off)
+// Kinetic energy sum p^2/(2m) of the lanes of a block (256), for the chain:
+// one partial per block, sums in a fixed order.
+__device__ void box_ke_part(double acc, double *part)
 {
-    const size_t n = (size_t)natoms * 3 * nb;
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    double v = p[i] - 0.5 * dt * g[i];
-    if (andersen_step > 0) {
-        const uint64_t istep = *step_base + (uint64_t)step_off + 1;
-        if (istep % (uint64_t)andersen_step == 0) {
-            const int k = (int)(i / ((size_t)natoms * 3));
-            const int c = (int)(i % ((size_t)natoms * 3));
-            v = andersen_normal(seed, 0u, istep, c, k) * sqrt(mass[c / 3] / (beta / nb));
+    __shared__ double red[4];
+    for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
+    __syncthreads();
+    if (threadIdx.x == 0) part[blockIdx.x] = ((red[0] + red[1]) + red[2]) + red[3];
+}
+
+// Second half kick and the Andersen draws; with a chain (part not NULL) also
+// the kinetic energy the chain starts from.
+__global__ __launch_bounds__(256) void box_kick_kernel(double *p, const double *g, const double *mass, int natoms,
+                                                       int nb, double dt, double beta, int andersen_step, uint64_t seed,
+                                                       const uint64_t *step_base, int step_off, double *part)
+{
+    const size_t ncol = (size_t)3 * natoms, n = ncol * nb;
+    double acc = 0.0;
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
+        double v = p[i] - 0.5 * dt * g[i];
+        if (andersen_step > 0) {
+            const uint64_t istep = *step_base + (uint64_t)step_off + 1;
+            if (istep % (uint64_t)andersen_step == 0)
+                v = andersen_normal(seed, 0u, istep, (int)(i % ncol), (int)(i / ncol)) *
+                    sqrt(mass[i % ncol / 3] / (beta / nb));
         }
+        p[i] = v;
+        if (part) acc += v * v / (2.0 * mass[i % ncol / 3]);
     }
-    p[i] = v;
+    if (part) box_ke_part(acc, part);
 }
 
 __global__ void box_advance_kernel(uint64_t *ctr, int n) { *ctr += (uint64_t)n; }
@@ -1688,25 +1741,22 @@ __global__ void box_energy_kernel(const double *q, const double *p, const double
 // centroid-momenta kinetic energy sum p^2/(2m)/nbeads^2 in per-block parts
 // (a fixed order, so runs repeat bit for bit), the chain in one thread, then
 // every momentum scaled.  st[0..3]: thermostat velocities, st[4]: the scale.
-constexpr int kBoxNhcBlocks = 256;
+//
+// On a few thousand atoms these kernels cost a launch each (4.6 us) whatever
+// they do, so the kinetic energy is summed where the momenta are written last
+// (the kick, transrot, the scaling) and the factor is applied where they are
+// read next (the normal-mode step, transrot): of the three kernels per chain
+// only the chain is left, and box_ke_kernel before the first step of a launch.
+constexpr int kBoxParts = 1024;         // partial sums at most: blocks of a summing kernel
 
 __global__ __launch_bounds__(256) void box_ke_kernel(const double *p, const double *mass, int natoms, int nb,
                                                      double *part)
 {
-    __shared__ double red[256];
-    const size_t n = (size_t)3 * natoms * nb;
+    const size_t ncol = (size_t)3 * natoms, n = ncol * nb;
     double acc = 0.0;
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
-        const double v = p[i];
-        acc += v * v / (2.0 * mass[(i % (3 * (size_t)natoms)) / 3]);
-    }
-    red[threadIdx.x] = acc;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) part[blockIdx.x] = red[0];
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256)
+        acc += p[i] * p[i] / (2.0 * mass[i % ncol / 3]);
+    box_ke_part(acc, part);
 }
 
 __global__ __launch_bounds__(64) void box_nhc_kernel(const double *part, int nparts, double *st, double beta,
@@ -1730,164 +1780,128 @@ __global__ __launch_bounds__(64) void box_nhc_kernel(const double *part, int npa
     st[4] = scale;
 }
 
-__global__ void box_scale_kernel(double *p, size_t n, const double *st)
+// The factor of the second chain where no transrot follows, and the kinetic
+// energy of the next step's first chain.
+__global__ __launch_bounds__(256) void box_scale_kernel(double *p, const double *mass, int natoms, int nb,
+                                                        const double *scale, double *part)
 {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = st[4] * p[i];
-}
-
-// transrot for one box (src/transrot.f90:36-237, with its total mass of
-// nbeads^2 * M): two passes of fixed-order block sums over every (bead,
-// atom) -- mass-weighted velocities and positions, then, about the centre
-// they give, the angular momentum and the inertia tensor -- one thread that
-// inverts the tensor, and the velocity update.  tr[0..2] vtot, [3..5] centre,
-// [6..8] angular velocity.
-constexpr int kTrBlocks = 64;
-
-__device__ void tr_block_sum(double *v, int nv, double *sh, double *out)
-{
-    // v: this thread's nv partial sums -> out[nv] for the block, fixed order
-    for (int c = 0; c < nv; ++c) sh[c * 256 + threadIdx.x] = v[c];
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w)
-            for (int c = 0; c < nv; ++c) sh[c * 256 + threadIdx.x] = sh[c * 256 + threadIdx.x] + sh[c * 256 + threadIdx.x + w];
-        __syncthreads();
+    const size_t ncol = (size_t)3 * natoms, n = ncol * nb;
+    double acc = 0.0;
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
+        const double v = *scale * p[i];
+        p[i] = v;
+        acc += v * v / (2.0 * mass[i % ncol / 3]);
     }
-    if (threadIdx.x == 0)
-        for (int c = 0; c < nv; ++c) out[c] = sh[c * 256];
+    box_ke_part(acc, part);
 }
 
-__global__ __launch_bounds__(256) void box_tr_pass1(const double *q, const double *p, const double *mass, int natoms,
-                                                    int nb, double *part)
+// transrot for one box (transrot.hpp; total mass of nbeads^2 * M): two passes
+// of fixed-order block sums over every (bead, atom), then the velocity update.
+// Each block of the second and third kernel sums the parts of the one before
+// and, in the third, solves for the angular velocity itself (a few hundred
+// flops), which costs less than a kernel of one block that does it between
+// them: pass1, pass2, solve and apply took 4.7 + 9.1 + 7.7 + 4.7 us for 1125
+// atoms x 16 beads, the three 5.0 + 4.7 + 5.3 us with the Nose-Hoover factor and kinetic
+// energy in them.
+constexpr int kTrBlocks = 64;           // one wave's lanes sum the parts
+constexpr int kTrApplyBlocks = 512;     // at most, for the solution each block repeats
+
+// v: this lane's NV partial sums -> out[NV] for the block, a fixed order
+template <int NV>
+__device__ __forceinline__ void tr_block_sum(double *v, double *sh, double *out)
 {
-    __shared__ double sh[6 * 256];
+#pragma unroll
+    for (int c = 0; c < NV; ++c)
+        for (int o = 32; o > 0; o >>= 1) v[c] += __shfl_xor(v[c], o);
+    if ((threadIdx.x & 63) == 0)
+#pragma unroll
+        for (int c = 0; c < NV; ++c) sh[(threadIdx.x >> 6) * NV + c] = v[c];
+    __syncthreads();
+    if (threadIdx.x < NV) {
+        const double *r = sh + threadIdx.x;
+        out[threadIdx.x] = ((r[0] + r[NV]) + r[2 * NV]) + r[3 * NV];
+    }
+}
+
+// the kTrBlocks parts of NV sums -> sh[NV] in every lane's view
+template <int NV>
+__device__ __forceinline__ void tr_parts(const double *part, double *sh)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for (int c = wave; c < NV; c += 4) {
+        double v = part[NV * lane + c];
+        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+        if (lane == 0) sh[c] = v;
+    }
+    __syncthreads();
+}
+
+__global__ __launch_bounds__(256) void box_tr_pass1(const double *q, double *p, const double *mass, int natoms, int nb,
+                                                    const double *scale, double *part)
+{
+    __shared__ double sh[4 * 6];
     double v[6] = { 0, 0, 0, 0, 0, 0 };
     const size_t n = (size_t)natoms * nb;
     for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (size_t)kTrBlocks * 256) {
-        const double w = mass[e % natoms];
-        for (int c = 0; c < 3; ++c) {
-            v[c] = v[c] + (p[3 * e + c] / w) * w;
-            v[3 + c] = v[3 + c] + q[3 * e + c] * w;
+        double *pe = p + 3 * e;
+        double w[3] = { pe[0], pe[1], pe[2] };
+        if (scale) {
+            for (int c = 0; c < 3; ++c) {
+                w[c] = *scale * w[c];
+                pe[c] = w[c];
+            }
         }
+        transrot_sums1(q + 3 * e, w, mass[e % natoms], v);
     }
-    tr_block_sum(v, 6, sh, part + 6 * blockIdx.x);
+    tr_block_sum<6>(v, sh, part + 6 * blockIdx.x);
 }
 
 __global__ __launch_bounds__(256) void box_tr_pass2(const double *q, const double *p, const double *mass, int natoms,
-                                                    int nb, const double *part1, double totmass, double *tr,
-                                                    double *part)
+                                                    int nb, const double *part1, double totmass, double *part)
 {
-    __shared__ double sh[9 * 256];
-    __shared__ double ctr[6];
-    if (threadIdx.x == 0) {
-        double s[6] = { 0, 0, 0, 0, 0, 0 };
-        for (int b = 0; b < kTrBlocks; ++b)
-            for (int c = 0; c < 6; ++c) s[c] = s[c] + part1[6 * b + c];
-        for (int c = 0; c < 6; ++c) ctr[c] = s[c] / totmass;
-        if (blockIdx.x == 0)
-            for (int c = 0; c < 6; ++c) tr[c] = ctr[c];
-    }
-    __syncthreads();
+    __shared__ double sh[4 * 9], s1[6];
+    tr_parts<6>(part1, s1);
+    const double xt[3] = { s1[3] / totmass, s1[4] / totmass, s1[5] / totmass };
     double v[9] = { 0, 0, 0, 0, 0, 0, 0, 0, 0 };
     const size_t n = (size_t)natoms * nb;
-    for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (size_t)kTrBlocks * 256) {
-        const double w = mass[e % natoms];
-        const double *x = q + 3 * e;
-        const double vx = p[3 * e] / w, vy = p[3 * e + 1] / w, vz = p[3 * e + 2] / w;
-        v[0] = v[0] + (x[1] * vz - x[2] * vy) * w;
-        v[1] = v[1] + (x[2] * vx - x[0] * vz) * w;
-        v[2] = v[2] + (x[0] * vy - x[1] * vx) * w;
-        const double xd = x[0] - ctr[3], yd = x[1] - ctr[4], zd = x[2] - ctr[5];
-        v[3] = v[3] + xd * xd * w;
-        v[4] = v[4] + xd * yd * w;
-        v[5] = v[5] + xd * zd * w;
-        v[6] = v[6] + yd * yd * w;
-        v[7] = v[7] + yd * zd * w;
-        v[8] = v[8] + zd * zd * w;
-    }
-    tr_block_sum(v, 9, sh, part + 9 * blockIdx.x);
+    for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (size_t)kTrBlocks * 256)
+        transrot_sums2(q + 3 * e, p + 3 * e, mass[e % natoms], xt, v);
+    tr_block_sum<9>(v, sh, part + 9 * blockIdx.x);
 }
 
-__global__ void box_tr_solve(const double *part, int natoms, double totmass, double *tr)
+__global__ __launch_bounds__(256) void box_tr_apply(const double *q, double *p, const double *mass, int natoms, int nb,
+                                                    const double *part1, const double *part2, double totmass,
+                                                    double *kepart)
 {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    double s[9] = { 0, 0, 0, 0, 0, 0, 0, 0, 0 };
-    for (int b = 0; b < kTrBlocks; ++b)
-        for (int c = 0; c < 9; ++c) s[c] = s[c] + part[9 * b + c];
-    const double vt[3] = { tr[0], tr[1], tr[2] }, xt = tr[3], yt = tr[4], zt = tr[5];
-    double mang[3];
-    mang[0] = s[0] - (yt * vt[2] - zt * vt[1]) * totmass;
-    mang[1] = s[1] - (zt * vt[0] - xt * vt[2]) * totmass;
-    mang[2] = s[2] - (xt * vt[1] - yt * vt[0]) * totmass;
-    const double xx = s[3], xy = s[4], xz = s[5], yy = s[6], yz = s[7], zz = s[8];
-    double ten[3][3];
-    ten[0][0] = yy + zz; ten[0][1] = -xy;    ten[0][2] = -xz;
-    ten[1][0] = -xy;     ten[1][1] = xx + zz; ten[1][2] = -yz;
-    ten[2][0] = -xz;     ten[2][1] = -yz;    ten[2][2] = xx + yy;
-    if (natoms <= 2) {
-        ten[0][0] += 0.000001;
-        ten[1][1] += 0.000001;
-        ten[2][2] += 0.000001;
+    __shared__ double s1[6], s2[9];
+    tr_parts<6>(part1, s1);
+    tr_parts<9>(part2, s2);
+    double vtot[3], xt[3], omega[3], sums[9];
+    for (int c = 0; c < 3; ++c) {
+        vtot[c] = s1[c] / totmass;
+        xt[c] = s1[3 + c] / totmass;
     }
-    // Gauss-Jordan inversion with full pivoting (src/invert.f90)
-    int ipiv[3] = { 0, 0, 0 }, indxr[3], indxc[3];
-    for (int i = 0; i < 3; ++i) {
-        double big = 0.0;
-        int irow = 0, icol = 0;
-        for (int j = 0; j < 3; ++j)
-            if (ipiv[j] != 1)
-                for (int kk = 0; kk < 3; ++kk)
-                    if (ipiv[kk] == 0 && fabs(ten[j][kk]) >= big) {
-                        big = fabs(ten[j][kk]);
-                        irow = j;
-                        icol = kk;
-                    }
-        ipiv[icol] += 1;
-        if (irow != icol)
-            for (int j = 0; j < 3; ++j) {
-                const double tmp = ten[irow][j];
-                ten[irow][j] = ten[icol][j];
-                ten[icol][j] = tmp;
-            }
-        indxr[i] = irow;
-        indxc[i] = icol;
-        const double piv = ten[icol][icol];
-        ten[icol][icol] = 1.0;
-        for (int j = 0; j < 3; ++j) ten[icol][j] = ten[icol][j] / piv;
-        for (int j = 0; j < 3; ++j)
-            if (j != icol) {
-                const double tmp = ten[j][icol];
-                ten[j][icol] = 0.0;
-                for (int kk = 0; kk < 3; ++kk) ten[j][kk] = ten[j][kk] - ten[icol][kk] * tmp;
-            }
+    for (int c = 0; c < 9; ++c) sums[c] = s2[c];
+    if (natoms <= 2) {                    // 1e-6 on the diagonal (src/transrot.f90:176-180)
+        const double d = 0.5 * 0.000001;  // each diagonal element is a sum of two of these
+        sums[3] += d;
+        sums[6] += d;
+        sums[8] += d;
     }
-    for (int i = 2; i >= 0; --i)
-        if (indxr[i] != indxc[i])
-            for (int kk = 0; kk < 3; ++kk) {
-                const double tmp = ten[kk][indxr[i]];
-                ten[kk][indxr[i]] = ten[kk][indxc[i]];
-                ten[kk][indxc[i]] = tmp;
-            }
-    for (int i = 0; i < 3; ++i) {
-        double v = 0.0;
-        for (int j = 0; j < 3; ++j) v = v + ten[i][j] * mang[j];
-        tr[6 + i] = v;
+    transrot_omega(vtot, xt, sums, totmass, omega);
+    const size_t n = (size_t)natoms * nb;
+    double acc = 0.0;
+    for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (size_t)gridDim.x * 256) {
+        double *pe = p + 3 * e;
+        double w[3] = { pe[0], pe[1], pe[2] };
+        const double m = mass[e % natoms];
+        transrot_apply(q + 3 * e, w, m, vtot, xt, omega);
+        for (int c = 0; c < 3; ++c) {
+            pe[c] = w[c];
+            acc += w[c] * w[c] / (2.0 * m);
+        }
     }
-}
-
-__global__ void box_tr_apply(const double *q, double *p, const double *mass, int natoms, int nb, const double *tr)
-{
-    const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= (size_t)natoms * nb) return;
-    const double w = mass[e % natoms];
-    double v[3];
-    for (int j = 0; j < 3; ++j) v[j] = p[3 * e + j] / w - tr[j];
-    const double xd = q[3 * e] - tr[3], yd = q[3 * e + 1] - tr[4], zd = q[3 * e + 2] - tr[5];
-    v[0] = v[0] - tr[7] * zd + tr[8] * yd;
-    v[1] = v[1] - tr[8] * xd + tr[6] * zd;
-    v[2] = v[2] - tr[6] * yd + tr[7] * xd;
-    for (int j = 0; j < 3; ++j) p[3 * e + j] = v[j] * w;
+    if (kepart) box_ke_part(acc, kepart);
 }
 
 }  // namespace
@@ -1905,10 +1919,10 @@ struct cam_box {
     uint64_t *step_base = nullptr;
     double nose_q = 0.0;               // Nose-Hoover chain on when > 0
     double *nhc = nullptr;             // chain state: 4 velocities and the last scale factor
-    double *nhc_part = nullptr;        // kinetic-energy parts (kBoxNhcBlocks)
+    double *nhc_part = nullptr;        // kinetic-energy parts (kBoxParts)
     bool transrot = false;             // remove centre-of-mass motion after every step (dynamic.x)
     double totmass = 0.0;              // transrot's nbeads^2 * M
-    double *tr = nullptr;              // transrot: partial sums and the solved velocities
+    double *tr = nullptr;              // transrot: partial sums
     bool have_state = false;
     std::map<int, hipGraphExec_t> graphs;
     hipEvent_t ev0 = nullptr, ev1 = nullptr, evf0 = nullptr, evf1 = nullptr;
@@ -1925,56 +1939,63 @@ int box_enqueue(cam_box *bx, int nsteps)
 {
     const int ncol = 3 * bx->natoms;
     const int cpb = 256 / bx->nb;
-    BoxNM a{ bx->q, bx->p, bx->g, bx->mass, bx->tfwd, bx->tinv, bx->natoms, bx->nb, bx->dt, bx->beta };
+    const bool nose = bx->nose_q > 0.0;
+    BoxNM a{ bx->q, bx->p, bx->g, bx->mass, bx->tfwd, bx->tinv, bx->natoms, bx->nb, bx->dt, bx->beta,
+             nose ? bx->nhc + 4 : nullptr, 0, { 0.0, 0.0, 0.0 } };
+    if (bx->ff->kind == 2) a.wrap = qmdff_box(bx->ff->qm, a.box);
     Theta th;
     std::memcpy(th.p, bx->theta, sizeof th.p);
     const size_t n = (size_t)ncol * bx->nb;
     const unsigned egrid = (unsigned)((n + 255) / 256);
-    auto chain = [&]() -> int {                        // src/verlet.f90:185-206, :1086-1106
-        if (bx->nose_q <= 0.0) return CAM_OK;
-        hipLaunchKernelGGL(box_ke_kernel, dim3(kBoxNhcBlocks), dim3(256), 0, bx->stream, bx->p, bx->mass, bx->natoms,
-                           bx->nb, bx->nhc_part);
-        CAM_LAUNCH_CHECK();
-        hipLaunchKernelGGL(box_nhc_kernel, dim3(1), dim3(64), 0, bx->stream, bx->nhc_part, kBoxNhcBlocks, bx->nhc,
+    // blocks of the kernels that leave one partial sum each
+    const unsigned pgrid = std::min<unsigned>(egrid, kBoxParts);
+    const unsigned agrid = std::min<unsigned>((unsigned)(((size_t)bx->natoms * bx->nb + 255) / 256), kTrApplyBlocks);
+    auto chain = [&](unsigned nparts) -> int {         // src/verlet.f90:185-206, :1086-1106
+        if (!nose) return CAM_OK;
+        hipLaunchKernelGGL(box_nhc_kernel, dim3(1), dim3(64), 0, bx->stream, bx->nhc_part, (int)nparts, bx->nhc,
                            bx->beta, bx->nose_q, bx->natoms, bx->nb, bx->dt);
-        CAM_LAUNCH_CHECK();
-        hipLaunchKernelGGL(box_scale_kernel, dim3(egrid), dim3(256), 0, bx->stream, bx->p, n, bx->nhc);
         CAM_LAUNCH_CHECK();
         return CAM_OK;
     };
+    if (nose && nsteps > 0) {
+        hipLaunchKernelGGL(box_ke_kernel, dim3(pgrid), dim3(256), 0, bx->stream, bx->p, bx->mass, bx->natoms, bx->nb,
+                           bx->nhc_part);
+        CAM_LAUNCH_CHECK();
+    }
+    unsigned parts = pgrid;                            // of the kinetic energy the last kernel left
     for (int s = 0; s < nsteps; ++s) {
-        int rc0 = chain();
+        int rc0 = chain(parts);
         if (rc0 != CAM_OK) return rc0;
         hipLaunchKernelGGL(box_nm_kernel, dim3((ncol + cpb - 1) / cpb), dim3(256), 2 * 256 * sizeof(double), bx->stream,
                            a);
         CAM_LAUNCH_CHECK();
-        if (bx->ff->kind == 2) {                       // the periodic wrap of src/verlet.f90:540-640
-            const int rw = qmdff_wrap(bx->ff->qm, bx->q, bx->nb, bx->stream);
-            if (rw != CAM_OK) return rw;
-        }
         int rc = bx->precision == CAM_PREC_MIXED
                      ? ff_launch<float>(bx->ff, th, bx->q, bx->nb, bx->e, bx->g, nullptr, nullptr, nullptr, bx->stream)
                      : ff_launch<double>(bx->ff, th, bx->q, bx->nb, bx->e, bx->g, nullptr, nullptr, nullptr, bx->stream);
         if (rc != CAM_OK) return rc;
-        hipLaunchKernelGGL(box_kick_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, bx->stream, bx->p, bx->g,
-                           bx->mass, bx->natoms, bx->nb, bx->dt, bx->beta, bx->andersen_step, bx->seed, bx->step_base, s);
+        hipLaunchKernelGGL(box_kick_kernel, dim3(nose ? pgrid : egrid), dim3(256), 0, bx->stream, bx->p, bx->g,
+                           bx->mass, bx->natoms, bx->nb, bx->dt, bx->beta, bx->andersen_step, bx->seed, bx->step_base, s,
+                           nose ? bx->nhc_part : nullptr);
         CAM_LAUNCH_CHECK();
-        rc = chain();
+        rc = chain(pgrid);
         if (rc != CAM_OK) return rc;
         if (bx->transrot) {                             // src/verlet.f90:1299-1305
-            double *part1 = bx->tr + 16, *part2 = part1 + 6 * kTrBlocks;
+            double *part1 = bx->tr, *part2 = part1 + 6 * kTrBlocks;
             hipLaunchKernelGGL(box_tr_pass1, dim3(kTrBlocks), dim3(256), 0, bx->stream, bx->q, bx->p, bx->mass,
-                               bx->natoms, bx->nb, part1);
+                               bx->natoms, bx->nb, a.scale, part1);
             CAM_LAUNCH_CHECK();
             hipLaunchKernelGGL(box_tr_pass2, dim3(kTrBlocks), dim3(256), 0, bx->stream, bx->q, bx->p, bx->mass,
-                               bx->natoms, bx->nb, part1, bx->totmass, bx->tr, part2);
+                               bx->natoms, bx->nb, part1, bx->totmass, part2);
             CAM_LAUNCH_CHECK();
-            hipLaunchKernelGGL(box_tr_solve, dim3(1), dim3(64), 0, bx->stream, part2, bx->natoms, bx->totmass, bx->tr);
+            hipLaunchKernelGGL(box_tr_apply, dim3(agrid), dim3(256), 0, bx->stream, bx->q, bx->p, bx->mass, bx->natoms,
+                               bx->nb, part1, part2, bx->totmass, nose ? bx->nhc_part : nullptr);
             CAM_LAUNCH_CHECK();
-            const size_t ne = (size_t)bx->natoms * bx->nb;
-            hipLaunchKernelGGL(box_tr_apply, dim3((unsigned)((ne + 255) / 256)), dim3(256), 0, bx->stream, bx->q,
-                               bx->p, bx->mass, bx->natoms, bx->nb, bx->tr);
+            parts = agrid;
+        } else if (nose) {
+            hipLaunchKernelGGL(box_scale_kernel, dim3(pgrid), dim3(256), 0, bx->stream, bx->p, bx->mass, bx->natoms,
+                               bx->nb, a.scale, bx->nhc_part);
             CAM_LAUNCH_CHECK();
+            parts = pgrid;
         }
     }
     hipLaunchKernelGGL(box_advance_kernel, dim3(1), dim3(1), 0, bx->stream, bx->step_base, nsteps);
@@ -2085,7 +2106,7 @@ int cam_box_set_transrot(cam_box *bx, int on)
 {
     CAM_CHECK_ARG(bx, "null box");
     clear_error();
-    if (on && !bx->tr) CAM_HIP(hipMalloc(&bx->tr, (16 + 15 * (size_t)kTrBlocks) * sizeof(double)));
+    if (on && !bx->tr) CAM_HIP(hipMalloc(&bx->tr, 15 * (size_t)kTrBlocks * sizeof(double)));
     // the reference's total mass: every atom counted once per bead, then
     // times nbeads (src/transrot.f90:62-72)
     std::vector<double> m(bx->natoms);
@@ -2108,7 +2129,7 @@ int cam_box_set_nhc(cam_box *bx, double nose_q)
     clear_error();
     if (nose_q > 0.0 && !bx->nhc) {
         CAM_HIP(hipMalloc(&bx->nhc, 5 * sizeof(double)));
-        CAM_HIP(hipMalloc(&bx->nhc_part, kBoxNhcBlocks * sizeof(double)));
+        CAM_HIP(hipMalloc(&bx->nhc_part, kBoxParts * sizeof(double)));
     }
     if (bx->nhc) CAM_HIP(hipMemsetAsync(bx->nhc, 0, 5 * sizeof(double), bx->stream));
     CAM_HIP(hipStreamSynchronize(bx->stream));

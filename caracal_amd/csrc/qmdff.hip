@@ -915,81 +915,6 @@ __global__ __launch_bounds__(64) void qm_reduce_kernel(const double *eslot, int 
     if (lane == 0) e[b] = s;
 }
 
-// src/verlet.f90:540-640 (orthorhombic box): an atom whose coordinate left
-// [0, L] in some bead is moved with all its beads, bead by bead in order.
-// One lane per (atom, coordinate): the beads are read in chunks of
-// independent loads and the shifts recorded in order; the rare lane that
-// shifts applies them to every bead in that order, as the reference adds them.
-constexpr int kWrapChunk = 16, kWrapMaxShift = 8;
-
-__global__ void qm_wrap_kernel(QDev f, double *x, int nbeads)
-{
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= 3 * f.n) return;
-    const int i = t / 3, c = t % 3;
-    const double L = f.box[c];
-    // the shifts so far, in registers (every index below is a constant)
-    double sh[kWrapMaxShift];
-#pragma unroll
-    for (int s = 0; s < kWrapMaxShift; ++s) sh[s] = 0.0;
-    int ns = 0;
-    bool over = false;
-    auto push = [&](double d) {
-        if (ns == kWrapMaxShift) {
-            over = true;
-            return;
-        }
-#pragma unroll
-        for (int s = 0; s < kWrapMaxShift; ++s)
-            if (s == ns) sh[s] = d;
-        ++ns;
-    };
-    auto shifted = [&](double w) {
-#pragma unroll
-        for (int s = 0; s < kWrapMaxShift; ++s)
-            if (s < ns) w = w + sh[s];
-        return w;
-    };
-    for (int k0 = 0; k0 < nbeads && !over; k0 += kWrapChunk) {
-        double v[kWrapChunk];
-#pragma unroll
-        for (int u = 0; u < kWrapChunk; ++u)
-            v[u] = k0 + u < nbeads ? x[((size_t)(k0 + u) * f.n + i) * 3 + c] : 0.5 * L;
-#pragma unroll
-        for (int u = 0; u < kWrapChunk; ++u) {
-            if (k0 + u >= nbeads || over) continue;
-            double w = shifted(v[u]);
-            while (w < 0.0 && !over) {
-                push(L);
-                if (!over) w = w + L;
-            }
-            while (w > L && !over) {
-                push(-L);
-                if (!over) w = w - L;
-            }
-        }
-    }
-    if (over) {                                 // many shifts: the reference's loop on memory
-        for (int k = 0; k < nbeads; ++k) {
-            int tries = 0;
-            while (x[((size_t)k * f.n + i) * 3 + c] < 0.0 && tries <= 100) {
-                for (int kk = 0; kk < nbeads; ++kk) x[((size_t)kk * f.n + i) * 3 + c] += L;
-                ++tries;
-            }
-            while (x[((size_t)k * f.n + i) * 3 + c] > L && tries <= 100) {
-                for (int kk = 0; kk < nbeads; ++kk) x[((size_t)kk * f.n + i) * 3 + c] -= L;
-                ++tries;
-            }
-        }
-        return;
-    }
-    if (ns == 0) return;
-    for (int k = 0; k < nbeads; ++k) {
-        double *p = x + ((size_t)k * f.n + i) * 3 + c;
-        *p = shifted(*p);
-    }
-}
-
 template <typename Tv>
 int upload(QmdffDev *q, const std::vector<Tv> &v, const Tv **out)
 {
@@ -1244,13 +1169,10 @@ int qmdff_launch(QmdffDev *q, const double *x, int nbeads, double *e, double *g,
 template int qmdff_launch<double>(QmdffDev *, const double *, int, double *, double *, hipStream_t);
 template int qmdff_launch<float>(QmdffDev *, const double *, int, double *, double *, hipStream_t);
 
-int qmdff_wrap(QmdffDev *q, double *x, int nbeads, hipStream_t s)
+bool qmdff_box(const QmdffDev *q, double box[3])
 {
-    if (!q->d.periodic) return CAM_OK;
-    const int nt = 3 * q->d.n;
-    hipLaunchKernelGGL(qm_wrap_kernel, dim3((nt + 255) / 256), dim3(256), 0, s, q->d, x, nbeads);
-    CAM_LAUNCH_CHECK();
-    return CAM_OK;
+    for (int c = 0; c < 3; ++c) box[c] = q->d.box[c];
+    return q->d.periodic != 0;
 }
 
 }  // namespace cam

@@ -16,9 +16,9 @@ int qmdff_natoms(const QmdffDev *q);
 // arithmetic (double or float with compensated sums).
 template <typename T>
 int qmdff_launch(QmdffDev *q, const double *x, int nbeads, double *e, double *g, hipStream_t s);
-// The reference's periodic wrap of every atom's ring polymer into the box
-// after the free ring-polymer step (src/verlet.f90:540-640); no-op when the
-// force field is not periodic.
-int qmdff_wrap(QmdffDev *q, double *x, int nbeads, hipStream_t s);
+// Whether the force field is periodic, and its box lengths: the engine then
+// wraps every atom's ring polymer into the box after the free ring-polymer
+// step (src/verlet.f90:540-640).
+bool qmdff_box(const QmdffDev *q, double box[3]);
 
 }  // namespace cam
