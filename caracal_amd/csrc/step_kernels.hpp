@@ -591,8 +591,11 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE))) v
         nred[tid] = part;
         __syncthreads();
         if (live && k == 0 && r == 0) {
-            double ek = 0.0;
-            for (int i = 0; i < NB * L; ++i) ek += nred[tl * NB * L + i];
+            // four sums, so that the additions do not wait for each other
+            double es[4] = { 0.0, 0.0, 0.0, 0.0 };
+#pragma unroll
+            for (int i = 0; i < NB * L; ++i) es[i & 3] += nred[tl * NB * L + i];
+            const double ek = (es[0] + es[1]) + (es[2] + es[3]);
             nscale[tl] = nhc_chain(vnh, qnh, ek / NB / NB, ekt_chain, NC, a.dt);
         }
         __syncthreads();
