@@ -535,28 +535,26 @@ __device__ void qhblist(const QDev &f, const double *x, int m, int role, double 
     for (int c = 0; c < 3; ++c) gv[c] = s[c];
 }
 
-// Intermolecular hydrogen bond of donor bond dn against acceptor slot ac
-// (src/ff_hb.f90:198-276): eabhag(j, A, H) when its distance conditions hold
-__device__ double qhbinter(const QDev &f, const double *x, int dn, int ac, double *gj, double *ga, double *gh)
+// Whether the intermolecular hydrogen bond of donor bond dn and acceptor slot
+// ac, eabhag(j, A, H), counts (src/ff_hb.f90:198-276)
+__device__ bool qhbnear(const QDev &f, const double *x, int dn, int ac)
 {
     const int A = f.don[2 * dn], H = f.don[2 * dn + 1], j = f.acc[ac];
-    gj[0] = gj[1] = gj[2] = ga[0] = ga[1] = ga[2] = gh[0] = gh[1] = gh[2] = 0.0;
-    if (f.mol[H] == f.mol[j]) return 0.0;
-    const double cpar = f.scal[A] * f.scal[j];
-    if (!(cpar > 1e-6)) return 0.0;
+    if (f.mol[H] == f.mol[j]) return false;
     double d[3];
+    qsub(x, A, j, d);
+    qimg(f, d);
+    const double r = sqrt((d[0] * d[0] + d[1] * d[1]) + d[2] * d[2]);
+    if (r > 15.0) return false;
+    const double cpar = f.scal[A] * f.scal[j];
+    if (!(cpar > 1e-6)) return false;
     qsub(x, A, H, d);
     qimg(f, d);
     const double ri = sqrt((d[0] * d[0] + d[1] * d[1]) + d[2] * d[2]);
     qsub(x, j, H, d);
     qimg(f, d);
     const double rj = sqrt((d[0] * d[0] + d[1] * d[1]) + d[2] * d[2]);
-    if (!(ri < f.don_lim[dn] || rj < f.acc_lim[ac])) return 0.0;
-    qsub(x, A, j, d);
-    qimg(f, d);
-    const double r = sqrt((d[0] * d[0] + d[1] * d[1]) + d[2] * d[2]);
-    if (r > 15.0) return 0.0;
-    return qeabhag(f, x, j, A, H, f.hbc[j], f.hbc[A], gj, ga, gh);
+    return ri < f.don_lim[dn] || rj < f.acc_lim[ac];
 }
 
 // ---------------------------------------------------------------------------
@@ -599,6 +597,15 @@ struct QTile {
     double tab[5][kQMaxElem * kQMaxElem];
     double e[kQWaves];
 };
+
+// A wave's LDS queue is its own and its LDS accesses are in order: no barrier,
+// only no reordering by the compiler.
+__device__ __forceinline__ void qwave_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 
 template <typename T>
 __device__ void qinter(const QDev &f, const double *__restrict__ x, int blk, QTile &s, double *gpart, double *epart)
@@ -701,19 +708,14 @@ __device__ void qinter(const QDev &f, const double *__restrict__ x, int blk, QTi
             const unsigned long long m = __ballot(in);
             if (in) s.queue[wave][count + __popcll(m & ((1ull << lane) - 1ull))] = (t0 + u) | s.elem[uu] << 20;
             count += __popcll(m);
-            // the queue is this wave's alone and its LDS accesses are in order
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            qwave_fence();
             const bool last = t0 + u0 + 64 >= n;
             while (count >= 64 || (last && count > 0)) {
                 const int k = min(count, 64);
                 pairs(k);
                 count -= k;
                 const int rest = s.queue[wave][64 + lane];
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                qwave_fence();
                 if (lane < count) s.queue[wave][lane] = rest;
             }
         }
@@ -768,57 +770,60 @@ __device__ void qslot(const QDev &f, const double *__restrict__ x, int blk, doub
     if (threadIdx.x == 0) *eslot = ((sred[0] + sred[1]) + sred[2]) + sred[3];
 }
 
-// acceptor side: one wave per acceptor atom, lanes over the donor bonds; the
-// acceptor's gradient and the energy (butterfly sums: a fixed order)
-__device__ void qhbacc(const QDev &f, const double *__restrict__ x, int ac, double *gacc, double *eacc)
+// Intermolecular hydrogen bonds, one wave per acceptor against all donor bonds
+// (gradient of the acceptor and energy) or, DON, per donor bond against all
+// acceptors (gradients of A and H); butterfly sums, a fixed order.
+//
+// A tenth of the pairs lies within the 15 bohr of the term, so a few lanes of
+// each 64 had a bond and the wave went through all of it for them, once per 64
+// partners.  Now those that count are queued and evaluated together, and the
+// blocks come first in the grid, as the waves with the longest chains: a force
+// call of 1125 atoms x 16 beads 130 -> 115 us.  Two or four acceptors to a wave
+// fill the evaluations better, but the longer chains cost more (122 and 138 us).
+template <bool DON>
+__device__ void qhb(const QDev &f, const double *__restrict__ x, int own, QTile &s, double *gout, double *eout)
 {
-    const int lane = threadIdx.x & 63;
-    if (ac >= f.nacc) return;
-    double g[3] = { 0.0, 0.0, 0.0 }, e = 0.0, gj[3], ga[3], gh[3];
-    for (int dn = lane; dn < f.ndon; dn += 64) {
-        e = e + qhbinter(f, x, dn, ac, gj, ga, gh);
-        g[0] = g[0] + gj[0];
-        g[1] = g[1] + gj[1];
-        g[2] = g[2] + gj[2];
+    const int lane = threadIdx.x & 63, n2 = DON ? f.nacc : f.ndon;
+    if (own >= (DON ? f.ndon : f.nacc)) return;
+    int *queue = s.queue[threadIdx.x >> 6];
+    double sum[6] = { 0.0, 0.0, 0.0, 0.0, 0.0, 0.0 };
+    int count = 0;
+    for (int o0 = 0; o0 < n2; o0 += 64) {
+        const int o = o0 + lane;
+        const bool in = o < n2 && qhbnear(f, x, DON ? own : o, DON ? o : own);
+        const unsigned long long m = __ballot(in);
+        if (in) queue[count + __popcll(m & ((1ull << lane) - 1ull))] = o;
+        count += __popcll(m);
+        qwave_fence();
+        const bool last = o0 + 64 >= n2;
+        while (count >= 64 || (last && count > 0)) {
+            const int k = min(count, 64);
+            const int other = queue[lane < k ? lane : 0], rest = queue[64 + lane];
+            const int dn = DON ? own : other, A = f.don[2 * dn], H = f.don[2 * dn + 1];
+            const int j = f.acc[DON ? other : own];
+            double gj[3], ga[3], gh[3];
+            const double e = qeabhag(f, x, j, A, H, f.hbc[j], f.hbc[A], gj, ga, gh);
+            if (lane < k) {
+                for (int c = 0; c < 3; ++c) {
+                    sum[c] = sum[c] + (DON ? ga[c] : gj[c]);
+                    if (DON) sum[3 + c] = sum[3 + c] + gh[c];
+                }
+                if (!DON) sum[3] = sum[3] + e;
+            }
+            count -= k;
+            if (lane < count) queue[lane] = rest;
+            qwave_fence();
+        }
     }
-    for (int o = 32; o > 0; o >>= 1) {
-        e = e + __shfl_xor(e, o);
-        for (int c = 0; c < 3; ++c) g[c] = g[c] + __shfl_xor(g[c], o);
-    }
-    if (lane == 0) {
-        for (int c = 0; c < 3; ++c) gacc[3 * (size_t)ac + c] = g[c];
-        eacc[ac] = e;
-    }
+    for (int c = 0; c < (DON ? 6 : 4); ++c)
+        for (int t = 32; t > 0; t >>= 1) sum[c] = sum[c] + __shfl_xor(sum[c], t);
+    if (lane != 0) return;
+    for (int c = 0; c < (DON ? 6 : 3); ++c) gout[(size_t)(DON ? 6 : 3) * own + c] = sum[c];
+    if (!DON) eout[own] = sum[3];
 }
 
-// donor side: one wave per donor bond, lanes over the acceptors; the A and H gradients
-__device__ void qhbdon(const QDev &f, const double *__restrict__ x, int dn, double *gdon)
-{
-    const int lane = threadIdx.x & 63;
-    if (dn >= f.ndon) return;
-    double sa[3] = { 0.0, 0.0, 0.0 }, sh[3] = { 0.0, 0.0, 0.0 }, gj[3], ga[3], gh[3];
-    for (int ac = lane; ac < f.nacc; ac += 64) {
-        (void)qhbinter(f, x, dn, ac, gj, ga, gh);
-        for (int c = 0; c < 3; ++c) {
-            sa[c] = sa[c] + ga[c];
-            sh[c] = sh[c] + gh[c];
-        }
-    }
-    for (int o = 32; o > 0; o >>= 1)
-        for (int c = 0; c < 3; ++c) {
-            sa[c] = sa[c] + __shfl_xor(sa[c], o);
-            sh[c] = sh[c] + __shfl_xor(sh[c], o);
-        }
-    if (lane == 0) {
-        for (int c = 0; c < 3; ++c) {
-            gdon[(size_t)dn * 6 + c] = sa[c];
-            gdon[(size_t)dn * 6 + 3 + c] = sh[c];
-        }
-    }
-}
-
-// Blocks of one bead (blockIdx.y), in this order: ninter of the intermolecular
-// pairs, nacc and ndon of the hydrogen bonds, nslot of the slots.  One launch:
+// Blocks of one bead (blockIdx.y): in this order nacc and ndon of the hydrogen
+// bonds, nslot of the slots, ninter of the intermolecular pairs.  One launch:
 // the hydrogen-bond and slot blocks, 17 to 25 us each as kernels of their own
 // that fill a part of the chip, run beside the pairs.
 struct QBlocks {
@@ -840,22 +845,22 @@ __global__ __launch_bounds__(kQTile) __attribute__((amdgpu_waves_per_eu(5))) voi
     const int b = blockIdx.y, wave = threadIdx.x >> 6;
     const double *x = xall + (size_t)b * f.n * 3;
     int k = blockIdx.x;
-    if (k < nb.ninter) {
-        qinter<T>(f, x, k, s, gpart + (size_t)b * f.n * 3, epart + (size_t)b * nb.ninter + k);
-        return;
-    }
-    k -= nb.ninter;
     if (k < nb.nacc) {
-        qhbacc(f, x, k * kQWaves + wave, gacc + (size_t)b * f.nacc * 3, eacc + (size_t)b * f.nacc);
+        qhb<false>(f, x, k * kQWaves + wave, s, gacc + (size_t)b * f.nacc * 3, eacc + (size_t)b * f.nacc);
         return;
     }
     k -= nb.nacc;
     if (k < nb.ndon) {
-        qhbdon(f, x, k * kQWaves + wave, gdon + (size_t)b * f.ndon * 6);
+        qhb<true>(f, x, k * kQWaves + wave, s, gdon + (size_t)b * f.ndon * 6, nullptr);
         return;
     }
     k -= nb.ndon;
-    qslot(f, x, k, s.e, gslot + (size_t)b * f.nslot * 3, eslot + (size_t)b * nb.nslot + k);
+    if (k < nb.nslot) {
+        qslot(f, x, k, s.e, gslot + (size_t)b * f.nslot * 3, eslot + (size_t)b * nb.nslot + k);
+        return;
+    }
+    k -= nb.nslot;
+    qinter<T>(f, x, k, s, gpart + (size_t)b * f.n * 3, epart + (size_t)b * nb.ninter + k);
 }
 
 // Four lanes per (bead, atom): its term slots and hydrogen-bond parts, every
