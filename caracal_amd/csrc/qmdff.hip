@@ -589,7 +589,7 @@ __device__ __forceinline__ float qrsq(float a) { return 1.0f / sqrtf(a); }
 // the sums over the lanes are butterflies, in a fixed order.  The per-element
 // tables are in LDS, C6 is read along the row of i, one reciprocal stands for
 // 1/t6 and 1/t8 and one reciprocal root for r and 1/r: with the slots and the
-// hydrogen bonds in the same launch 113 us, 329 us as four kernels before.
+// hydrogen bonds in the same launch 98 us, 329 us as four kernels before.
 struct QTile {
     double x[3][kQTile];                // j atoms of the tile
     int mol[kQTile], elem[kQTile];
