@@ -40,6 +40,7 @@ namespace cam {
 
 constexpr int kQTile = 256;         // lanes per block; j atoms per LDS tile
 constexpr int kQWaves = kQTile / 64;    // waves per block: atoms i of an intermolecular block
+constexpr int kQSplit = 8;          // parts of the j range that are summed on their own
 constexpr int kQMaxElem = 16;       // distinct elements of one force field
 constexpr int kQImageCap = 64;      // minimum-image iterations (the reference loops until inside)
 
@@ -374,11 +375,15 @@ __device__ void qtors(const QDev &f, const double *x, int m, int role, double &e
 }
 
 // Dispersion and repulsion of the pair (a, b) scaled by s, gradient on a for
-// d = x_a - x_b (src/ff_nonb.f90:118-175, :228-320); T is the arithmetic.
+// d = x_a - x_b (src/ff_nonb.f90:118-175, :228-320); T is the arithmetic, t
+// the element tables (of QDev, or their copy in LDS) and pe the pair's place.
+struct QTables {
+    const double *r0, *r06, *sr42, *zab, *alpha;
+};
+
 template <typename T>
-__device__ inline void qdisp_rep(const QDev &f, int ea, int eb, double c6d, const T *d, T r2, T r, T s, T &e, T *ga)
+__device__ inline void qdisp_rep(const QTables &f, int pe, double c6d, const T *d, T r2, T r, T s, T &e, T *ga)
 {
-    const int pe = ea * f.ne + eb;
     const T R0 = (T)f.r0[pe];
     const T c6 = (T)c6d;
     const T r4 = r2 * r2, r6 = r4 * r2;
@@ -434,8 +439,9 @@ __device__ void qnci(const QDev &f, const double *x, int m, int role, double &e,
     const double vdw = f.periodic ? f.vdw_cut : 10.0 / 0.52917721092;
     double ga[3] = { 0.0, 0.0, 0.0 }, gc[3];
     e = 0.0;
-    if (!(f.periodic && r > vdw)) qdisp_rep<double>(f, f.elem[i1], f.elem[i2], f.c6[(size_t)i1 * f.n + i2], d, r2, r,
-                                                    f.eps2[nk], e, ga);
+    if (!(f.periodic && r > vdw))
+        qdisp_rep<double>({ f.r0, f.r06, f.sr42, f.zab, f.alpha }, f.elem[i1] * f.ne + f.elem[i2],
+                          f.c6[(size_t)i1 * f.n + i2], d, r2, r, f.eps2[nk], e, ga);
     double ec;
     if (qcoulomb<double>(f, f.q[i1], f.q[i2], d, r2, r, f.eps1[nk], ec, gc)) {
         e = e + ec;
@@ -445,7 +451,13 @@ __device__ void qnci(const QDev &f, const double *x, int m, int role, double &e,
     for (int c = 0; c < 3; ++c) gv[c] = sgn * ga[c];
 }
 
-// eabhag (src/eabhag.f90): energy and the gradient of all three atoms
+// eabhag (src/eabhag.f90): energy and the gradient of all three atoms.  PART
+// kHbAcceptor: only the energy and ga are used, kHbDonor: only gb and gh.
+// Those two state which product of a sum is rounded: left to the compiler it
+// is one or the other with what else is in the kernel, and the bits with it.
+enum { kHbListed = 0, kHbAcceptor = 1, kHbDonor = 2 };
+
+template <int PART>
 __device__ double qeabhag(const QDev &f, const double *x, int A, int B, int H, double ca, double cb, double *ga,
                           double *gb, double *gh)
 {
@@ -477,7 +489,9 @@ __device__ double qeabhag(const QDev &f, const double *x, int A, int B, int H, d
     aterm = aterm * apref;
     apref = alp3 * 0.5 * apref;
     const double rah4 = rah2 * rah2, rbh4 = rbh2 * rbh2;
-    const double denom = 1.0 / (rah4 + rbh4);
+    const double denom = 1.0 / (PART == kHbListed     ? rah4 + rbh4
+                                : PART == kHbAcceptor ? fma(rah2, rah2, rbh4)
+                                                      : fma(rbh2, rbh2, rah4));
     const double da = (ca * rah4 + cb * rbh4) * denom;
     const double eabh = -da * rdampl * aterm;
     if (eabh > -1e-8) {
@@ -486,34 +500,43 @@ __device__ double qeabhag(const QDev &f, const double *x, int A, int B, int H, d
     }
     double gi = 4.0 * (ca - cb) * rah2 * rbh4 * denom * denom;
     gi = -gi * rdampl * aterm;
-    for (int c = 0; c < 3; ++c) ga[c] = gi * drah[c];
-    gi = 4.0 * (cb - ca) * rbh2 * rah4 * denom * denom;
-    gi = -gi * rdampl * aterm;
-    for (int c = 0; c < 3; ++c) gb[c] = gi * drbh[c];
-    for (int c = 0; c < 3; ++c) gh[c] = -ga[c] - gb[c];
-    gi = rdampl * rdampl * rab * (3.0 + (3.0 + alp7) * ratio);
-    gi = gi * da * aterm;
-    for (int c = 0; c < 3; ++c) {
-        dg[c] = gi * drab[c];
-        ga[c] = ga[c] + dg[c];
-        gb[c] = gb[c] - dg[c];
-    }
-    gi = -da * rdampl * apref;
-    if (rah2 > rbh2) {
+    double gib = 4.0 * (cb - ca) * rbh2 * rah4 * denom * denom;
+    gib = -gib * rdampl * aterm;
+    double gd = rdampl * rdampl * rab * (3.0 + (3.0 + alp7) * ratio);
+    gd = gd * da * aterm;
+    const double ge = -da * rdampl * apref;
+    if constexpr (PART == kHbListed) {
+        for (int c = 0; c < 3; ++c) ga[c] = gi * drah[c];
+        for (int c = 0; c < 3; ++c) gb[c] = gib * drbh[c];
+        for (int c = 0; c < 3; ++c) gh[c] = -ga[c] - gb[c];
         for (int c = 0; c < 3; ++c) {
-            dg[c] = gi * (-aprod * drbh[c] - cosabh * drab[c] / rab2);
-            dg2[c] = gi * (aprod * drab[c] + cosabh * drbh[c] / rbh2);
+            dg[c] = gd * drab[c];
             ga[c] = ga[c] + dg[c];
-            gh[c] = gh[c] + dg2[c];
-            gb[c] = gb[c] - dg[c] - dg2[c];
+            gb[c] = gb[c] - dg[c];
         }
     } else {
         for (int c = 0; c < 3; ++c) {
-            dg[c] = gi * (-aprod * drah[c] + cosabh * drab[c] / rab2);
-            dg2[c] = gi * (-aprod * drab[c] + cosabh * drah[c] / rah2);
-            gb[c] = gb[c] + dg[c];
-            gh[c] = gh[c] + dg2[c];
-            ga[c] = ga[c] - dg[c] - dg2[c];
+            const double gbh = gib * drbh[c];
+            ga[c] = fma(gd, drab[c], gi * drah[c]);
+            gb[c] = fma(-gd, drab[c], gbh);
+            gh[c] = fma(-gi, drah[c], -gbh);
+        }
+    }
+    if (rah2 > rbh2) {
+        for (int c = 0; c < 3; ++c) {
+            dg[c] = fma(-aprod, drbh[c], -(cosabh * drab[c] / rab2));
+            dg2[c] = fma(aprod, drab[c], cosabh * drbh[c] / rbh2);
+            ga[c] = fma(ge, dg[c], ga[c]);
+            gh[c] = fma(ge, dg2[c], gh[c]);
+            gb[c] = fma(-ge, dg2[c], fma(-ge, dg[c], gb[c]));
+        }
+    } else {
+        for (int c = 0; c < 3; ++c) {
+            dg[c] = fma(-aprod, drah[c], cosabh * drab[c] / rab2);
+            dg2[c] = fma(-aprod, drab[c], cosabh * drah[c] / rah2);
+            gb[c] = fma(ge, dg[c], gb[c]);
+            gh[c] = fma(ge, dg2[c], gh[c]);
+            ga[c] = fma(-ge, dg2[c], fma(-ge, dg[c], ga[c]));
         }
     }
     return eabh;
@@ -530,7 +553,7 @@ __device__ void qhblist(const QDev &f, const double *x, int m, int role, double 
     e = 0.0;
     gv[0] = gv[1] = gv[2] = 0.0;
     if (r > 15.0) return;
-    e = qeabhag(f, x, a, b, h, f.vhb[2 * m], f.vhb[2 * m + 1], ga, gb, gh);
+    e = qeabhag<kHbListed>(f, x, a, b, h, f.vhb[2 * m], f.vhb[2 * m + 1], ga, gb, gh);
     const double *s = role == 0 ? ga : role == 1 ? gb : gh;
     for (int c = 0; c < 3; ++c) gv[c] = s[c];
 }
@@ -559,41 +582,57 @@ __device__ bool qhbnear(const QDev &f, const double *x, int dn, int ac)
 
 // ---------------------------------------------------------------------------
 
-// FP64 reciprocal and reciprocal square root from the hardware estimates with
-// two Newton steps each (positive normal arguments); binary32: 1 ulp.
-__device__ __forceinline__ double qrcp(double a)
-{
-    double y = __builtin_amdgcn_rcp(a);
-    y = y * fma(-a, y, 2.0);
-    return y * fma(-a, y, 2.0);
-}
-__device__ __forceinline__ float qrcp(float a) { return 1.0f / a; }
-__device__ __forceinline__ double qrsq(double a)
-{
-    double y = __builtin_amdgcn_rsq(a);
-    const double h = 0.5 * a;
-    y = y * fma(-h * y, y, 1.5);
-    return y * fma(-h * y, y, 1.5);
-}
-__device__ __forceinline__ float qrsq(float a) { return 1.0f / sqrtf(a); }
+// Sums of an atom's pair terms: FP64, compensated where the terms are binary32.
+template <typename T>
+struct QAcc {
+    double s = 0.0;
+    __device__ void add(T v) { s = s + (double)v; }
+    __device__ double get() const { return s; }
+};
+template <>
+struct QAcc<float> {
+    double s = 0.0, c = 0.0;
+    __device__ void add(float v)
+    {
+        const double y = (double)v - c;
+        const double t = s + y;
+        c = (t - s) - y;
+        s = t;
+    }
+    __device__ double get() const { return s; }
+};
 
-// Intermolecular pairs of atom i (one wave) with every other atom of a bead,
-// terms as qdisp_rep and qcoulomb.
+// a + b, never fused with the product that a or b is.
+template <typename T>
+__device__ __forceinline__ T qadd(T a, T b)
+{
+#pragma clang fp contract(off)
+    return a + b;
+}
+
+// Intermolecular pairs of atom i (one wave) with every other atom of a bead.
 //
 // A fifth of the atoms of the 51 bohr ethanol box lies within the 19 bohr
 // cutoff.  With a lane per atom i and the block's 64 or 256 atoms walking all j
 // together, nearly every j was inside for some lane, so every lane went
 // through the whole pair (262 us for 1125 atoms x 16 beads).  Here the lanes
-// stand for 64 atoms j: the distance check is 1/5 of a pair's work, those
-// inside are compacted into a queue, and the pair runs with all lanes full;
-// the sums over the lanes are butterflies, in a fixed order.  The per-element
-// tables are in LDS, C6 is read along the row of i, one reciprocal stands for
-// 1/t6 and 1/t8 and one reciprocal root for r and 1/r: with the slots and the
-// hydrogen bonds in the same launch 98 us, 329 us as four kernels before.
+// stand for 64 atoms j: the distance check is a small part of a pair's work,
+// those inside are queued, and the pair runs with the lanes full.
+//
+// The j range is summed in eighths, each in the order of j, and the gather adds
+// the eighths in order: these are the sums, and the pair's are the operations,
+// of lanes that walk an eighth each.  Summed over the lanes, or with 1/r and
+// 1/t6 from reciprocal estimates (115 us a force call of 16 beads instead of
+// 148), forces move by an ulp, which a torsion next to planar (1/sin phi) makes
+// 1e-9 of the momenta in 50 steps.  A step takes eight atoms of every eighth,
+// so that a batch holds some of each and the additions, which wait for each
+// other, are few in a row: four lanes per eighth add the batch's terms from LDS
+// (with the atoms taken in order, 28 in a row instead of 8, a call took 160 us).
 struct QTile {
     double x[3][kQTile];                // j atoms of the tile
-    int mol[kQTile], elem[kQTile];
-    int queue[kQWaves][128];            // per wave: accepted atoms, at most 63 + 64: j and its element << 20
+    int mol[kQTile];
+    unsigned short queue[kQWaves][kQSplit][64];    // per wave and eighth: accepted atoms, from the eighth's first
+    double res[kQWaves][67 * 4];        // per wave: the terms of a batch, [component][lane] (binary32 ones exact)
     double tab[5][kQMaxElem * kQMaxElem];
     double e[kQWaves];
 };
@@ -607,8 +646,10 @@ __device__ __forceinline__ void qwave_fence()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// gpart: [eighth][bead][atom][3], here at this bead; stride between eighths.
 template <typename T>
-__device__ void qinter(const QDev &f, const double *__restrict__ x, int blk, QTile &s, double *gpart, double *epart)
+__device__ void qinter(const QDev &f, const double *__restrict__ x, int blk, QTile &s, double *gpart, size_t stride,
+                       double *epart)
 {
     const int n = f.n, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int i = blk * kQWaves + wave;
@@ -616,7 +657,7 @@ __device__ void qinter(const QDev &f, const double *__restrict__ x, int blk, QTi
     const int ii = act ? i : n - 1;
     const double xi0 = x[3 * ii], xi1 = x[3 * ii + 1], xi2 = x[3 * ii + 2];
     const int mi = f.mol[ii], ei = f.elem[ii] * f.ne;
-    const T qi = (T)f.q[ii];
+    const double qi = f.q[ii];
     const double *c6 = f.c6 + (size_t)ii * n;
     for (int k = tid; k < f.ne * f.ne; k += kQTile) {
         s.tab[0][k] = f.r0[k];
@@ -625,115 +666,89 @@ __device__ void qinter(const QDev &f, const double *__restrict__ x, int blk, QTi
         s.tab[3][k] = f.zab[k];
         s.tab[4][k] = f.alpha[k];
     }
-    const T vdw = (T)f.vdw_cut, coul = (T)f.coul_cut;
+    const T vdw = f.periodic ? (T)f.vdw_cut : (T)(10.0 / 0.52917721092);
     // the queue holds every pair either cutoff takes; a NaN distance is kept
     const double rmax = f.vdw_cut > f.coul_cut ? f.vdw_cut : f.coul_cut;
     const double cut2 = f.periodic ? rmax * rmax * (1.0 + 1e-6) : INFINITY;
-    auto image = [&](double *d) {
-        if (!f.periodic) return;
-        d[0] = fma(-f.box[0], rint(d[0] * f.ibox[0]), d[0]);
-        d[1] = fma(-f.box[1], rint(d[1] * f.ibox[1]), d[1]);
-        d[2] = fma(-f.box[2], rint(d[2] * f.ibox[2]), d[2]);
-    };
-    double gx = 0.0, gy = 0.0, gz = 0.0, ee = 0.0;
-    auto pairs = [&](int m) {
-        const bool on = lane < m;
-        const int l = on ? lane : 0, code = s.queue[wave][l];
-        const int j = code & 0xFFFFF, pe = ei + (code >> 20);
+    const int chunk = (n + kQSplit - 1) / kQSplit;
+    // of a step: eighth and place; of the sums: eighth and component (3: energy)
+    const int sp = lane >> 3, comp = lane & 7;
+    double *res = s.res[wave];
+    QAcc<T> acc;
+    int queued = 0, mine = 0;                      // in the wave's queues, and in this lane's eighth
+    auto pairs = [&]() {
+        // a lane per queued atom, one eighth after the other
+        int start = 0, from = 0, q = 0, first = 0;
+#pragma unroll
+        for (int k = 1; k < kQSplit; ++k) {
+            start += __builtin_amdgcn_readlane(mine, 8 * (k - 1));
+            first = sp >= k ? start : first;       // of this lane's eighth
+            q = lane >= start ? k : q;             // the eighth of this lane's atom
+            from = lane >= start ? start : from;
+        }
+        const bool on = lane < queued;
+        const int j = on ? q * chunk + s.queue[wave][q][lane - from] : 0;
         double dd[3] = { xi0 - x[3 * j], xi1 - x[3 * j + 1], xi2 - x[3 * j + 2] };
-        image(dd);
-        const T d0 = (T)dd[0], d1 = (T)dd[1], d2 = (T)dd[2];
-        const T r2 = (d0 * d0 + d1 * d1) + d2 * d2;
-        const T oner = qrsq(r2), r = r2 * oner, ir2 = oner * oner;
-        T e = (T)0, dr = (T)0;                     // gradient of i = d * dr
-        if (!(f.periodic && r > vdw)) {
-            const T R0 = (T)s.tab[0][pe], r06 = (T)s.tab[1][pe];
-            const T r4 = r2 * r2, r6 = r4 * r2;
-            const T t6 = r6 + r06, t8 = r6 * r2 + r06 * R0 * R0;
-            // beyond 1e5 bohr (no cutoff without periodicity) the terms are below 1e-25 hartree
-            const T c = r2 < (T)1e10 ? (T)c6[j] : (T)0;
-            const T ip = qrcp(r2 < (T)1e10 ? (sizeof(T) == 8 ? t6 * t8 : t8) : (T)1);
-            const T i6 = sizeof(T) == 8 ? t8 * ip : (T)1 / t6, i8 = sizeof(T) == 8 ? t6 * ip : ip;
-            const T c6t6 = c * i6;
-            T t27 = (T)s.tab[2][pe] * (c * i8);
-            e = -(c6t6 + t27);
-            dr = c6t6 * (T)6.0 * r4 * i6 + (T)8.0 * t27 * r6 * i8;
-            if (r < (T)25) {
-                const T alpha = (T)s.tab[4][pe];
-                t27 = (T)s.tab[3][pe] * exp(-alpha * r) * oner;
-                e = e + t27;
-                dr = dr - t27 * (alpha * r + (T)1.0) * ir2;
-            }
+        qimg(f, dd);
+        const T d[3] = { (T)dd[0], (T)dd[1], (T)dd[2] };
+        const T r2 = (d[0] * d[0] + d[1] * d[1]) + d[2] * d[2];
+        const T r = sqrt(r2);
+        T ga[3] = { (T)0, (T)0, (T)0 }, e = (T)0;
+        if (!(f.periodic && r > vdw))
+            qdisp_rep<T>({ s.tab[0], s.tab[1], s.tab[2], s.tab[3], s.tab[4] }, ei + f.elem[j], c6[j], d, r2, r, (T)1.0, e,
+                         ga);
+        T ec, gc[3];
+        if (qcoulomb<T>(f, qi, f.q[j], d, r2, r, (T)1.0, ec, gc)) {
+            e = qadd(e, ec);
+            for (int c = 0; c < 3; ++c) ga[c] = qadd(ga[c], gc[c]);
         }
-        if (!(r > coul)) {
-            const T qq = qi * (T)f.q[j];
-            T ec;
-            if (f.zahn) {
-                ec = qq * ((erfc((T)f.zahn_a * r) * oner) - (T)f.zahn_par * (r - coul));
-            } else {
-                T sw = (T)1.0;
-                if (f.periodic && r > (T)f.cut_low) {
-                    const T xv = (r - (T)f.cut_low) / (coul - (T)f.cut_low);
-                    sw = (T)exp(1.0) * exp((T)1.0 / (xv - (T)1.0));
-                }
-                ec = qq * oner * sw;
+        for (int c = 0; c < 3; ++c) res[67 * c + lane] = (double)ga[c];
+        res[67 * 3 + lane] = (double)e;
+        qwave_fence();
+        if (comp < 4)
+            for (int k = 0; k < mine; k += 4) {    // 4 reads at a time; only the additions wait
+                const double *v = res + 67 * comp + first + k;
+                double t[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) t[u] = v[u];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) acc.add(k + u < mine ? (T)t[u] : (T)0);    // + 0 changes neither sum
             }
-            e = e + ec;
-            dr = dr - ec * ir2;
-        }
-        gx += on ? (double)(d0 * dr) : 0.0;
-        gy += on ? (double)(d1 * dr) : 0.0;
-        gz += on ? (double)(d2 * dr) : 0.0;
-        ee += on ? (double)e : 0.0;
+        qwave_fence();
+        queued = mine = 0;
     };
-    int count = 0;
-    for (int t0 = 0; t0 < n; t0 += kQTile) {
+    for (int t0 = 0; t0 < chunk; t0 += kQTile / kQSplit) {
         __syncthreads();
-        const int jt = t0 + tid;
-        if (jt < n) {
+        const int jt = (tid >> 5) * chunk + t0 + (tid & 31);
+        if (t0 + (tid & 31) < chunk && jt < n) {
             for (int c = 0; c < 3; ++c) s.x[c][tid] = x[3 * jt + c];
             s.mol[tid] = f.mol[jt];
-            s.elem[tid] = f.elem[jt];
         }
         __syncthreads();
-        const int nt = min(kQTile, n - t0);
         if (!act) continue;                        // the whole wave
-        for (int u0 = 0; u0 < nt; u0 += 64) {
-            const int u = u0 + lane;
-            const int uu = u < nt ? u : 0;
-            bool in = u < nt && s.mol[uu] != mi;                  // not i's own molecule (nor i)
+        for (int u0 = 0; u0 < kQTile / kQSplit && t0 + u0 < chunk; u0 += 8) {
+            const int jj = t0 + u0 + comp, u = 32 * sp + u0 + comp;
+            const bool there = jj < chunk && sp * chunk + jj < n;
+            const int uu = there ? u : 0;
+            bool in = there && s.mol[uu] != mi;                   // not i's own molecule (nor i)
             double d[3] = { xi0 - s.x[0][uu], xi1 - s.x[1][uu], xi2 - s.x[2][uu] };
-            image(d);
+            if (f.periodic)                                       // a nearest image in one step; the pair has its own
+                for (int c = 0; c < 3; ++c) d[c] = fma(-f.box[c], rint(d[c] * f.ibox[c]), d[c]);
             in = in && !((d[0] * d[0] + d[1] * d[1]) + d[2] * d[2] > cut2);
             const unsigned long long m = __ballot(in);
-            if (in) s.queue[wave][count + __popcll(m & ((1ull << lane) - 1ull))] = (t0 + u) | s.elem[uu] << 20;
-            count += __popcll(m);
+            if (queued + __popcll(m) > 64) pairs();
+            const unsigned eighth = (unsigned)(m >> (8 * sp)) & 0xFFu;
+            if (in) s.queue[wave][sp][mine + __popc(eighth & ((1u << comp) - 1u))] = (unsigned short)jj;
+            mine += __popc(eighth);
+            queued += __popcll(m);
             qwave_fence();
-            const bool last = t0 + u0 + 64 >= n;
-            while (count >= 64 || (last && count > 0)) {
-                const int k = min(count, 64);
-                pairs(k);
-                count -= k;
-                const int rest = s.queue[wave][64 + lane];
-                qwave_fence();
-                if (lane < count) s.queue[wave][lane] = rest;
-            }
         }
     }
-    for (int o = 32; o > 0; o >>= 1) {
-        gx += __shfl_xor(gx, o);
-        gy += __shfl_xor(gy, o);
-        gz += __shfl_xor(gz, o);
-        ee += __shfl_xor(ee, o);
-    }
-    if (lane == 0) {
-        if (act) {
-            gpart[3 * i] = gx;
-            gpart[3 * i + 1] = gy;
-            gpart[3 * i + 2] = gz;
-        }
-        s.e[wave] = act ? 0.5 * ee : 0.0;          // every pair counted from both sides
-    }
+    if (queued > 0) pairs();
+    if (act && comp < 3) gpart[sp * stride + 3 * i + comp] = acc.get();
+    double ee = act && comp == 3 ? acc.get() : 0.0;
+    for (int o = 32; o > 0; o >>= 1) ee += __shfl_xor(ee, o);
+    if (lane == 0) s.e[wave] = 0.5 * ee;           // every pair counted from both sides
     __syncthreads();
     if (tid == 0) *epart = ((s.e[0] + s.e[1]) + s.e[2]) + s.e[3];
 }
@@ -777,17 +792,34 @@ __device__ void qslot(const QDev &f, const double *__restrict__ x, int blk, doub
 // A tenth of the pairs lies within the 15 bohr of the term, so a few lanes of
 // each 64 had a bond and the wave went through all of it for them, once per 64
 // partners.  Now those that count are queued and evaluated together, and the
-// blocks come first in the grid, as the waves with the longest chains: a force
-// call of 1125 atoms x 16 beads 130 -> 115 us.  Two or four acceptors to a wave
-// fill the evaluations better, but the longer chains cost more (122 and 138 us).
+// blocks come first in the grid, as the waves with the longest chains: 15 of
+// the 130 us of a force call of 1125 atoms x 16 beads.  Two or four acceptors
+// to a wave fill the evaluations better, but the longer chains cost more (7
+// and 23 us).
+//
+// The terms of a batch go to LDS, and the lane that the partner's number names
+// (mod 64) adds its own in their order: the sums of lanes that stride over the
+// partners, whatever the batches were (3 us of the call).
 template <bool DON>
 __device__ void qhb(const QDev &f, const double *__restrict__ x, int own, QTile &s, double *gout, double *eout)
 {
     const int lane = threadIdx.x & 63, n2 = DON ? f.nacc : f.ndon;
     if (own >= (DON ? f.ndon : f.nacc)) return;
-    int *queue = s.queue[threadIdx.x >> 6];
+    int *queue = reinterpret_cast<int *>(s.queue[threadIdx.x >> 6]);     // 63 + 64 at most
+    static_assert(sizeof s.queue[0] >= 128 * sizeof(int), "");
+    double *res = s.res[threadIdx.x >> 6];
     double sum[6] = { 0.0, 0.0, 0.0, 0.0, 0.0, 0.0 };
     int count = 0;
+    // sum[at..at + nv - 1] += v of the terms whose partner is this lane's, places `mine` of the batch
+    auto own_terms = [&](unsigned long long mine, int at, int nv, const double *v) {
+        for (int c = 0; c < nv; ++c) res[4 * lane + c] = v[c];
+        qwave_fence();
+        for (; mine; mine &= mine - 1) {
+            const double *r = res + 4 * __builtin_ctzll(mine);
+            for (int c = 0; c < nv; ++c) sum[at + c] = sum[at + c] + r[c];
+        }
+        qwave_fence();
+    };
     for (int o0 = 0; o0 < n2; o0 += 64) {
         const int o = o0 + lane;
         const bool in = o < n2 && qhbnear(f, x, DON ? own : o, DON ? o : own);
@@ -802,13 +834,16 @@ __device__ void qhb(const QDev &f, const double *__restrict__ x, int own, QTile 
             const int dn = DON ? own : other, A = f.don[2 * dn], H = f.don[2 * dn + 1];
             const int j = f.acc[DON ? other : own];
             double gj[3], ga[3], gh[3];
-            const double e = qeabhag(f, x, j, A, H, f.hbc[j], f.hbc[A], gj, ga, gh);
-            if (lane < k) {
-                for (int c = 0; c < 3; ++c) {
-                    sum[c] = sum[c] + (DON ? ga[c] : gj[c]);
-                    if (DON) sum[3 + c] = sum[3 + c] + gh[c];
-                }
-                if (!DON) sum[3] = sum[3] + e;
+            const double e = qeabhag<DON ? kHbDonor : kHbAcceptor>(f, x, j, A, H, f.hbc[j], f.hbc[A], gj, ga, gh);
+            unsigned long long mine = 0;
+            for (int t = 0; t < k; ++t)
+                mine |= (unsigned long long)((__builtin_amdgcn_readlane(other, t) & 63) == lane) << t;
+            if (DON) {
+                own_terms(mine, 0, 3, ga);
+                own_terms(mine, 3, 3, gh);
+            } else {
+                const double v[4] = { gj[0], gj[1], gj[2], e };
+                own_terms(mine, 0, 4, v);
             }
             count -= k;
             if (lane < count) queue[lane] = rest;
@@ -830,12 +865,11 @@ struct QBlocks {
     int ninter, nacc, ndon, nslot;
 };
 
-//
 // Built without machine-level loop-invariant code motion (see the Makefile):
 // with it the constants of exp and erfc were held in 128 registers across the
-// loops and others spilled inside them; without, 103 registers, and five waves
-// per SIMD cost 28 bytes of spills in the slots (FP64 call 151 us, 132 us at
-// four waves, 126 us at five, 134 us at six).
+// loops and others spilled inside them (151 us a call, 132 without).  Five
+// waves per SIMD, the most that the LDS allows, cost 52 bytes of spills in the
+// slots: an FP64 call of 1125 atoms x 16 beads takes 148 us, 161 at four.
 template <typename T>
 __global__ __launch_bounds__(kQTile) __attribute__((amdgpu_waves_per_eu(5))) void qm_terms_kernel(
     QDev f, QBlocks nb, const double *__restrict__ xall, double *gpart, double *epart, double *gacc, double *eacc,
@@ -860,13 +894,14 @@ __global__ __launch_bounds__(kQTile) __attribute__((amdgpu_waves_per_eu(5))) voi
         return;
     }
     k -= nb.nslot;
-    qinter<T>(f, x, k, s, gpart + (size_t)b * f.n * 3, epart + (size_t)b * nb.ninter + k);
+    qinter<T>(f, x, k, s, gpart + (size_t)b * f.n * 3, (size_t)gridDim.y * f.n * 3, epart + (size_t)b * nb.ninter + k);
 }
 
 // Four lanes per (bead, atom): its term slots and hydrogen-bond parts, every
-// fourth of the list to a lane (the loads of a list entry wait for its code, so
-// one lane's list was a chain of some twenty memory latencies: 16 us, now
-// 7.5), then the intermolecular sum; the acceptors' energies.
+// fourth of the list loaded by a lane (the loads of a list entry wait for its
+// code, so one lane's list was a chain of some twenty memory latencies: 16 us,
+// now 9.0) and added by all four in the list's order, then the eighths of
+// the intermolecular sum; the acceptors' energies.
 __global__ __launch_bounds__(256) void qm_gather_kernel(QDev f, const double *gslot, const double *gpart,
                                                         const double *gacc, const double *eacc, const double *gdon,
                                                         double *gout, double *egather)
@@ -876,29 +911,36 @@ __global__ __launch_bounds__(256) void qm_gather_kernel(QDev f, const double *gs
     const bool act = i < f.n;
     double g[3] = { 0.0, 0.0, 0.0 }, e = 0.0;
     if (act) {
-        for (int k = f.rptr[i] + sub; k < f.rptr[i + 1]; k += 4) {
-            const int code = f.rcode[k];
-            const int kind = code >> 28, payload = code & 0x0FFFFFFF;
-            const double *src;
-            if (kind == kTHbAcc) {
-                src = gacc + ((size_t)b * f.nacc + payload) * 3;
-                e = e + eacc[(size_t)b * f.nacc + payload];
-            } else if (kind == kTHbDon) {
-                const int role = payload >> 26, dn = payload & 0x03FFFFFF;
-                src = gdon + ((size_t)b * f.ndon + dn) * 6 + (role == 1 ? 0 : 3);
-            } else {
-                src = gslot + ((size_t)b * f.nslot + payload) * 3;
+        const int end = f.rptr[i + 1];
+        for (int k0 = f.rptr[i]; k0 < end; k0 += 4) {          // the same trips on all four lanes
+            double v[3] = { 0.0, 0.0, 0.0 };
+            if (k0 + sub < end) {
+                const int code = f.rcode[k0 + sub];
+                const int kind = code >> 28, payload = code & 0x0FFFFFFF;
+                const double *src;
+                if (kind == kTHbAcc) {
+                    src = gacc + ((size_t)b * f.nacc + payload) * 3;
+                    e = e + eacc[(size_t)b * f.nacc + payload];
+                } else if (kind == kTHbDon) {
+                    const int role = payload >> 26, dn = payload & 0x03FFFFFF;
+                    src = gdon + ((size_t)b * f.ndon + dn) * 6 + (role == 1 ? 0 : 3);
+                } else {
+                    src = gslot + ((size_t)b * f.nslot + payload) * 3;
+                }
+                for (int c = 0; c < 3; ++c) v[c] = src[c];
             }
-            g[0] = g[0] + src[0];
-            g[1] = g[1] + src[1];
-            g[2] = g[2] + src[2];
+            for (int c = 0; c < 3; ++c)                        // past the end: + 0
+                g[c] = (((g[c] + quad::bcast<0>(v[c])) + quad::bcast<1>(v[c])) + quad::bcast<2>(v[c])) +
+                       quad::bcast<3>(v[c]);
         }
-    }
-    for (int c = 0; c < 3; ++c) g[c] = quad::sum(g[c]);
-    if (act && gout && sub < 3) {
-        const size_t o = ((size_t)b * f.n + i) * 3 + sub;
-        const double own = sub == 0 ? g[0] : sub == 1 ? g[1] : g[2];
-        gout[o] = f.inter ? own + gpart[o] : own;
+        if (gout && sub < 3) {
+            double own = sub == 0 ? g[0] : sub == 1 ? g[1] : g[2];
+            const size_t o = ((size_t)b * f.n + i) * 3 + sub, stride = (size_t)gridDim.y * f.n * 3;
+            if (f.inter)
+#pragma unroll
+                for (int s = 0; s < kQSplit; ++s) own = own + gpart[s * stride + o];
+            gout[o] = own;
+        }
     }
     for (int o = 32; o > 0; o >>= 1) e = e + __shfl_xor(e, o);
     if ((threadIdx.x & 63) == 0) sred[threadIdx.x >> 6] = e;
@@ -1132,7 +1174,7 @@ int qmdff_ensure(QmdffDev *q, int nbeads)
     const QDev &d = q->d;
     const int nbx = (d.n + kQWaves - 1) / kQWaves;
     const int ngx = (d.n + 63) / 64;
-    CAM_HIP(hipMalloc(&q->gpart, (size_t)nbeads * d.n * 3 * sizeof(double)));
+    CAM_HIP(hipMalloc(&q->gpart, (size_t)kQSplit * nbeads * d.n * 3 * sizeof(double)));
     CAM_HIP(hipMalloc(&q->epart, (size_t)nbeads * (nbx + ngx) * sizeof(double)));
     CAM_HIP(hipMalloc(&q->gacc, ((size_t)std::max(1, d.nacc) * nbeads * 4) * sizeof(double)));
     CAM_HIP(hipMalloc(&q->eacc, ((size_t)std::max(1, d.nacc) * nbeads) * sizeof(double)));

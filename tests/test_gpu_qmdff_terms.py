@@ -1,17 +1,16 @@
 """The QMDFF terms kernel at the edges of its split: one wave per atom, four
-atoms to a block, 64 candidate atoms at a time from tiles of 256, accepted ones
-queued and evaluated 64 at a time.
+atoms to a block, 64 candidate atoms at a time (eight of each eighth of the
+atoms) from tiles of 256, accepted ones queued and evaluated 64 at a time.
 
 Subsets of the ethanol box (9 atoms a molecule) around those sizes, with no,
 some and every pair inside the cutoff, molecules displaced by whole boxes, both
 electrostatics, one and several beads, FP64 and mixed, against the oracle.
 
 Tolerances: an energy or gradient component is a sum of at most n terms whose
-own relative error is below 1e-13 in FP64 (two Newton steps on the reciprocals,
-2 ulp exp and erfc) and 1e-6 in binary32 (1 ulp reciprocal and root of a
-squared distance, times the exponent 8); terms of opposite sign cancel to no
-less than a hundredth of their size in these liquids, so 1e-11 and 1e-4 of the
-largest component."""
+own relative error is below 1e-13 in FP64 (2 ulp exp and erfc) and 1e-6 in
+binary32 (1 ulp quotient and root of a squared distance, times the exponent
+8); terms of opposite sign cancel to no less than a hundredth of their size in
+these liquids, so 1e-11 and 1e-4 of the largest component."""
 import numpy as np
 import pytest
 import torch
@@ -43,7 +42,7 @@ def _subset(nmol):
     (1, 1, 0, 1.0, 1),        # no other molecule: no intermolecular block
     (2, 1, 0, 1.0, 1),        # 18 atoms: one partly filled group of 64
     (2, 0, 0, 1.0, 3),
-    (7, 1, 0, 1.0, 2),        # 63, 64 + 8 atoms: either side of a group
+    (7, 1, 0, 1.0, 2),        # 63 and 72 atoms: either side of a group
     (8, 0, 1, 1.0, 2),
     (28, 1, 1, 1.0, 1),       # 252 and 261: either side of a tile
     (29, 1, 0, 1.0, 5),
