@@ -27,7 +27,6 @@
 #include "nhc.hpp"
 #include "philox.hpp"
 #include "qmdff.hpp"
-#include "transrot.hpp"
 
 namespace cam {
 namespace {
@@ -1579,6 +1578,13 @@ struct BoxNM {
     double box[3];
 };
 
+// a b rounded, never fused with an addition that follows.
+__device__ __forceinline__ double mul_rn(double a, double b)
+{
+#pragma clang fp contract(off)
+    return a * b;
+}
+
 // One block: 256/nb columns (atom, dim) x nb beads.
 //
 // The wrap (src/verlet.f90:540-640): a coordinate that left [0, L] in some
@@ -1603,7 +1609,7 @@ __global__ __launch_bounds__(256) void box_nm_kernel(BoxNM a)
     double p = 0.0, q = 0.0;
     if (act) {
         p = a.p[o];
-        if (a.scale) p = *a.scale * p;
+        if (a.scale) p = mul_rn(*a.scale, p);
         p = p - 0.5 * a.dt * a.g[o];
         q = a.q[o];
     }
@@ -1669,15 +1675,32 @@ __global__ __launch_bounds__(256) void box_nm_kernel(BoxNM a)
     }
 }
 
-// Kinetic energy sum p^2/(2m) of the lanes of a block (256), for the chain:
-// one partial per block, sums in a fixed order.
+// Blocks of the kernels that sum the kinetic energy for the chain, each over
+// the elements (bead, atom, coordinate) i = block 256 + lane + k 65536: one
+// partition in all of them, so that a trajectory does not depend on where a
+// run ends and the next begins.
+constexpr int kBoxParts = 256;
+
+// v of the 256 lanes of a block summed as a halving tree (lane t adds lane
+// t + 128, then t + 64, ...), in lane 0 of the calling wave; sh: 256 doubles
+// that all lanes have written.
+__device__ __forceinline__ double block_tree(const double *sh)
+{
+    const int lane = threadIdx.x & 63;
+    double v = (sh[lane] + sh[lane + 128]) + (sh[lane + 64] + sh[lane + 192]);
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+    return v;
+}
+
+// Kinetic energy sum p^2/(2m) of the lanes of a block, one partial per block.
 __device__ void box_ke_part(double acc, double *part)
 {
-    __shared__ double red[4];
-    for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
+    __shared__ double red[256];
+    red[threadIdx.x] = acc;
     __syncthreads();
-    if (threadIdx.x == 0) part[blockIdx.x] = ((red[0] + red[1]) + red[2]) + red[3];
+    if (threadIdx.x >= 64) return;
+    acc = block_tree(red);
+    if (threadIdx.x == 0) part[blockIdx.x] = acc;
 }
 
 // Second half kick and the Andersen draws; with a chain (part not NULL) also
@@ -1747,8 +1770,6 @@ __global__ void box_energy_kernel(const double *q, const double *p, const double
 // (the kick, transrot, the scaling) and the factor is applied where they are
 // read next (the normal-mode step, transrot): of the three kernels per chain
 // only the chain is left, and box_ke_kernel before the first step of a launch.
-constexpr int kBoxParts = 1024;         // partial sums at most: blocks of a summing kernel
-
 __global__ __launch_bounds__(256) void box_ke_kernel(const double *p, const double *mass, int natoms, int nb,
                                                      double *part)
 {
@@ -1795,63 +1816,130 @@ __global__ __launch_bounds__(256) void box_scale_kernel(double *p, const double 
     box_ke_part(acc, part);
 }
 
-// transrot for one box (transrot.hpp; total mass of nbeads^2 * M): two passes
-// of fixed-order block sums over every (bead, atom), then the velocity update.
+// transrot for one box (src/transrot.f90:36-237, with its total mass of
+// nbeads^2 * M): two passes of fixed-order block sums over every (bead, atom)
+// -- mass-weighted velocities and positions, then, about the centre they give,
+// the angular momentum and the inertia tensor -- and the velocity update.  The
+// reference's divisions and products by the masses stay: left out they change
+// a rounding, which the box's terms can amplify (qmdff.hip).
 // Each block of the second and third kernel sums the parts of the one before
 // and, in the third, solves for the angular velocity itself (a few hundred
 // flops), which costs less than a kernel of one block that does it between
 // them: pass1, pass2, solve and apply took 4.7 + 9.1 + 7.7 + 4.7 us for 1125
-// atoms x 16 beads, the three 5.0 + 4.7 + 5.3 us with the Nose-Hoover factor and kinetic
+// atoms x 16 beads, the three 5.2 + 5.0 + 7.9 us with the Nose-Hoover factor and kinetic
 // energy in them.
-constexpr int kTrBlocks = 64;           // one wave's lanes sum the parts
-constexpr int kTrApplyBlocks = 512;     // at most, for the solution each block repeats
+constexpr int kTrBlocks = 64;
 
-// v: this lane's NV partial sums -> out[NV] for the block, a fixed order
+// v: this lane's NV partial sums -> out[NV] for the block, a fixed order; sh: NV * 256
 template <int NV>
-__device__ __forceinline__ void tr_block_sum(double *v, double *sh, double *out)
+__device__ __forceinline__ void tr_block_sum(const double *v, double *sh, double *out)
 {
 #pragma unroll
-    for (int c = 0; c < NV; ++c)
-        for (int o = 32; o > 0; o >>= 1) v[c] += __shfl_xor(v[c], o);
-    if ((threadIdx.x & 63) == 0)
-#pragma unroll
-        for (int c = 0; c < NV; ++c) sh[(threadIdx.x >> 6) * NV + c] = v[c];
+    for (int c = 0; c < NV; ++c) sh[c * 256 + threadIdx.x] = v[c];
     __syncthreads();
-    if (threadIdx.x < NV) {
-        const double *r = sh + threadIdx.x;
-        out[threadIdx.x] = ((r[0] + r[NV]) + r[2 * NV]) + r[3 * NV];
+    for (int c = threadIdx.x >> 6; c < NV; c += 4) {
+        const double t = block_tree(sh + c * 256);
+        if ((threadIdx.x & 63) == 0) out[c] = t;
     }
 }
 
-// the kTrBlocks parts of NV sums -> sh[NV] in every lane's view
+// the kTrBlocks parts of NV sums, added one after the other -> sum[NV]; sh: NV * kTrBlocks
 template <int NV>
-__device__ __forceinline__ void tr_parts(const double *part, double *sh)
+__device__ __forceinline__ void tr_parts(const double *part, double *sh, double *sum)
 {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for (int c = wave; c < NV; c += 4) {
-        double v = part[NV * lane + c];
-        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-        if (lane == 0) sh[c] = v;
+    for (int i = threadIdx.x; i < NV * kTrBlocks; i += 256) sh[i] = part[i];
+    __syncthreads();
+    if (threadIdx.x < NV) {
+        double t = 0.0;
+#pragma unroll 8
+        for (int b = 0; b < kTrBlocks; ++b) t = t + sh[NV * b + threadIdx.x];
+        sum[threadIdx.x] = t;
     }
     __syncthreads();
+}
+
+// Angular velocity from the sums s (angular momentum, inertia tensor), the
+// total velocity vt and the centre x.
+__device__ void tr_solve(const double *s, const double *vt, const double *x, int natoms, double totmass, double *omega)
+{
+    const double xt = x[0], yt = x[1], zt = x[2];
+    double mang[3];
+    mang[0] = s[0] - (yt * vt[2] - zt * vt[1]) * totmass;
+    mang[1] = s[1] - (zt * vt[0] - xt * vt[2]) * totmass;
+    mang[2] = s[2] - (xt * vt[1] - yt * vt[0]) * totmass;
+    const double xx = s[3], xy = s[4], xz = s[5], yy = s[6], yz = s[7], zz = s[8];
+    double ten[3][3];
+    ten[0][0] = yy + zz; ten[0][1] = -xy;    ten[0][2] = -xz;
+    ten[1][0] = -xy;     ten[1][1] = xx + zz; ten[1][2] = -yz;
+    ten[2][0] = -xz;     ten[2][1] = -yz;    ten[2][2] = xx + yy;
+    if (natoms <= 2) {
+        ten[0][0] += 0.000001;
+        ten[1][1] += 0.000001;
+        ten[2][2] += 0.000001;
+    }
+    // Gauss-Jordan inversion with full pivoting (src/invert.f90)
+    int ipiv[3] = { 0, 0, 0 }, indxr[3], indxc[3];
+    for (int i = 0; i < 3; ++i) {
+        double big = 0.0;
+        int irow = 0, icol = 0;
+        for (int j = 0; j < 3; ++j)
+            if (ipiv[j] != 1)
+                for (int kk = 0; kk < 3; ++kk)
+                    if (ipiv[kk] == 0 && fabs(ten[j][kk]) >= big) {
+                        big = fabs(ten[j][kk]);
+                        irow = j;
+                        icol = kk;
+                    }
+        ipiv[icol] += 1;
+        if (irow != icol)
+            for (int j = 0; j < 3; ++j) {
+                const double tmp = ten[irow][j];
+                ten[irow][j] = ten[icol][j];
+                ten[icol][j] = tmp;
+            }
+        indxr[i] = irow;
+        indxc[i] = icol;
+        const double piv = ten[icol][icol];
+        ten[icol][icol] = 1.0;
+        for (int j = 0; j < 3; ++j) ten[icol][j] = ten[icol][j] / piv;
+        for (int j = 0; j < 3; ++j)
+            if (j != icol) {
+                const double tmp = ten[j][icol];
+                ten[j][icol] = 0.0;
+                for (int kk = 0; kk < 3; ++kk) ten[j][kk] = ten[j][kk] - ten[icol][kk] * tmp;
+            }
+    }
+    for (int i = 2; i >= 0; --i)
+        if (indxr[i] != indxc[i])
+            for (int kk = 0; kk < 3; ++kk) {
+                const double tmp = ten[kk][indxr[i]];
+                ten[kk][indxr[i]] = ten[kk][indxc[i]];
+                ten[kk][indxc[i]] = tmp;
+            }
+    for (int i = 0; i < 3; ++i) {
+        double v = 0.0;
+        for (int j = 0; j < 3; ++j) v = v + ten[i][j] * mang[j];
+        omega[i] = v;
+    }
 }
 
 __global__ __launch_bounds__(256) void box_tr_pass1(const double *q, double *p, const double *mass, int natoms, int nb,
                                                     const double *scale, double *part)
 {
-    __shared__ double sh[4 * 6];
+    __shared__ double sh[6 * 256];
     double v[6] = { 0, 0, 0, 0, 0, 0 };
     const size_t n = (size_t)natoms * nb;
     for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (size_t)kTrBlocks * 256) {
-        double *pe = p + 3 * e;
-        double w[3] = { pe[0], pe[1], pe[2] };
-        if (scale) {
-            for (int c = 0; c < 3; ++c) {
-                w[c] = *scale * w[c];
-                pe[c] = w[c];
+        const double w = mass[e % natoms];
+        for (int c = 0; c < 3; ++c) {
+            double pc = p[3 * e + c];
+            if (scale) {
+                pc = *scale * pc;
+                p[3 * e + c] = pc;
             }
+            v[c] = v[c] + (pc / w) * w;
+            v[3 + c] = v[3 + c] + q[3 * e + c] * w;
         }
-        transrot_sums1(q + 3 * e, w, mass[e % natoms], v);
     }
     tr_block_sum<6>(v, sh, part + 6 * blockIdx.x);
 }
@@ -1859,47 +1947,56 @@ __global__ __launch_bounds__(256) void box_tr_pass1(const double *q, double *p, 
 __global__ __launch_bounds__(256) void box_tr_pass2(const double *q, const double *p, const double *mass, int natoms,
                                                     int nb, const double *part1, double totmass, double *part)
 {
-    __shared__ double sh[4 * 9], s1[6];
-    tr_parts<6>(part1, s1);
-    const double xt[3] = { s1[3] / totmass, s1[4] / totmass, s1[5] / totmass };
+    __shared__ double sh[9 * 256], s1[6];
+    tr_parts<6>(part1, sh, s1);
+    const double xt = s1[3] / totmass, yt = s1[4] / totmass, zt = s1[5] / totmass;
     double v[9] = { 0, 0, 0, 0, 0, 0, 0, 0, 0 };
     const size_t n = (size_t)natoms * nb;
-    for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (size_t)kTrBlocks * 256)
-        transrot_sums2(q + 3 * e, p + 3 * e, mass[e % natoms], xt, v);
+    for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (size_t)kTrBlocks * 256) {
+        const double w = mass[e % natoms];
+        const double *x = q + 3 * e;
+        const double vx = p[3 * e] / w, vy = p[3 * e + 1] / w, vz = p[3 * e + 2] / w;
+        v[0] = v[0] + (x[1] * vz - x[2] * vy) * w;
+        v[1] = v[1] + (x[2] * vx - x[0] * vz) * w;
+        v[2] = v[2] + (x[0] * vy - x[1] * vx) * w;
+        const double xd = x[0] - xt, yd = x[1] - yt, zd = x[2] - zt;
+        v[3] = v[3] + xd * xd * w;
+        v[4] = v[4] + xd * yd * w;
+        v[5] = v[5] + xd * zd * w;
+        v[6] = v[6] + yd * yd * w;
+        v[7] = v[7] + yd * zd * w;
+        v[8] = v[8] + zd * zd * w;
+    }
     tr_block_sum<9>(v, sh, part + 9 * blockIdx.x);
 }
 
+// A lane per element, the partition of the kinetic energy that follows.
 __global__ __launch_bounds__(256) void box_tr_apply(const double *q, double *p, const double *mass, int natoms, int nb,
                                                     const double *part1, const double *part2, double totmass,
                                                     double *kepart)
 {
-    __shared__ double s1[6], s2[9];
-    tr_parts<6>(part1, s1);
-    tr_parts<9>(part2, s2);
-    double vtot[3], xt[3], omega[3], sums[9];
-    for (int c = 0; c < 3; ++c) {
-        vtot[c] = s1[c] / totmass;
-        xt[c] = s1[3 + c] / totmass;
+    __shared__ double sh[9 * kTrBlocks], s1[6], s2[9], vc[6], om[3];
+    tr_parts<6>(part1, sh, s1);
+    tr_parts<9>(part2, sh, s2);
+    if (threadIdx.x == 0) {
+        for (int c = 0; c < 6; ++c) vc[c] = s1[c] / totmass;
+        double omega[3];
+        tr_solve(s2, vc, vc + 3, natoms, totmass, omega);
+        for (int c = 0; c < 3; ++c) om[c] = omega[c];
     }
-    for (int c = 0; c < 9; ++c) sums[c] = s2[c];
-    if (natoms <= 2) {                    // 1e-6 on the diagonal (src/transrot.f90:176-180)
-        const double d = 0.5 * 0.000001;  // each diagonal element is a sum of two of these
-        sums[3] += d;
-        sums[6] += d;
-        sums[8] += d;
-    }
-    transrot_omega(vtot, xt, sums, totmass, omega);
-    const size_t n = (size_t)natoms * nb;
+    __syncthreads();
+    const size_t n = (size_t)3 * natoms * nb;
     double acc = 0.0;
-    for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (size_t)gridDim.x * 256) {
-        double *pe = p + 3 * e;
-        double w[3] = { pe[0], pe[1], pe[2] };
-        const double m = mass[e % natoms];
-        transrot_apply(q + 3 * e, w, m, vtot, xt, omega);
-        for (int c = 0; c < 3; ++c) {
-            pe[c] = w[c];
-            acc += w[c] * w[c] / (2.0 * m);
-        }
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
+        const size_t e = i / 3;
+        const int j = (int)(i % 3), j1 = j == 2 ? 0 : j + 1, j2 = j == 0 ? 2 : j - 1;
+        const double w = mass[e % natoms];
+        double v = p[i] / w - vc[j];
+        const double d2 = q[3 * e + j2] - vc[3 + j2], d1 = q[3 * e + j1] - vc[3 + j1];
+        v = v - om[j1] * d2 + om[j2] * d1;
+        v = v * w;
+        p[i] = v;
+        acc += v * v / (2.0 * w);
     }
     if (kepart) box_ke_part(acc, kepart);
 }
@@ -1919,7 +2016,7 @@ struct cam_box {
     uint64_t *step_base = nullptr;
     double nose_q = 0.0;               // Nose-Hoover chain on when > 0
     double *nhc = nullptr;             // chain state: 4 velocities and the last scale factor
-    double *nhc_part = nullptr;        // kinetic-energy parts (kBoxParts)
+    double *nhc_part = nullptr;        // kinetic-energy parts
     bool transrot = false;             // remove centre-of-mass motion after every step (dynamic.x)
     double totmass = 0.0;              // transrot's nbeads^2 * M
     double *tr = nullptr;              // transrot: partial sums
@@ -1947,24 +2044,20 @@ int box_enqueue(cam_box *bx, int nsteps)
     std::memcpy(th.p, bx->theta, sizeof th.p);
     const size_t n = (size_t)ncol * bx->nb;
     const unsigned egrid = (unsigned)((n + 255) / 256);
-    // blocks of the kernels that leave one partial sum each
-    const unsigned pgrid = std::min<unsigned>(egrid, kBoxParts);
-    const unsigned agrid = std::min<unsigned>((unsigned)(((size_t)bx->natoms * bx->nb + 255) / 256), kTrApplyBlocks);
-    auto chain = [&](unsigned nparts) -> int {         // src/verlet.f90:185-206, :1086-1106
+    auto chain = [&]() -> int {                        // src/verlet.f90:185-206, :1086-1106
         if (!nose) return CAM_OK;
-        hipLaunchKernelGGL(box_nhc_kernel, dim3(1), dim3(64), 0, bx->stream, bx->nhc_part, (int)nparts, bx->nhc,
+        hipLaunchKernelGGL(box_nhc_kernel, dim3(1), dim3(64), 0, bx->stream, bx->nhc_part, kBoxParts, bx->nhc,
                            bx->beta, bx->nose_q, bx->natoms, bx->nb, bx->dt);
         CAM_LAUNCH_CHECK();
         return CAM_OK;
     };
     if (nose && nsteps > 0) {
-        hipLaunchKernelGGL(box_ke_kernel, dim3(pgrid), dim3(256), 0, bx->stream, bx->p, bx->mass, bx->natoms, bx->nb,
+        hipLaunchKernelGGL(box_ke_kernel, dim3(kBoxParts), dim3(256), 0, bx->stream, bx->p, bx->mass, bx->natoms, bx->nb,
                            bx->nhc_part);
         CAM_LAUNCH_CHECK();
     }
-    unsigned parts = pgrid;                            // of the kinetic energy the last kernel left
     for (int s = 0; s < nsteps; ++s) {
-        int rc0 = chain(parts);
+        int rc0 = chain();
         if (rc0 != CAM_OK) return rc0;
         hipLaunchKernelGGL(box_nm_kernel, dim3((ncol + cpb - 1) / cpb), dim3(256), 2 * 256 * sizeof(double), bx->stream,
                            a);
@@ -1973,11 +2066,11 @@ int box_enqueue(cam_box *bx, int nsteps)
                      ? ff_launch<float>(bx->ff, th, bx->q, bx->nb, bx->e, bx->g, nullptr, nullptr, nullptr, bx->stream)
                      : ff_launch<double>(bx->ff, th, bx->q, bx->nb, bx->e, bx->g, nullptr, nullptr, nullptr, bx->stream);
         if (rc != CAM_OK) return rc;
-        hipLaunchKernelGGL(box_kick_kernel, dim3(nose ? pgrid : egrid), dim3(256), 0, bx->stream, bx->p, bx->g,
+        hipLaunchKernelGGL(box_kick_kernel, dim3(nose ? kBoxParts : egrid), dim3(256), 0, bx->stream, bx->p, bx->g,
                            bx->mass, bx->natoms, bx->nb, bx->dt, bx->beta, bx->andersen_step, bx->seed, bx->step_base, s,
                            nose ? bx->nhc_part : nullptr);
         CAM_LAUNCH_CHECK();
-        rc = chain(pgrid);
+        rc = chain();
         if (rc != CAM_OK) return rc;
         if (bx->transrot) {                             // src/verlet.f90:1299-1305
             double *part1 = bx->tr, *part2 = part1 + 6 * kTrBlocks;
@@ -1987,15 +2080,13 @@ int box_enqueue(cam_box *bx, int nsteps)
             hipLaunchKernelGGL(box_tr_pass2, dim3(kTrBlocks), dim3(256), 0, bx->stream, bx->q, bx->p, bx->mass,
                                bx->natoms, bx->nb, part1, bx->totmass, part2);
             CAM_LAUNCH_CHECK();
-            hipLaunchKernelGGL(box_tr_apply, dim3(agrid), dim3(256), 0, bx->stream, bx->q, bx->p, bx->mass, bx->natoms,
+            hipLaunchKernelGGL(box_tr_apply, dim3(kBoxParts), dim3(256), 0, bx->stream, bx->q, bx->p, bx->mass, bx->natoms,
                                bx->nb, part1, part2, bx->totmass, nose ? bx->nhc_part : nullptr);
             CAM_LAUNCH_CHECK();
-            parts = agrid;
         } else if (nose) {
-            hipLaunchKernelGGL(box_scale_kernel, dim3(pgrid), dim3(256), 0, bx->stream, bx->p, bx->mass, bx->natoms,
+            hipLaunchKernelGGL(box_scale_kernel, dim3(kBoxParts), dim3(256), 0, bx->stream, bx->p, bx->mass, bx->natoms,
                                bx->nb, a.scale, bx->nhc_part);
             CAM_LAUNCH_CHECK();
-            parts = pgrid;
         }
     }
     hipLaunchKernelGGL(box_advance_kernel, dim3(1), dim3(1), 0, bx->stream, bx->step_base, nsteps);

@@ -52,20 +52,20 @@ def forces(p, xs, precision):
     return g
 
 
-def trajectory(nose, transrot, cuts, precision=cam.CAM_PREC_FP64):
-    """q and p after runs of the given lengths of a 16-molecule box."""
-    p, x = _subset(NMOL)
+def trajectory(nose, transrot, cuts, precision=cam.CAM_PREC_FP64, nmol=NMOL, nbeads=NBEADS, nose_steps=20):
+    """q and p after runs of the given lengths of a box."""
+    p, x = _subset(nmol)
     rng = np.random.default_rng(5)
-    xs = x[None] + rng.normal(0.0, 0.02, (NBEADS,) + x.shape)
+    xs = x[None] + rng.normal(0.0, 0.02, (nbeads,) + x.shape)
     m = mass_au([MASS[int(z)] for z in p["at"]])
     beta, dt = float(cam.beta_of(200.0)), 0.5 * cam.FS_TO_AU
     ff = cff.ForceField.qmdff(p)
-    eng = cff.BoxEngine(ff, NBEADS, dt, m, beta, None, precision=precision)
+    eng = cff.BoxEngine(ff, nbeads, dt, m, beta, None, precision=precision)
     if nose:
-        eng.set_nhc(20 * dt)
+        eng.set_nhc(nose_steps * dt)
     if transrot:
         eng.set_transrot(True)
-    eng.set_state(xs, rng.normal(size=xs.shape) * np.sqrt(m[None, :, None] * NBEADS / beta))
+    eng.set_state(xs, rng.normal(size=xs.shape) * np.sqrt(m[None, :, None] * nbeads / beta))
     for n in cuts:
         eng.run(n)
     q, pm = eng.get_state()
