@@ -57,12 +57,17 @@ __device__ inline void vhx(double rdif, double ex1, double ex2, double v[4], dou
 // packed lower triangle, row-wise (0-based)
 __host__ __device__ constexpr int pk(int i, int j) { return i >= j ? i * (i + 1) / 2 + j : j * (j + 1) / 2 + i; }
 
-// Tangent and cosine of the Jacobi rotation that clears apq.
+// Tangent and cosine of the Jacobi rotation that clears apq.  Beyond some 33
+// bohr between all three atoms every element is below 1e-150; d and b are
+// brought up together there, or their squares would vanish (a NaN angle).
 __device__ inline void rotation(double app, double aqq, double apq, double &t, double &c)
 {
-    const double d = aqq - app, b = 2.0 * apq;
+    double d = aqq - app, b = 2.0 * apq;
+    const double up = fmax(fabs(d), fabs(b)) < 0x1p-400 ? 0x1p600 : 1.0;
+    d *= up;
+    b *= up;
     const double h = fabs(d) + sqrt(d * d + b * b);
-    t = apq == 0.0 ? 0.0 : (d < 0.0 ? -b : b) / h;
+    t = b == 0.0 ? 0.0 : (d < 0.0 ? -b : b) / h;
     c = rsqrt(t * t + 1.0);
 }
 

@@ -14,7 +14,7 @@ import torch
 import caracal_amd as cam
 import oracle_lib as ol
 from caracal_amd import workloads
-from test_oracle_brh2 import _cloud, _special
+from test_oracle_brh2 import _cloud, _separated, _special
 
 pytestmark = pytest.mark.gpu
 
@@ -38,6 +38,34 @@ def test_brh2_forces_match_oracle():
     with pytest.raises(cam.CamError, match="FP64 only"):
         cam.egrad_dev(cam.CAM_SURFACE_BRH2, qd.data_ptr(), len(q), vd.data_ptr(), gd.data_ptr(),
                       precision=cam.CAM_PREC_MIXED)
+
+
+def test_brh2_separated_atoms_match_oracle():
+    """Three free atoms: no NaN, and nothing but the zero of energy is left."""
+    q = _separated()
+    v, g = cam.egrad_brh2(q)
+    vr, gr = ol.egrad_brh2(q)
+    print(f"{len(q)} separated triples: {np.isnan(v).sum()} NaN, max |dV| {np.nanmax(np.abs(v - vr)):.1e}, "
+          f"max |dg| {np.nanmax(np.abs(g - gr)):.1e}, largest |g| {np.abs(gr).max():.1e}")
+    assert np.isfinite(v).all() and np.isfinite(g).all()
+    assert np.abs(v - vr).max() <= 1e-13 and np.abs(g - gr).max() <= 1e-13
+
+
+@pytest.mark.parametrize("ntraj", [300, 3200], ids=["four-lanes", "one-lane"])
+def test_brh2_separated_atoms_in_the_engine(ntraj):
+    """The step kernels on both sides of the line between four lanes per bead
+    and one (256 blocks of 12 folded 8-bead polymers): free atoms at rest stay."""
+    w, nb = workloads.brh2_nve(nbeads=8), 8
+    q = _separated()
+    q = q[np.random.default_rng(1).permutation(len(q))[:ntraj]]
+    q = np.repeat(q[:, None], nb, axis=1)
+    e = cam.RPMDEngine(cam.CAM_SURFACE_BRH2, nb, ntraj, w["dt"], w["masses"])
+    e.set_state(q, np.zeros_like(q), np.full(ntraj, w["beta"]))
+    e.run(3)
+    q1, p1 = e.get_state()
+    e.close()
+    # forces of 1e-10 hartree/bohr for three steps; the transform rounds at 60 bohr
+    assert np.abs(q1 - q).max() <= 1e-12 and np.abs(p1).max() <= 1e-6
 
 
 @pytest.mark.parametrize("nb,nmk", [(1, cam.CAM_NMK_AUTO), (6, cam.CAM_NMK_AUTO), (16, cam.CAM_NMK_VALU),

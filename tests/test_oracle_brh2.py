@@ -55,6 +55,27 @@ def _special():
     return np.array(out)
 
 
+def _separated():
+    """Three free atoms: every element of the DIM matrix is below 1e-100, its
+    squares below the smallest number.  Right angles with equal Br-H distances
+    (equal diagonal elements) and random triples, 27 to 60 bohr apart."""
+    r = np.arange(30.0, 60.0, 0.01)
+    o = np.zeros_like(r)
+    right = np.stack([np.stack([-r, o, o], 1), np.stack([o, o, o], 1), np.stack([o, r, o], 1)], 1)
+    x = np.random.default_rng(4).uniform(-45.0, 45.0, (60000, 3, 3))
+    d = np.stack([np.linalg.norm(x[:, i] - x[:, j], axis=1) for i, j in ((0, 1), (0, 2), (1, 2))])
+    x = x[(d.min(0) > 27.0) & (d.max(0) < 60.0)]
+    # one triple that the squares alone made NaN, around it
+    near = np.array([[33.8751, 0, 0], [0, 0, 0], [24.8421, 26.2322, 0]])[None] * np.linspace(0.97, 0.985, 300)[:, None, None]
+    return np.concatenate([right, x, near])
+
+
+def test_separated_atoms_are_free():
+    v, g = ol.egrad_brh2(_separated())
+    assert np.abs(v - DHH).max() <= 1e-10        # the reference's zero is H2 + Br
+    assert np.abs(g).max() <= 1e-10
+
+
 @needs_ref
 @pytest.mark.parametrize("q", [_cloud(400, 0.15, 0), _cloud(300, 0.5, 1), _cloud(300, 1.0, 2), _special()],
                          ids=["near-saddle", "wide", "wider", "special"])
