@@ -867,8 +867,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE))) v
             // penalty.
             if constexpr (NB == 1) __syncthreads();
             const int gi = tid % XG::GL;
+            // slots past the last trajectory too: they hold a copy of it
             for (int t = tid / XG::GL; t < TPB; t += NG) {
-                if ((int)blockIdx.x * TPB + t >= a.ntraj) break;
                 auto &w = xw[tid / XG::GL];
                 const bool on = gi < NC;
                 const double c = on ? cent[t * NC + gi] : 0.0, dprev = on ? pdir[t * NC + gi] : 0.0;
@@ -946,8 +946,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE))) v
             {
                 const int gi = tid % XG::GL;
                 for (int t = tid / XG::GL; t < TPB; t += NG) {
-                    const int tr = blockIdx.x * TPB + t;
-                    if (tr >= a.ntraj) break;
+                    const int tr = min((int)blockIdx.x * TPB + t, a.ntraj - 1);
                     auto &w = xw[tid / XG::GL];
                     if (gi < NC) w.pts[gi] = cent[t * NC + gi];
                     double xi1, gk, gh;
