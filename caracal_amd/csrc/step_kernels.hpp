@@ -867,8 +867,18 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE))) v
             // penalty.
             if constexpr (NB == 1) __syncthreads();
             const int gi = tid % XG::GL;
-            // slots past the last trajectory too: they hold a copy of it
-            for (int t = tid / XG::GL; t < TPB; t += NG) {
+            // Slots past the last trajectory too: they hold a copy of it.  A
+            // wave without a slot leaves the loop by a scalar branch, and a
+            // group without one beside groups with one takes a turn on the last
+            // slot and stores nothing: at the join behind a loop that some lanes
+            // of a wave skip the compiler put copies of other registers (dt/2
+            // among them) ahead of the restored execution mask, in the O3
+            // kernels of 6, 16, 24 and 48 beads, and the momenta of the skipped
+            // lanes were kicked with whatever was there
+            // (tests/test_compiled_joins.py looks for such joins).
+            const int group0 = __builtin_amdgcn_readfirstlane(tid / XG::GL);
+            for (int i = 0; i < TPB - group0; i += NG) {
+                const int slot = tid / XG::GL + i, t = min(slot, TPB - 1);
                 auto &w = xw[tid / XG::GL];
                 const bool on = gi < NC;
                 const double c = on ? cent[t * NC + gi] : 0.0, dprev = on ? pdir[t * NC + gi] : 0.0;
@@ -886,16 +896,16 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE))) v
                     const double dx = sigma / (XG::sum(dxn * dm) * (a.dt * a.dt / NB));
                     mult = mult - dx;
                     // single-precision literals 1.0E-8 and 1.0E-10 of the reference
-                    if (fabs(dx) < (double)1.0e-8f || fabs(sigma) < (double)1.0e-10f) break;
+                    if (fabs(dx) < (double)1.0e-8f || fabs(sigma) < (double)1.0e-10f || slot >= TPB) break;
                     if (iter == 200) good = false;
                 }
                 const double n2 = XG::sum(on ? dnew * dnew * xt.inv_mass[gi / 3] : 0.0);
-                if (on) {
+                if (on && slot < TPB) {
                     pdir[t * NC + gi] = dnew;
                     pshift[(2 * t) * NC + gi] = good ? coeff * dm : 0.0;
                     pshift[(2 * t + 1) * NC + gi] = good ? mult * a.dt / NB * dprev : 0.0;
                 }
-                if (gi == 0) {
+                if (gi == 0 && slot < TPB) {
                     pgood[t] = good;
                     pnorm[t] = n2;
                 }

@@ -52,6 +52,63 @@ def test_both_sides_of_the_line_give_the_same_trajectories(name, ens, prec):
     assert not np.array_equal(g4, g1) or name != "h3"       # two forms ran: their roundings differ
 
 
+REACTION = {"h3": workloads.h3_reaction, "oh3": workloads.oh3_reaction, "brh2": workloads.brh2_reaction,
+            "o3": workloads.o3_reaction}
+
+
+@pytest.mark.parametrize("nb", [64, 24])
+@pytest.mark.parametrize("kind", ["nve transrot", "andersen transrot", "window", "window transrot", "parent"])
+@pytest.mark.parametrize("name", list(SURF))
+def test_both_sides_of_the_line_with_what_a_step_adds(name, kind, nb):
+    """transrot, the window's bias and the parent's constraints in the kernels
+    of one and of four lanes per bead, five steps as launches of three and two;
+    the larger batch does not fill its last one-lane block at 24 beads.
+    Tolerances as where these are compared to the oracle: 1e-12 of the largest
+    position and momentum for transrot, 1e-11 of the momenta for the bias,
+    1e-10 and 1e-9 under the constraint, whose iteration stops at |xi| < 1e-10;
+    O3's forces add 1e-12 hartree/bohr."""
+    surface, amu, ts = SURF[name]
+    limit = (256 if name == "brh2" else 512) * (64 // nb)
+    masses, beta, dt = cam.mass_au(amu), float(cam.beta_of(300.0)), 0.1 * cam.FS_TO_AU
+    rng = np.random.default_rng(2)
+    q = ts + rng.normal(0.0, 0.02, (limit + 1, nb) + ts.shape)
+    p = workloads.mb_momenta(rng, masses, nb, beta, q.shape)
+    kw = dict(seed=4, steps_per_launch=3, remove_com="transrot" in kind)
+    kw["ensemble"] = {"nve": cam.CAM_ENS_NVE, "andersen": cam.CAM_ENS_ANDERSEN, "window": cam.CAM_ENS_UMBRELLA,
+                      "parent": cam.CAM_ENS_PARENT}[kind.split()[0]]
+    if not kind.startswith("nve"):
+        kw["andersen_step"] = 4
+    steered = kind.startswith(("window", "parent"))
+    if steered:
+        kw["reaction"] = REACTION[name]()
+    out = []
+    for n in (limit, limit + 1):
+        with cam.RPMDEngine(surface, nb, n, dt, masses, **kw) as e:
+            if kind.startswith("window"):
+                e.set_windows(np.linspace(0.9, 1.05, limit + 1)[:n], np.full(n, 1.5))
+            e.set_state(q[:n], p[:n], beta)
+            if kind.startswith("window"):
+                e.begin_umbrella(bias=True)
+            if kind == "parent":
+                assert not e.constrain(project_p=True).any()
+                e.begin_parent(0.2)
+            e.run(5)
+            out.append([x[:limit] for x in e.get_state()])
+            if kind.startswith("window"):
+                out[-1] += [x[:limit] for x in e.umbrella_stats()]
+            if kind == "parent":
+                assert not e.observables()["flags"].any()
+    (q4, p4), (q1, p1) = out[0][:2], out[1][:2]
+    tq, tp = (1e-10, 1e-9) if kind == "parent" else (1e-12, 1e-11 if kind.startswith("window") else 1e-12)
+    df = 1e-12 if name == "o3" else 1e-14
+    assert np.isfinite(q4).all() and np.isfinite(p4).all()
+    assert np.abs(p4 - p1).max() <= 5 * dt * df + tp * np.abs(p1).max()
+    assert np.abs(q4 - q1).max() <= 25 * dt * dt * df / masses.min() + tq * np.abs(q1).max()
+    for a, b in zip(out[0][2:], out[1][2:]):                # mean and variance of xi, itself about 1
+        assert np.abs(a - b).max() <= 1e-12
+    assert not np.array_equal(p4, p1)                       # two forms ran: their roundings differ
+
+
 @pytest.mark.parametrize("name", list(SURF))
 def test_four_lane_forces_match_oracle_in_every_branch(name):
     """Compressed and stretched geometries, every atom in turn moved away (H3's

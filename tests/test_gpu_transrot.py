@@ -28,8 +28,7 @@ def test_transrot_in_the_step_loop_matches_oracle(name, nb, nmk, ens):
     part of the momentum that is smaller by the same ratio."""
     surface, osurf, amu, ts = SURF[name]
     masses = cam.mass_au(amu)
-    per_block = 256 // ((4 if name == "ch4h" else 1) * nb)
-    ntraj = max(2, per_block + 1)                    # the last block holds one trajectory
+    ntraj = 64 // nb + 1                             # four lanes per bead; the last block holds one trajectory
     rng = np.random.default_rng(nb)
     beta = float(cam.beta_of(300.0))
     q = ts + rng.normal(0.0, 0.02, (ntraj, nb) + ts.shape) + rng.normal(0.0, 2.0, (ntraj, 1, 1, 3))
