@@ -57,9 +57,9 @@ __device__ inline void vhx(double rdif, double ex1, double ex2, double v[4], dou
 // packed lower triangle, row-wise (0-based)
 __host__ __device__ constexpr int pk(int i, int j) { return i >= j ? i * (i + 1) / 2 + j : j * (j + 1) / 2 + i; }
 
-// Tangent and cosine of the Jacobi rotation that clears apq.  Beyond some 33
-// bohr between all three atoms every element is below 1e-150; d and b are
-// brought up together there, or their squares would vanish (a NaN angle).
+// Tangent and cosine of the Jacobi rotation that clears apq.  With all three
+// atoms some 30 bohr apart elements fall below 1e-160; d and b are brought up
+// together there, or their squares would vanish (a NaN angle).
 __device__ inline void rotation(double app, double aqq, double apq, double &t, double &c)
 {
     double d = aqq - app, b = 2.0 * apq;

@@ -463,7 +463,7 @@ __device__ __forceinline__ void egrad_bead(const double x[9], double& v, double 
 // Half of the one-lane work or less sits on each lane (the H2 curves and 48 of
 // 75 divisions go from three to one).  A step of a batch that leaves the SIMDs
 // with one wave each is this serial chain: 100 trajectories of 8 beads take
-// 14.1 us a step on one lane a bead, 5.6 on four.
+// 14.1 us a step on one lane a bead, 5.0 on four.
 // ---------------------------------------------------------------------------
 namespace q4 {
 template <typename T>

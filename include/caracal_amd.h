@@ -136,8 +136,8 @@ enum { CAM_NM_REFERENCE = 0, CAM_NM_ORTHOGONAL = 1 };
  *              (cam_engine_set_windows); the running sums of xi (mode 1)
  *              give each trajectory's average and variance
  *              (cam_engine_umbrella_stats).  Andersen as PARENT.  The fused
- *              schedule evaluates the bias inside the step kernel (one lane
- *              per trajectory, vector-ALU normal modes); the split schedule
+ *              schedule evaluates the bias inside the step kernel (16 or 32
+ *              lanes per trajectory, vector-ALU normal modes); the split schedule
  *              (or nm_kernel MFMA) in a kernel of its own after the force
  *              kernel.  Start it with cam_engine_begin_umbrella;
  *  NHC      -- dynamic.x with the Nose-Hoover chain thermostat (thermostat
@@ -216,6 +216,10 @@ typedef struct {
 
 typedef struct cam_engine cam_engine;
 
+/* Kernels are chosen by the size of the batch (for H3, OH3, BrH2 and O3 four
+ * lanes per bead in small and medium batches, one in large ones): a
+ * trajectory repeats bit for bit in batches of one size, and to rounding in
+ * batches of another. */
 int cam_engine_create(const cam_config *cfg, cam_engine **out);
 int cam_engine_destroy(cam_engine *eng);
 

@@ -56,8 +56,8 @@ def _special():
 
 
 def _separated():
-    """Three free atoms: every element of the DIM matrix is below 1e-100, its
-    squares below the smallest number.  Right angles with equal Br-H distances
+    """Three free atoms: elements of the DIM matrix whose squares are below the
+    smallest number.  Right angles with equal Br-H distances
     (equal diagonal elements) and random triples, 27 to 60 bohr apart."""
     r = np.arange(30.0, 60.0, 0.01)
     o = np.zeros_like(r)
