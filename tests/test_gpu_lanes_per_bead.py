@@ -56,27 +56,31 @@ REACTION = {"h3": workloads.h3_reaction, "oh3": workloads.oh3_reaction, "brh2": 
             "o3": workloads.o3_reaction}
 
 
-@pytest.mark.parametrize("nb", [64, 24])
-@pytest.mark.parametrize("kind", ["nve transrot", "andersen transrot", "window", "window transrot", "parent"])
+@pytest.mark.parametrize("kind,nb,nmk", [
+    (kind, nb, nmk) for nb, nmk in ((64, cam.CAM_NMK_VALU), (24, cam.CAM_NMK_VALU), (64, cam.CAM_NMK_MFMA))
+    for kind in ("nve transrot", "andersen transrot", "parent", "nhc", "window", "window transrot")
+    if nmk == cam.CAM_NMK_VALU or kind in ("nve transrot", "andersen transrot", "parent")])
 @pytest.mark.parametrize("name", list(SURF))
-def test_both_sides_of_the_line_with_what_a_step_adds(name, kind, nb):
-    """transrot, the window's bias and the parent's constraints in the kernels
-    of one and of four lanes per bead, five steps as launches of three and two;
-    the larger batch does not fill its last one-lane block at 24 beads.
+def test_both_sides_of_the_line_with_what_a_step_adds(name, kind, nb, nmk):
+    """transrot, the chain, the window's bias and the parent's constraints in the
+    kernels of one and of four lanes per bead, five steps as launches of three
+    and two; the larger batch does not fill its last one-lane block at 24 beads.
     Tolerances as where these are compared to the oracle: 1e-12 of the largest
-    position and momentum for transrot, 1e-11 of the momenta for the bias,
-    1e-10 and 1e-9 under the constraint, whose iteration stops at |xi| < 1e-10;
-    O3's forces add 1e-12 hartree/bohr."""
+    position and momentum for transrot and the chain, 1e-11 of the momenta for
+    the bias, 1e-10 and 1e-9 under the constraint, whose iteration stops at
+    |xi| < 1e-10; O3's forces add 1e-12 hartree/bohr."""
     surface, amu, ts = SURF[name]
     limit = (256 if name == "brh2" else 512) * (64 // nb)
     masses, beta, dt = cam.mass_au(amu), float(cam.beta_of(300.0)), 0.1 * cam.FS_TO_AU
     rng = np.random.default_rng(2)
     q = ts + rng.normal(0.0, 0.02, (limit + 1, nb) + ts.shape)
     p = workloads.mb_momenta(rng, masses, nb, beta, q.shape)
-    kw = dict(seed=4, steps_per_launch=3, remove_com="transrot" in kind)
+    kw = dict(seed=4, steps_per_launch=3, nm_kernel=nmk, remove_com="transrot" in kind)
     kw["ensemble"] = {"nve": cam.CAM_ENS_NVE, "andersen": cam.CAM_ENS_ANDERSEN, "window": cam.CAM_ENS_UMBRELLA,
-                      "parent": cam.CAM_ENS_PARENT}[kind.split()[0]]
-    if not kind.startswith("nve"):
+                      "parent": cam.CAM_ENS_PARENT, "nhc": cam.CAM_ENS_NHC}[kind.split()[0]]
+    if kind == "nhc":
+        kw["nose_q"] = 20 * dt
+    elif not kind.startswith("nve"):
         kw["andersen_step"] = 4
     steered = kind.startswith(("window", "parent"))
     if steered:
